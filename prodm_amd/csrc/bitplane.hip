@@ -18,6 +18,10 @@ namespace prodm {
 
 constexpr int kThreads = 256;
 
+// wave-wide prefix sum (inclusive or not) and total (DPP reductions of the device library)
+extern "C" __device__ uint32_t __ockl_wfscan_add_u32(uint32_t, bool);
+extern "C" __device__ uint32_t __ockl_wfred_add_u32(uint32_t);
+
 // ------------------------------------------------------------------------------
 // fills
 // ------------------------------------------------------------------------------
@@ -175,6 +179,117 @@ __device__ inline void stage_out(T *__restrict__ out, uint64_t n, uint64_t e0, c
         const uint32_t le = i * TPB + threadIdx.x;
         const uint64_t e = e0 + le;
         if (e < n) out[e] = sx[(le / B) * PI + (le % B)];
+    }
+}
+
+// ------------------------------------------------------------------------------
+// wave rows: a wave's 64 lanes take 32 consecutive elements each
+// ------------------------------------------------------------------------------
+// f32: lane l holds block l of the wave (64 blocks of 32). f64: block i of the
+// wave's 32 blocks of 64 is held by lanes i (elements 0..31, the low word of
+// every plane word) and i + 32 (elements 32..63, the high word).
+// Lanes read and write their elements through wave-private LDS rows of 128
+// bytes (a whole cache line per row and global access; f64 in two rounds of
+// 16 elements), so no barrier is involved. The row pitch of 36 words keeps
+// the 16-byte LDS accesses of consecutive lanes on different banks.
+constexpr int kRowElems = 32, kRowPitch = 36;
+template <class T> struct WaveRows {
+    static constexpr int kHalves = sizeof(T) / 4;             // lanes per block
+    static constexpr int kBlocks = 64 / kHalves;              // blocks per wave
+    static constexpr int kRound = 128 / (int)sizeof(T);       // elements of a row
+    static constexpr int kRounds = kRowElems / kRound;
+    // first element (in the wave's 2048) of lane row r in round h
+    static __device__ __forceinline__ uint32_t first(uint32_t r, uint32_t h) {
+        if constexpr (sizeof(T) == 4) return r * 32;
+        else return (r & 31) * 64 + (r >> 5) * 32 + h * 16;
+    }
+};
+
+// whether the wave's 2048 elements from e0 are all below n and 16-byte aligned
+template <class T> __device__ __forceinline__ bool rows_whole(const T *x, uint64_t n, uint64_t e0) {
+    return ((uintptr_t)x & 15) == 0 && e0 + 64 * kRowElems <= n;
+}
+
+// f(j, x_j) for the lane's 32 elements (0 past n) of the wave whose first
+// element is e0, a round at a time (its conversions overlap the next loads)
+template <class T, class Fn>
+__device__ __forceinline__ void rows_in(const T *__restrict__ x, uint64_t n, uint64_t e0, uint32_t *rows, Fn &&f) {
+    using R = WaveRows<T>;
+    constexpr int E = R::kRound, C = 16 / (int)sizeof(T);  // elements of a row / of 16 bytes
+    const uint32_t lane = lane_id();
+    T *const tr = reinterpret_cast<T *>(rows);
+    constexpr int kP = kRowPitch * 4 / (int)sizeof(T);     // row pitch in elements
+    const bool whole = rows_whole(x, n, e0);
+#pragma unroll
+    for (int h = 0; h < R::kRounds; h++) {
+        if (whole) {
+            float4 q[8];
+#pragma unroll
+            for (int i = 0; i < 8; i++)
+                q[i] = *reinterpret_cast<const float4 *>(x + e0 + R::first(8 * i + (lane >> 3), h) + (lane & 7) * C);
+#pragma unroll
+            for (int i = 0; i < 8; i++)
+                *reinterpret_cast<float4 *>(rows + (8 * i + (lane >> 3)) * kRowPitch + (lane & 7) * 4) = q[i];
+        } else {
+            // the last wave of the data, or an input that starts off a 16-byte line
+            T q[E];
+#pragma unroll
+            for (int i = 0; i < E; i++) {
+                const uint32_t k = 64u * i + lane;
+                const uint64_t e = e0 + R::first(k / E, h) + k % E;
+                q[i] = e < n ? x[e] : (T)0;
+            }
+#pragma unroll
+            for (int i = 0; i < E; i++) {
+                const uint32_t k = 64u * i + lane;
+                tr[(k / E) * kP + k % E] = q[i];
+            }
+        }
+        wave_lds_sync();
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            T t[C];
+            const float4 q = *reinterpret_cast<const float4 *>(rows + lane * kRowPitch + 4 * i);
+            __builtin_memcpy(t, &q, 16);
+#pragma unroll
+            for (int c = 0; c < C; c++) f(h * E + i * C + c, t[c]);
+        }
+        wave_lds_sync();
+    }
+}
+// the inverse: the lane's 32 elements to out (those below n)
+template <class T>
+__device__ __forceinline__ void rows_out(T *__restrict__ out, uint64_t n, uint64_t e0, uint32_t *rows,
+                                         const T (&v)[kRowElems]) {
+    using R = WaveRows<T>;
+    constexpr int E = R::kRound, C = 16 / (int)sizeof(T);
+    const uint32_t lane = lane_id();
+    T *const tr = reinterpret_cast<T *>(rows);
+    constexpr int kP = kRowPitch * 4 / (int)sizeof(T);
+    const bool whole = rows_whole(out, n, e0);
+#pragma unroll
+    for (int h = 0; h < R::kRounds; h++) {
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            float4 t;
+            __builtin_memcpy(&t, &v[h * E + i * C], 16);
+            *reinterpret_cast<float4 *>(rows + lane * kRowPitch + 4 * i) = t;
+        }
+        wave_lds_sync();
+        if (whole) {
+#pragma unroll
+            for (int i = 0; i < 8; i++)
+                *reinterpret_cast<float4 *>(out + e0 + R::first(8 * i + (lane >> 3), h) + (lane & 7) * C) =
+                    *reinterpret_cast<const float4 *>(rows + (8 * i + (lane >> 3)) * kRowPitch + (lane & 7) * 4);
+        } else {
+#pragma unroll
+            for (int i = 0; i < E; i++) {
+                const uint32_t k = 64u * i + lane, r = k / E, c = k % E;
+                const uint64_t e = e0 + R::first(r, h) + c;
+                if (e < n) out[e] = tr[r * kP + c];
+            }
+        }
+        wave_lds_sync();
     }
 }
 
@@ -483,163 +598,296 @@ template <class F> __device__ inline int rb_of(F orv, int nb) {
     return nb - 1 - msb;
 }
 
-// Pass 1: rb per block and an rb histogram per workgroup (hist[wg][0..nb]).
+// Encode and decode run in workgroups of 4 waves (f32: 256 blocks, f64: 128),
+// each wave on its own rows, bound by the memory's rate and the compacted
+// stores. 1025 x 1025 x 257 f64, 64 planes, finest level (1.9 GB): rb 0.78 ->
+// 0.37 ms, words 1.70 -> 0.76 ms, decode of 24 planes 1.68 -> 0.71 ms against
+// workgroups of one wave per 64 blocks (33 KB of LDS, 4 waves per CU, two
+// barriers per plane); the whole refactor + retrieve 13.06 -> 7.11 ms.
+// A row of the workspace holds, per workgroup, the words of every plane p,
+// #(rb <= p) + #(rb == p); the scan turns rows into offsets in place.
+constexpr int kGbWaves = 4, kGbTPB = 64 * kGbWaves;
+template <class T> constexpr uint32_t gb_wg_blocks() { return kGbWaves * WaveRows<T>::kBlocks; }
+
+// h[r] counts a workgroup's blocks by recording plane: the words of planes
+// pstart .. pstart + k - 1 into row[0 .. k), by the first wave (k <= 64)
+__device__ __forceinline__ void gb_row(const uint32_t *h, int pstart, int k, uint32_t *__restrict__ row) {
+    const int lane = (int)lane_id();
+    const uint32_t below = __ockl_wfscan_add_u32(h[lane], true);  // #(rb <= lane)
+    if (lane >= pstart && lane < pstart + k) row[lane - pstart] = below + h[lane];
+}
+
+// Pass 1: rb per block and the words row of each workgroup. The recording
+// plane is the top bit of the OR of the block's magnitudes; they are monotone
+// in |x| while the largest stays below 2^nb, so the largest |x| alone gives
+// it and a block needs no lane of its own: 8 (f32) or 32 (f64) lanes share
+// it through 16-byte loads and the pass reads at the memory's rate. Blocks
+// with a larger value (an exponent below the level's, infinities) take the OR.
 template <class T>
-__global__ __launch_bounds__(BlkStage<T>::kTPB) void k_gb_rb(const T *__restrict__ x, uint32_t n, int32_t exp,
-                                                          const KeyOf<T> *key, int nb, int compat,
-                                                          uint8_t *__restrict__ rb, uint32_t *__restrict__ hist) {
+__global__ __launch_bounds__(kGbTPB) void k_gb_rb(const T *__restrict__ x, uint32_t n, int32_t exp,
+                                                  const KeyOf<T> *key, int nb, int compat, uint8_t *__restrict__ rb,
+                                                  uint32_t *__restrict__ rowsum) {
     using F = typename Traits<T>::Fixed;
-    constexpr int TPB = BlkStage<T>::kTPB, B = BlkStage<T>::kB, PI = BlkStage<T>::kPitch;
-    __shared__ T sx[TPB * PI];
-    __shared__ uint32_t h[65];
-    for (int i = threadIdx.x; i <= nb; i += TPB) h[i] = 0;
-    const uint64_t b0 = (uint64_t)blockIdx.x * TPB;
-    stage_in<T>(x, n, b0 * B, sx);
+    using K = KeyOf<T>;
+    constexpr int B = Traits<T>::kBlock, C = 16 / (int)sizeof(T);
+    constexpr int G = B / C;                               // lanes per block
+    constexpr int kLoads = 64 * kRowElems / (64 * C);      // 16-byte loads per lane
+    constexpr K kInf = sizeof(T) == 4 ? (K)0x7f800000u : (K)0x7ff0000000000000ull;
+    __shared__ uint32_t h[128];
+    if (threadIdx.x < 128) h[threadIdx.x] = 0;
     __syncthreads();
+    const uint32_t lane = lane_id(), wv = threadIdx.x / 64;
+    const uint64_t b0 = (uint64_t)blockIdx.x * gb_wg_blocks<T>() + (uint64_t)wv * WaveRows<T>::kBlocks;
+    const uint64_t e0 = b0 * B;
+    const uint64_t nblk = ((uint64_t)n - 1) / B + 1;
     const int shift = nb - level_exp<T>(exp, key);
-    const uint64_t b = b0 + threadIdx.x;
-    const uint32_t nblk = (n - 1) / B + 1;
-    const T *row = sx + threadIdx.x * PI;
-    F orv = 0;
-#pragma unroll 8
-    for (int j = 0; j < B; j++) orv |= gb_mag<T>(row[j], shift, compat);
-    if (b < nblk) {
+    auto mag_key = [](T v) __attribute__((always_inline)) -> K {
+        const K q = (K)abs_key(v);
+        return q > kInf ? (K)0 : q;  // NaN has magnitude 0
+    };
+    K m[kLoads];
+    if (rows_whole(x, n, e0)) {
+        float4 q[kLoads];
+#pragma unroll
+        for (int i = 0; i < kLoads; i++) q[i] = *reinterpret_cast<const float4 *>(x + e0 + (64u * i + lane) * C);
+#pragma unroll
+        for (int i = 0; i < kLoads; i++) {
+            T t[C];
+            __builtin_memcpy(t, &q[i], 16);
+            m[i] = 0;
+#pragma unroll
+            for (int c = 0; c < C; c++) { const K a = mag_key(t[c]); m[i] = a > m[i] ? a : m[i]; }
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < kLoads; i++) {
+            m[i] = 0;
+#pragma unroll
+            for (int c = 0; c < C; c++) {
+                const uint64_t e = e0 + (64u * i + lane) * C + c;
+                const K a = e < n ? mag_key(x[e]) : (K)0;
+                m[i] = a > m[i] ? a : m[i];
+            }
+        }
+    }
+    // load i's lane group g holds block i * (64 / G) + g; lane g G + i of
+    // the group's lanes keeps block i's maximum
+    K mine = 0;
+#pragma unroll
+    for (int i = 0; i < kLoads; i++) {
+        K a = m[i];
+#pragma unroll
+        for (int o = 1; o < G; o <<= 1) {
+            const K t = __shfl_xor(a, o, 64);
+            a = t > a ? t : a;
+        }
+        if ((lane % G) == (uint32_t)i % G) mine = a;
+    }
+    static_assert(kLoads <= G, "a lane of the group per load");
+    const uint32_t bl = (lane % G) * (64 / G) + lane / G;  // this lane's block in the wave
+    const uint64_t b = b0 + bl;
+    if (lane % G < (uint32_t)kLoads && b < nblk) {
+        F orv = 0;
+        const T top = key_to_value<T>((uint64_t)mine);
+        if (dev_ldexp(top, shift) < dev_ldexp((T)1, nb)) {
+            orv = gb_mag<T>(top, shift, compat);
+        } else {
+            const uint64_t end = min((uint64_t)n, b * B + B);
+            for (uint64_t e = b * B; e < end; e++) orv |= gb_mag<T>(x[e], shift, compat);
+        }
         const int r = rb_of<F>(orv, nb);
         rb[b] = (uint8_t)r;
         atomicAdd(&h[r], 1u);
     }
     __syncthreads();
-    for (int i = threadIdx.x; i <= nb; i += TPB) hist[(uint64_t)blockIdx.x * (nb + 1) + i] = h[i];
+    if (wv == 0) gb_row(h, 0, nb, rowsum + (uint64_t)blockIdx.x * nb);
 }
 
-// words per plane p of each workgroup: #(rb <= p) + #(rb == p). One
-// workgroup per plane scans these over workgroups: off[wg][i] exclusive.
-__global__ __launch_bounds__(1024) void k_gb_scan(const uint32_t *__restrict__ hist, uint32_t nwg, int nbins,
-                                                  int pstart, int k, uint32_t *__restrict__ off,
-                                                  uint32_t *__restrict__ totals) {
-    __shared__ uint32_t sh[1024];
-    const int i = blockIdx.x;  // plane index within [pstart, pstart + k)
-    const int p = pstart + i;
-    uint32_t carry = 0;
-    for (uint32_t c0 = 0; c0 < nwg; c0 += 1024) {
-        const uint32_t wg = c0 + threadIdx.x;
-        uint32_t v = 0;
-        if (wg < nwg) {
-            const uint32_t *hh = hist + (uint64_t)wg * nbins;
-            uint32_t le = 0;
-            for (int r = 0; r <= p && r < nbins; r++) le += hh[r];
-            v = le + (p < nbins ? hh[p] : 0);
-        }
-        sh[threadIdx.x] = v;
-        __syncthreads();
-        for (int o = 1; o < 1024; o <<= 1) {
-            uint32_t t = threadIdx.x >= (uint32_t)o ? sh[threadIdx.x - o] : 0;
-            __syncthreads();
-            sh[threadIdx.x] += t;
-            __syncthreads();
-        }
-        if (wg < nwg) off[(uint64_t)wg * k + i] = carry + sh[threadIdx.x] - v;
-        carry += sh[1023];
-        __syncthreads();
+// Offsets: rows of k words are scanned down the workgroups, a lane per plane
+// (k <= 64), kGbScanRows rows per workgroup with every row load in flight.
+// k_gb_sums takes the column sums of each such group, k_gb_offsets adds those
+// of the groups before its own. (One workgroup per plane that summed the
+// histogram bins of every row took 1,600 us for 57,700 rows x 64 planes; the
+// two launches take 41 us for that level, now 28,850 rows.) A level of at
+// most kGbScanRows workgroups takes no scan launch: gb_wave_base adds the rows
+// of the workgroups before its own, which costs each of them less than the
+// 6 us launch (129^3 GroupedBP refactor + retrieve 413 -> 361 us).
+constexpr int kGbScanRows = 256, kGbScanPer = kGbScanRows / kGbWaves;
+__device__ __forceinline__ void gb_scan_load(const uint32_t *__restrict__ rows, uint32_t nrow, int k, uint32_t r0,
+                                             uint32_t (&v)[kGbScanPer], uint32_t &sum) {
+    const int lane = (int)lane_id();
+    const bool on = lane < k;
+#pragma unroll
+    for (int i = 0; i < kGbScanPer; i++) {
+        // unconditional loads (an unused one reads the first word), so that none waits for another
+        const uint32_t t = rows[on && r0 + i < nrow ? (uint64_t)(r0 + i) * k + lane : 0];
+        v[i] = on && r0 + i < nrow ? t : 0u;
     }
-    if (threadIdx.x == 0) totals[i] = carry;
+    sum = 0;
+#pragma unroll
+    for (int i = 0; i < kGbScanPer; i++) sum += v[i];
+}
+__global__ __launch_bounds__(kGbTPB) void k_gb_sums(const uint32_t *__restrict__ rows, uint32_t nrow, int k,
+                                                    uint32_t *__restrict__ sums) {
+    __shared__ uint32_t part[kGbWaves][64];
+    const uint32_t lane = lane_id(), wv = threadIdx.x / 64;
+    uint32_t v[kGbScanPer], s;
+    gb_scan_load(rows, nrow, k, blockIdx.x * kGbScanRows + wv * kGbScanPer, v, s);
+    part[wv][lane] = s;
+    __syncthreads();
+    if (wv == 0 && (int)lane < k)
+        sums[(uint64_t)blockIdx.x * k + lane] = (part[0][lane] + part[1][lane]) + (part[2][lane] + part[3][lane]);
+}
+__global__ __launch_bounds__(kGbTPB) void k_gb_offsets(uint32_t *__restrict__ rows, uint32_t nrow, int k,
+                                                       const uint32_t *__restrict__ sums,
+                                                       uint32_t *__restrict__ totals) {
+    __shared__ uint32_t part[kGbWaves][64], below[kGbWaves][64];
+    const uint32_t lane = lane_id(), wv = threadIdx.x / 64;
+    const uint32_t r0 = blockIdx.x * kGbScanRows + wv * kGbScanPer;
+    uint32_t v[kGbScanPer], s;
+    gb_scan_load(rows, nrow, k, r0, v, s);
+    // the scan groups before this one, a quarter per wave
+    uint32_t b = 0;
+    if ((int)lane < k) {
+#pragma unroll 8
+        for (uint32_t c = wv; c < blockIdx.x; c += kGbWaves) b += sums[(uint64_t)c * k + lane];
+    }
+    part[wv][lane] = s;
+    below[wv][lane] = b;
+    __syncthreads();
+    uint32_t o = (below[0][lane] + below[1][lane]) + (below[2][lane] + below[3][lane]);
+    for (uint32_t w = 0; w < wv; w++) o += part[w][lane];
+    if ((int)lane >= k) return;
+#pragma unroll
+    for (int i = 0; i < kGbScanPer; i++) {
+        if (r0 + i < nrow) rows[(uint64_t)(r0 + i) * k + lane] = o;
+        o += v[i];
+    }
+    if (totals && blockIdx.x == gridDim.x - 1 && wv == kGbWaves - 1) totals[lane] = o;  // the whole plane's words
+}
+static int gb_scan(uint32_t *rows, uint32_t nrow, int k, uint32_t *sums, uint32_t *totals, hipStream_t s) {
+    const uint32_t grid = div_up(nrow, kGbScanRows);
+    if (grid <= 1) return kOk;  // gb_wave_base sums the rows itself
+    hipLaunchKernelGGL(k_gb_sums, dim3(grid), dim3(kGbTPB), 0, s, rows, nrow, k, sums);
+    PRODM_CHECK_LAUNCH();
+    hipLaunchKernelGGL(k_gb_offsets, dim3(grid), dim3(kGbTPB), 0, s, rows, nrow, k, sums, totals);
+    PRODM_CHECK_LAUNCH();
+    return kOk;
 }
 
-// in-workgroup exclusive position of this lane's words for plane p, given
-// its counts (c1 = rb <= p, c2 = rb == p): wave prefix by ballot + mbcnt,
-// cross-wave prefix through LDS. All threads must call it (barriers).
-template <int TPB>
-__device__ inline uint32_t wg_prefix(bool c1, bool c2, uint32_t *wtot) {
-    const uint32_t wv = threadIdx.x / 64;
-    const uint64_t m1 = ballot64(c1), m2 = ballot64(c2);
-    if (lane_id() == 0) wtot[wv] = __popcll(m1) + __popcll(m2);
-    __syncthreads();
-    uint32_t pre = lanes_below(m1) + lanes_below(m2);
-    for (uint32_t q = 0; q < wv; q++) pre += wtot[q];
-    __syncthreads();
-    return pre;
-}
-
-// Pass 2: plane words, compacted per plane.
+// Positions of a wave's blocks in the planes. Lane p of the result holds where
+// the wave's first word of plane pstart + p goes: the workgroup's offset plus
+// the words of the waves before it, from the recording planes of the
+// workgroup's blocks (one barrier). rows: offsets per workgroup, or with at
+// most kGbScanRows workgroups their words, which are summed here; totals
+// (then, if any) takes the words of every plane. r: the lane's block's rb, 255
+// past the data. Both lanes of an f64 block hold the same r.
+struct GbWaveLds {
+    uint32_t hw[kGbWaves][64], below[kGbWaves][64];
+};
 template <class T>
-__global__ __launch_bounds__(BlkStage<T>::kTPB) void k_gb_write(const T *__restrict__ x, uint32_t n, int32_t exp,
-                                                             const KeyOf<T> *key, int nb, int compat,
-                                                             const uint32_t *__restrict__ off,
-                                                             typename Traits<T>::Stream *__restrict__ planes,
-                                                             uint64_t stride) {
-    using F = typename Traits<T>::Fixed;
-    using S = typename Traits<T>::Stream;
-    constexpr int TPB = BlkStage<T>::kTPB, B = BlkStage<T>::kB, PI = BlkStage<T>::kPitch;
-    __shared__ T sx[TPB * PI];
-    __shared__ uint32_t wtot[TPB / 64];
-    const uint64_t b0 = (uint64_t)blockIdx.x * TPB;
-    stage_in<T>(x, n, b0 * B, sx);
+__device__ __forceinline__ uint32_t gb_wave_base(int r, const uint32_t *__restrict__ rows, int pstart, int k,
+                                                 uint32_t *__restrict__ totals, GbWaveLds &lds) {
+    const uint32_t lane = lane_id(), wv = threadIdx.x / 64;
+    const bool on = (int)lane < k, direct = gridDim.x <= (uint32_t)kGbScanRows;
+    lds.hw[wv][lane] = 0;
+    if (r < 64 && lane < (uint32_t)WaveRows<T>::kBlocks) atomicAdd(&lds.hw[wv][r], 1u);
+    uint32_t b = 0;
+    if (direct && on) {
+#pragma unroll 8
+        for (uint32_t c = wv; c < blockIdx.x; c += kGbWaves) b += rows[(uint64_t)c * k + lane];
+    }
+    lds.below[wv][lane] = b;
     __syncthreads();
-    const int shift = nb - level_exp<T>(exp, key);
-    const uint64_t b = b0 + threadIdx.x;
-    const uint32_t nblk = (n - 1) / B + 1;
-    const T *row = sx + threadIdx.x * PI;
-    S sg = 0;
-    F orv = 0;
-    int r;
+    uint32_t hb = 0;
+    for (uint32_t w = 0; w < wv; w++) hb += lds.hw[w][lane];
+    const uint32_t words = __ockl_wfscan_add_u32(hb, true) + hb;  // lane p: plane p
+    // window lane i <- plane pstart + i
+    const uint32_t shifted = __shfl(words, (int)((lane + (uint32_t)pstart) & 63u), 64);
+    uint32_t own = on && (!direct || totals) ? rows[(uint64_t)blockIdx.x * k + lane] : 0u;
+    if (direct) {
+        const uint32_t o = (lds.below[0][lane] + lds.below[1][lane]) + (lds.below[2][lane] + lds.below[3][lane]);
+        if (totals && on && wv == 0 && blockIdx.x == gridDim.x - 1) totals[lane] = o + own;
+        own = o;
+    }
+    return on ? own + shifted : 0u;
+}
+// word index of this lane's block in plane window index i, from the wave's
+// ballots of (rb <= p) and (rb == p)
+template <class T>
+__device__ __forceinline__ uint32_t gb_pos(uint32_t base, int i, uint64_t le, uint64_t eq) {
     if constexpr (sizeof(T) == 4) {
-        uint32_t m[32];
-#pragma unroll
-        for (int j = 0; j < 32; j++) {
-            m[j] = gb_mag<T>(row[j], shift, compat);
-            orv |= m[j];
-            sg |= (S)(row[j] < 0) << j;
-        }
-        r = b < nblk ? rb_of<F>(orv, nb) : 255;
-        transpose32(m);
-#pragma unroll
-        for (int k = 31; k >= 0; k--) {
-            const int p = nb - 1 - k;  // plane p holds bit nb - 1 - p
-            if (p >= 0) {
-                const uint32_t pre = wg_prefix<TPB>(r <= p, r == p, wtot);
-                uint64_t pos = off[(uint64_t)blockIdx.x * nb + p] + pre;
-                S *dst = planes + (uint64_t)p * stride;
-                if (r == p) dst[pos++] = sg;
-                if (r <= p) dst[pos] = m[k];
-            }
-        }
+        return readlane_u32(base, i) + lanes_below(le) + lanes_below(eq);
     } else {
-        uint32_t lo[64], hi[64];
-#pragma unroll
-        for (int j = 0; j < 64; j++) {
-            const uint64_t q = gb_mag<T>(row[j], shift, compat);
-            orv |= q;
-            lo[j] = (uint32_t)q;
-            hi[j] = (uint32_t)(q >> 32);
-            sg |= (S)(row[j] < 0) << j;
-        }
-        r = b < nblk ? rb_of<F>(orv, nb) : 255;
-        transpose64(lo, hi);
-        static_for<0, 64>([&](auto kc) {
-            constexpr int k = decltype(kc)::value;
-            const int p = nb - 1 - k;
-            if (p >= 0) {
-                const uint32_t pre = wg_prefix<TPB>(r <= p, r == p, wtot);
-                uint64_t pos = off[(uint64_t)blockIdx.x * nb + p] + pre;
-                S *dst = planes + (uint64_t)p * stride;
-                if (r == p) dst[pos++] = sg;
-                if (r <= p) dst[pos] = word64_get<k>(lo, hi);
-            }
-        });
+        const uint32_t bm = (1u << (lane_id() & 31u)) - 1u;
+        return readlane_u32(base, i) + __popc((uint32_t)le & bm) + __popc((uint32_t)eq & bm);
     }
 }
 
-template <class T> static uint32_t gb_nwg(uint32_t n) {
+// Pass 2: plane words, compacted per plane. The positions need no barrier
+// inside the plane loop (gb_wave_base).
+template <class T>
+__global__ __launch_bounds__(kGbTPB) void k_gb_write(const T *__restrict__ x, uint32_t n, int32_t exp,
+                                                     const KeyOf<T> *key, int nb, int compat,
+                                                     const uint8_t *__restrict__ rb, const uint32_t *__restrict__ off,
+                                                     typename Traits<T>::Stream *__restrict__ planes, uint64_t stride,
+                                                     uint32_t *__restrict__ totals) {
+    using R = WaveRows<T>;
+    constexpr int B = Traits<T>::kBlock, W = 8 * (int)sizeof(T);
+    __shared__ __align__(16) uint32_t rows[kGbWaves][64 * kRowPitch];
+    __shared__ GbWaveLds wl;
+    const uint32_t lane = lane_id(), wv = threadIdx.x / 64;
+    const uint64_t b0 = (uint64_t)blockIdx.x * gb_wg_blocks<T>() + (uint64_t)wv * R::kBlocks;
+    const uint32_t bl = lane % R::kBlocks, half = lane / R::kBlocks;
+    const uint64_t b = b0 + bl, nblk = ((uint64_t)n - 1) / B + 1;
+    const int r = b < nblk ? rb[b] : 255;
+    // before the elements: its loop over rows would hold registers beside them
+    const uint32_t base = gb_wave_base<T>(r, off, 0, nb, totals, wl);
+    const int shift = nb - level_exp<T>(exp, key);
+    uint32_t w[W], sg = 0;
+    rows_in<T>(x, n, b0 * B, rows[wv], [&](int j, T v) __attribute__((always_inline)) {
+        const uint64_t q = gb_mag<T>(v, shift, compat);
+        w[j] = (uint32_t)q;
+        if constexpr (sizeof(T) == 8) w[32 + j] = (uint32_t)(q >> 32);
+        sg |= (uint32_t)(v < 0) << j;
+    });
+    transpose32_at<0>(w);
+    if constexpr (sizeof(T) == 8) transpose32_at<32>(w);
+    static_for<0, W>([&](auto kc) __attribute__((always_inline)) {
+        constexpr int k = decltype(kc)::value;
+        const int p = nb - 1 - k;  // plane p holds bit nb - 1 - p
+        if (p >= 0) {
+            const uint64_t le = ballot64(r <= p), eq = ballot64(r == p);
+            uint32_t pos = gb_pos<T>(base, p, le, eq);
+            uint32_t *dst = reinterpret_cast<uint32_t *>(planes + (uint64_t)p * stride) + half;
+            if (r == p) { dst[(uint64_t)pos * R::kHalves] = sg; pos++; }
+            if (r <= p) dst[(uint64_t)pos * R::kHalves] = w[k];
+        }
+    });
+}
+
+// workgroups of the formula the workspace sizes were first given out with;
+// the buffers below need less
+template <class T> static uint32_t gb_ws_rows(uint32_t n) {
     const uint32_t nblk = (n - 1) / Traits<T>::kBlock + 1;
     return div_up(nblk, BlkStage<T>::kTPB);
 }
+template <class T> static uint32_t gb_nwg(uint32_t n) {
+    const uint32_t nblk = (n - 1) / Traits<T>::kBlock + 1;
+    return div_up(nblk, gb_wg_blocks<T>());
+}
 
 template <class T> size_t gb_workspace_bytes(uint32_t n, int nb) {
-    const uint32_t nwg = gb_nwg<T>(n);
+    const uint32_t nwg = gb_ws_rows<T>(n);
     return (size_t)nwg * (nb + 1) * 4 + (size_t)nwg * nb * 4 + 256;
 }
 template size_t gb_workspace_bytes<float>(uint32_t, int);
 template size_t gb_workspace_bytes<double>(uint32_t, int);
+// rows and the scan's column sums, in words
+template <class T> static size_t gb_scan_words(uint32_t n, int k) {
+    const uint32_t nwg = gb_nwg<T>(n);
+    return ((size_t)nwg + div_up(nwg, kGbScanRows)) * k;
+}
 
 template <class T>
 int launch_gb_encode(const T *x, uint32_t n, int32_t exp, const KeyOf<T> *key, int nb, int compat, uint8_t *rb,
@@ -649,16 +897,17 @@ int launch_gb_encode(const T *x, uint32_t n, int32_t exp, const KeyOf<T> *key, i
     if (n == 0 || nb < 1 || nb > B) { set_error("grouped encode: bad n or num_bitplanes"); return kErrArg; }
     const uint32_t nblk = (n - 1) / B + 1;
     if (stride < 2ull * nblk) { set_error("grouped encode: plane stride below 2 * nblocks"); return kErrArg; }
-    if (ws_bytes < gb_workspace_bytes<T>(n, nb)) { set_error("grouped encode: workspace too small"); return kErrArg; }
+    if (ws_bytes < gb_workspace_bytes<T>(n, nb) || ws_bytes < gb_scan_words<T>(n, nb) * 4) {
+        set_error("grouped encode: workspace too small");
+        return kErrArg;
+    }
     const uint32_t nwg = gb_nwg<T>(n);
-    uint32_t *hist = static_cast<uint32_t *>(ws);
-    uint32_t *off = hist + (size_t)nwg * (nb + 1);
-    hipLaunchKernelGGL(k_gb_rb<T>, dim3(nwg), dim3(BlkStage<T>::kTPB), 0, s, x, n, exp, key, nb, compat, rb, hist);
+    uint32_t *rows = static_cast<uint32_t *>(ws), *sums = rows + (size_t)nwg * nb;
+    hipLaunchKernelGGL(k_gb_rb<T>, dim3(nwg), dim3(kGbTPB), 0, s, x, n, exp, key, nb, compat, rb, rows);
     PRODM_CHECK_LAUNCH();
-    hipLaunchKernelGGL(k_gb_scan, dim3(nb), dim3(1024), 0, s, hist, nwg, nb + 1, 0, nb, off, words_per_plane);
-    PRODM_CHECK_LAUNCH();
-    hipLaunchKernelGGL(k_gb_write<T>, dim3(nwg), dim3(BlkStage<T>::kTPB), 0, s, x, n, exp, key, nb, compat, off, planes,
-                       stride);
+    if (int rc = gb_scan(rows, nwg, nb, sums, words_per_plane, s)) return rc;
+    hipLaunchKernelGGL(k_gb_write<T>, dim3(nwg), dim3(kGbTPB), 0, s, x, n, exp, key, nb, compat, rb, rows, planes,
+                       stride, words_per_plane);
     PRODM_CHECK_LAUNCH();
     return kOk;
 }
@@ -668,101 +917,87 @@ template int launch_gb_encode<double>(const double *, uint32_t, int32_t, const u
                                       uint8_t *, uint64_t *, uint64_t, uint32_t *, void *, size_t, hipStream_t);
 
 // ---- GroupedBP progressive decode ----------------------------------------------
-// rb histogram per workgroup (same block ranges as the encoder)
+// words rows of planes [start, start + k) from the recording planes
 template <class T>
-__global__ __launch_bounds__(256) void k_gb_rbhist(const uint8_t *__restrict__ rb, uint32_t nblk, int nbins,
-                                                   uint32_t *__restrict__ hist) {
-    constexpr int TPB = BlkStage<T>::kTPB;
-    __shared__ uint32_t h[256];
-    for (int i = threadIdx.x; i < nbins; i += 256) h[i] = 0;
+__global__ __launch_bounds__(kGbTPB) void k_gb_rbrows(const uint8_t *__restrict__ rb, uint32_t nblk, int start, int k,
+                                                      uint32_t *__restrict__ rows) {
+    __shared__ uint32_t h[64];
+    if (threadIdx.x < 64) h[threadIdx.x] = 0;
     __syncthreads();
-    const uint64_t b0 = (uint64_t)blockIdx.x * TPB;
-    for (uint32_t i = threadIdx.x; i < (uint32_t)TPB; i += 256) {
-        const uint64_t b = b0 + i;
-        if (b < nblk) {
-            const int r = rb[b];
-            if (r < nbins) atomicAdd(&h[r], 1u);
-        }
+    const uint64_t b = (uint64_t)blockIdx.x * gb_wg_blocks<T>() + threadIdx.x;
+    if (threadIdx.x < gb_wg_blocks<T>() && b < nblk) {
+        const int r = rb[b];
+        if (r < 64) atomicAdd(&h[r], 1u);
     }
     __syncthreads();
-    for (int i = threadIdx.x; i < nbins; i += 256) hist[(uint64_t)blockIdx.x * nbins + i] = h[i];
+    if (threadIdx.x < 64) gb_row(h, start, k, rows + (uint64_t)blockIdx.x * k);
 }
 
-template <class S> __device__ inline S load_word(const uint8_t *base, uint64_t byte_off, bool aligned) {
-    if (aligned) return *reinterpret_cast<const S *>(base + byte_off);
-    S v = 0;
-#pragma unroll
-    for (int i = 0; i < (int)sizeof(S); i++) v |= (S)base[byte_off + i] << (8 * i);
-    return v;
+// 32-bit word at any byte offset (stream 0's words follow its header)
+__device__ __forceinline__ uint32_t load_bytes32(const uint8_t *p) {
+    return (uint32_t)p[0] | ((uint32_t)p[1] << 8) | ((uint32_t)p[2] << 16) | ((uint32_t)p[3] << 24);
 }
 
+// Lanes hold 32 elements of a block as in the encode. The words of all k
+// planes are loaded without branches: a lane without a word in a plane (rb
+// above it) takes the offset past the buffer's range and reads 0. A plane
+// holds at most 2 words per block, 2^30 bytes at 2^32 elements.
 template <class T>
-__global__ __launch_bounds__(BlkStage<T>::kTPB) void k_gb_decode(PlanePtrs pl, uint32_t n, int32_t exp,
-                                                              const KeyOf<T> *key, int start, int k,
-                                                              const uint8_t *__restrict__ rb,
-                                                              typename Traits<T>::Stream *__restrict__ signs,
-                                                              const uint32_t *__restrict__ off, T *__restrict__ out,
-                                                              uint64_t hdr0) {
-    using S = typename Traits<T>::Stream;
-    constexpr int TPB = BlkStage<T>::kTPB, B = BlkStage<T>::kB, PI = BlkStage<T>::kPitch;
-    __shared__ T sx[TPB * PI];
-    __shared__ uint32_t wtot[TPB / 64];
-    const uint64_t b0 = (uint64_t)blockIdx.x * TPB;
-    const uint64_t b = b0 + threadIdx.x;
-    const uint32_t nblk = (n - 1) / B + 1;
+__global__ __launch_bounds__(kGbTPB) void k_gb_decode(PlanePtrs pl, uint32_t n, int32_t exp, const KeyOf<T> *key,
+                                                      int start, int k, const uint8_t *__restrict__ rb,
+                                                      typename Traits<T>::Stream *__restrict__ signs,
+                                                      const uint32_t *__restrict__ off, T *__restrict__ out,
+                                                      uint64_t hdr0) {
+    using R = WaveRows<T>;
+    constexpr int B = Traits<T>::kBlock, W = 8 * (int)sizeof(T);
+    __shared__ __align__(16) uint32_t rows[kGbWaves][64 * kRowPitch];
+    __shared__ GbWaveLds wl;
+    const uint32_t lane = lane_id(), wv = threadIdx.x / 64;
+    const uint64_t b0 = (uint64_t)blockIdx.x * gb_wg_blocks<T>() + (uint64_t)wv * R::kBlocks;
+    const uint32_t bl = lane % R::kBlocks, half = lane / R::kBlocks;
+    const uint64_t b = b0 + bl, nblk = ((uint64_t)n - 1) / B + 1;
+    const bool valid = b < nblk;
     const int e0 = level_exp<T>(exp, key);
     const int end = start + k;
-    const bool valid = b < nblk;
     const int r = valid ? rb[b] : 255;
-    S sg = valid ? signs[b] : 0;
+    uint32_t *const sgw = reinterpret_cast<uint32_t *>(signs) + b * R::kHalves + half;
+    uint32_t sg = valid ? *sgw : 0u;
+    const uint32_t base = gb_wave_base<T>(r, off, start, k, nullptr, wl);
     // acc bit (end - 1 - p) comes from plane p; planes below rb are zero
-    constexpr int W = 8 * sizeof(S);
-    uint32_t lo[W], hi[sizeof(T) == 8 ? W : 1];
-#pragma unroll
-    for (int q = 0; q < W; q++) {
-        lo[q] = 0;
-        if constexpr (sizeof(T) == 8) hi[q] = 0;
-    }
-    static_for<0, W>([&](auto qc) {
+    const uint8_t *sgat = nullptr;
+    uint32_t w[W];
+    static_for<0, W>([&](auto qc) __attribute__((always_inline)) {
         constexpr int q = decltype(qc)::value;
-        const int p = end - 1 - q;  // acc bit q <- plane p
-        if (p >= start) {
-            const int i = p - start;
-            const uint32_t pre = wg_prefix<TPB>(r <= p, r == p, wtot);
-            uint64_t pos = off[(uint64_t)blockIdx.x * k + i] + pre;
-            const uint8_t *sb = static_cast<const uint8_t *>(pl.p[i]);
-            const uint64_t hb = (i == 0) ? hdr0 : 0;
-            const bool al = (hb % sizeof(S)) == 0;
-            if (r == p) { sg = load_word<S>(sb, hb + pos * sizeof(S), al); pos++; }
-            if (r <= p) {
-                const S w = load_word<S>(sb, hb + pos * sizeof(S), al);
-                if constexpr (sizeof(T) == 4) lo[q] = (uint32_t)w;
-                else word64_set<q>(lo, hi, (uint64_t)w);
+        const int p = end - 1 - q, i = p - start;
+        w[q] = 0;
+        if (i >= 0) {
+            const uint64_t le = ballot64(r <= p), eq = ballot64(r == p);
+            const uint32_t pos = gb_pos<T>(base, i, le, eq), at = (pos * R::kHalves + half) * 4;
+            const uint8_t *sb = static_cast<const uint8_t *>(pl.p[i]) + (i == 0 ? hdr0 : 0);
+            if (eq && r == p) sgat = sb + at;
+            const uint32_t word = at + (r == p ? 4 * R::kHalves : 0);
+            if (i == 0 && (hdr0 & 3)) {
+                if (r <= p) w[q] = load_bytes32(sb + word);
+            } else {
+                w[q] = buf_load<uint32_t>(buf_rsrc(sb, true), r <= p ? word : kOffNone);
             }
         }
     });
-    // persist the signs of blocks recorded in this window
-    if (valid && r >= start && r < end) signs[b] = sg;
-    T *row = sx + threadIdx.x * PI;
-    if constexpr (sizeof(T) == 4) {
-        transpose32(lo);
+    const bool fresh = r >= start && r < end;  // recorded in this window: its sign word precedes plane r's
+    if (fresh) sg = r == start && (hdr0 & 3) ? load_bytes32(sgat) : *reinterpret_cast<const uint32_t *>(sgat);
+    if (fresh) *sgw = sg;
+    transpose32_at<0>(w);
+    if constexpr (sizeof(T) == 8) transpose32_at<32>(w);
+    T v[kRowElems];
 #pragma unroll
-        for (int j = 0; j < 32; j++) {
-            T y = dev_ldexp((T)lo[j], e0 - end);
-            if ((sg >> j) & 1u) y = -y;
-            row[j] = (r >= end) ? (T)0 : y;
-        }
-    } else {
-        transpose64(lo, hi);
-#pragma unroll
-        for (int j = 0; j < 64; j++) {
-            T y = dev_ldexp((T)(((uint64_t)hi[j] << 32) | lo[j]), e0 - end);
-            if ((sg >> j) & 1u) y = -y;
-            row[j] = (r >= end) ? (T)0 : y;
-        }
+    for (int j = 0; j < kRowElems; j++) {
+        T y;
+        if constexpr (sizeof(T) == 4) y = dev_ldexp((T)w[j], e0 - end);
+        else y = dev_ldexp((T)(((uint64_t)w[32 + j] << 32) | w[j]), e0 - end);
+        if ((sg >> j) & 1u) y = -y;
+        v[j] = (r >= end) ? (T)0 : y;
     }
-    __syncthreads();
-    stage_out<T>(out, n, b0 * B, sx);
+    rows_out<T>(out, n, b0 * B, rows[wv], v);
 }
 
 template <class T>
@@ -778,20 +1013,18 @@ int launch_gb_decode(const PlanePtrs &streams, uint32_t n, int32_t exp, const Ke
     }
     const uint32_t nblk = (n - 1) / B + 1;
     const uint32_t nwg = gb_nwg<T>(n);
-    const int nbins = start + k;  // rb values >= end never contribute
-    if (ws_bytes < (size_t)nwg * (nbins + k) * 4 + (size_t)k * 4) {
+    if (ws_bytes < gb_decode_workspace_bytes<T>(n, start, k) || ws_bytes < gb_scan_words<T>(n, k) * 4) {
         set_error("grouped decode: workspace too small");
         return kErrArg;
     }
-    uint32_t *hist = static_cast<uint32_t *>(ws);
-    uint32_t *off = hist + (size_t)nwg * nbins;
-    uint32_t *totals = off + (size_t)nwg * k;
-    hipLaunchKernelGGL(k_gb_rbhist<T>, dim3(nwg), dim3(256), 0, s, rb, nblk, nbins, hist);
-    PRODM_CHECK_LAUNCH();
-    hipLaunchKernelGGL(k_gb_scan, dim3(k), dim3(1024), 0, s, hist, nwg, nbins, start, k, off, totals);
-    PRODM_CHECK_LAUNCH();
-    hipLaunchKernelGGL(k_gb_decode<T>, dim3(nwg), dim3(BlkStage<T>::kTPB), 0, s, streams, n, exp, key, start, k, rb, signs,
-                       off, out, hdr0);
+    uint32_t *rows = static_cast<uint32_t *>(ws), *sums = rows + (size_t)nwg * k;
+    if (nwg > 1) {  // a single workgroup has no offset
+        hipLaunchKernelGGL(k_gb_rbrows<T>, dim3(nwg), dim3(kGbTPB), 0, s, rb, nblk, start, k, rows);
+        PRODM_CHECK_LAUNCH();
+    }
+    if (int rc = gb_scan(rows, nwg, k, sums, nullptr, s)) return rc;
+    hipLaunchKernelGGL(k_gb_decode<T>, dim3(nwg), dim3(kGbTPB), 0, s, streams, n, exp, key, start, k, rb, signs, rows,
+                       out, hdr0);
     PRODM_CHECK_LAUNCH();
     return kOk;
 }
@@ -801,7 +1034,7 @@ template int launch_gb_decode<double>(const PlanePtrs &, uint32_t, int32_t, cons
                                       const uint8_t *, uint64_t *, double *, void *, size_t, uint64_t, hipStream_t);
 
 template <class T> size_t gb_decode_workspace_bytes(uint32_t n, int start, int k) {
-    const uint32_t nwg = gb_nwg<T>(n);
+    const uint32_t nwg = gb_ws_rows<T>(n);
     return (size_t)nwg * (start + 2 * k) * 4 + 64 * 4 + 256;
 }
 template size_t gb_decode_workspace_bytes<float>(uint32_t, int, int);
@@ -836,10 +1069,6 @@ __device__ inline typename Traits<T>::Fixed pb_mag(T x, int shift, int compat) {
     const int64_t q = fabs(v) < (T)9.2233720368547758e18 ? (int64_t)v : INT64_MIN;
     return (F)(x < 0 ? (uint64_t)0 - (uint64_t)q : (uint64_t)q);
 }
-
-// wave-wide exclusive prefix sum and total (DPP reductions of the device library)
-extern "C" __device__ uint32_t __ockl_wfscan_add_u32(uint32_t, bool);
-extern "C" __device__ uint32_t __ockl_wfred_add_u32(uint32_t);
 
 // Every lane takes 32 consecutive elements (f32 and f64), a wave 2048, a
 // workgroup of 4 waves 8192; a lane's run in a stream is at most 64 bits.
