@@ -938,8 +938,161 @@ __global__ __launch_bounds__(512) void k_solve_strided(SolveParams<T> S, uint32_
     solve_strided_lines<T, SEG>(S, m, nlines, d, blockDim.x / 64, blockIdx.x, threadIdx.x / 64, 0, true);
 }
 
-// Lines longer than the register-resident solves hold (dim 2: more than
-// 64 x 16 nodes; dims 1 / 0: more than 8 x 72): a lane per line runs the
+// Lines past the forms above (dim 2: more than 64 x 16 nodes; dims 1 / 0: more
+// than 8 x 72): a workgroup of 512 threads holds LW whole lines in LDS, thread
+// t solving segment t / LW of line t % LW; the affine maps of the segments are
+// scanned by shuffles inside a wave and through LDS over the 8 waves. LW = 1
+// is dim 2, read in coalesced runs; the others read runs of 8 LW bytes, the
+// more lines the longer the run and the shorter the lines that fit. Bound by
+// latency: of the batches of loads, of the LDS reads and FP64 operations of
+// the segments' chains, of the scans. 769-node lines of a 1537 x 769 f64 grid:
+// 342 us per solve with a lane per line in node order (13 waves on the GPU),
+// 19 us with 16 lines per workgroup (25-node segments), 13 us with 4.
+constexpr int kWideThreads = 512, kWidePitch = kWideThreads + 1;
+constexpr uint32_t kWideFix = 64;  // factors up to the fixed point, kept in LDS
+template <class T, int SEG, int LW>
+__global__ __launch_bounds__(kWideThreads) void k_solve_wide(SolveParams<T> S, uint32_t m, uint64_t nlines, int d) {
+    constexpr int NW = kWideThreads / 64, NS = kWideThreads / LW;
+    __shared__ double node[SEG * kWidePitch];  // node i of thread t's segment at i * kWidePitch + t
+    __shared__ double sA[NW][LW], sB[NW][LW], tab[kWideFix];
+    const uint32_t lane = lane_id(), wv = threadIdx.x / 64, l = threadIdx.x % LW, sg = threadIdx.x / LW;
+    const uint64_t q = (uint64_t)blockIdx.x * LW + l;
+    const uint64_t fp = S.fp, c1 = S.c[1], c2 = S.c[2];
+    bool act = q < nlines;
+    uint64_t base = 0, stride = 1, ubase = 0, ustride = 1;
+    if (LW == 1) {
+        if (act) { base = q * fp; ubase = q * c2; }
+    } else {
+        const uint64_t j2 = q % fp, r = q / fp;
+        act = act && j2 < c2;
+        stride = d == 1 ? fp : c1 * fp;
+        ustride = d == 1 ? c2 : c1 * c2;
+        if (act) {
+            base = (d == 1 ? r * c1 * fp : r * fp) + j2;
+            ubase = (d == 1 ? r * c1 * c2 : r * c2) + j2;
+        }
+    }
+    PRODM_GLOBAL double *const f = (PRODM_GLOBAL double *)S.f;
+    if (threadIdx.x < kWideFix) tab[threadIdx.x] = threadIdx.x < S.nfix ? ((const PRODM_GLOBAL double *)S.inv)[threadIdx.x] : S.lim;
+    const uint32_t seg = (m + NS - 1) / NS;
+    const uint32_t b = min(m, sg * seg), len = act ? min(m, b + seg) - b : 0u;
+    double *const v = node + threadIdx.x;
+    // the thread's share of the line for global accesses: coalesced along dim
+    // 2, else its own segment. Node j of the share is line node gat(j), at
+    // node[lat(j)]. Loads go in batches of kBatch whole ones (past the share
+    // its last node again), so that each batch waits once.
+    const uint32_t cnt = LW > 1 ? len : act && threadIdx.x < m ? (m - 1 - threadIdx.x) / kWideThreads + 1 : 0u;
+    auto gat = [&](uint32_t j) __attribute__((always_inline)) -> uint32_t {
+        return LW > 1 ? b + j : j * kWideThreads + threadIdx.x;
+    };
+    auto lat = [&](uint32_t j) __attribute__((always_inline)) -> uint32_t {
+        if constexpr (LW > 1) return j * kWidePitch + threadIdx.x;
+        const uint32_t k = gat(j);
+        return (k % seg) * kWidePitch + k / seg;
+    };
+    constexpr uint32_t kBatch = 12;
+    for (uint32_t j0 = 0; j0 < cnt; j0 += kBatch) {
+        double t[kBatch];
+#pragma unroll
+        for (uint32_t j = 0; j < kBatch; j++) t[j] = f[base + gat(min(j0 + j, cnt - 1)) * stride];
+#pragma unroll
+        for (uint32_t j = 0; j < kBatch; j++) node[lat(min(j0 + j, cnt - 1))] = t[j];
+    }
+    __syncthreads();
+    // The passes read their nodes and factors kStep at a time, before any of
+    // the step's stores; a slot past the segment reads its end node again and
+    // is discarded by selects.
+    constexpr uint32_t kStep = 4;
+    auto each = [&](bool up, bool last0, auto &&op) __attribute__((always_inline)) {
+        for (uint32_t i0 = 0; i0 < len; i0 += kStep) {
+            double x[kStep], t[kStep];
+#pragma unroll
+            for (uint32_t j = 0; j < kStep; j++) {
+                const uint32_t i = min(i0 + j, len - 1), k = up ? i : len - 1 - i;
+                x[j] = v[k * kWidePitch];
+                t[j] = b + k == m - 1 ? (last0 ? 0.0 : S.last) : tab[min(b + k, kWideFix - 1)];
+            }
+#pragma unroll
+            for (uint32_t j = 0; j < kStep; j++) {
+                const uint32_t i = min(i0 + j, len - 1);
+                op(up ? i : len - 1 - i, x[j], t[j], i0 + j < len);
+            }
+        }
+    };
+    // the map of everything before (after) this thread's segment, from the
+    // maps of the wave's segments and of the other waves, applied to 0
+    auto across = [&](double A, double Bm, bool up) __attribute__((always_inline)) -> double {
+#pragma unroll 1
+        for (int o = LW; o < 64; o <<= 1) {
+            const double pA = up ? __shfl_up(A, o, 64) : __shfl_down(A, o, 64);
+            const double pB = up ? __shfl_up(Bm, o, 64) : __shfl_down(Bm, o, 64);
+            if (up ? (int)lane >= o : (int)lane + o < 64) { A = A + Bm * pA; Bm = Bm * pB; }
+        }
+        const uint32_t pos = up ? lane : 63 - lane;
+        if (pos >= 64 - LW) { sA[wv][l] = A; sB[wv][l] = Bm; }
+        double xA = up ? __shfl_up(A, LW, 64) : __shfl_down(A, LW, 64);
+        double xB = up ? __shfl_up(Bm, LW, 64) : __shfl_down(Bm, LW, 64);
+        if (pos < LW) { xA = 0.0; xB = 1.0; }
+        __syncthreads();
+        double wA[NW], wB[NW], r = 0.0;
+#pragma unroll
+        for (int w = 0; w < NW; w++) {
+            const int g = up ? w : NW - 1 - w;
+            wA[w] = sA[g][l];
+            wB[w] = sB[g][l];
+        }
+        const int before = up ? (int)wv : NW - 1 - (int)wv;
+#pragma unroll
+        for (int w = 0; w < NW - 1; w++) r = w < before ? wA[w] + wB[w] * r : r;
+        return xA + xB * r;
+    };
+    // forward: y_i = (f_i - y_{i-1}) inv_i, the segment's map y -> A + B y
+    double A = 0.0, Bm = 1.0;
+    each(true, false, [&](uint32_t, double x, double t, bool in) __attribute__((always_inline)) {
+        A = in ? (x - A) * t : A;
+        Bm = in ? -Bm * t : Bm;
+    });
+    double y = across(A, Bm, true);
+    each(true, false, [&](uint32_t i, double x, double t, bool in) __attribute__((always_inline)) {
+        y = in ? (x - y) * t : y;
+        v[i * kWidePitch] = y;
+    });
+    // backward: z_i = y_i - cp_i z_{i+1} (z_{m-1} = y_{m-1})
+    A = 0.0;
+    Bm = 1.0;
+    each(false, true, [&](uint32_t, double x, double c, bool in) __attribute__((always_inline)) {
+        A = in ? x - c * A : A;
+        Bm = in ? -c * Bm : Bm;
+    });
+    __syncthreads();  // every wave has read the forward maps
+    double z = across(A, Bm, false);
+    each(false, true, [&](uint32_t i, double x, double c, bool in) __attribute__((always_inline)) {
+        z = in ? x - c * z : z;
+        v[i * kWidePitch] = z;
+    });
+    if constexpr (LW == 1) __syncthreads();
+    // results from LDS; u_c is updated in place, every node by one thread, a
+    // batch's loads before its stores
+    using GT = PRODM_GLOBAL T;
+    if (S.epi == kEpiNone) {
+        for (uint32_t j = 0; j < cnt; j++) f[base + gat(j) * stride] = node[lat(j)];
+        return;
+    }
+    for (uint32_t j0 = 0; j0 < cnt; j0 += kBatch) {
+        T u[kBatch];
+#pragma unroll
+        for (uint32_t j = 0; j < kBatch; j++) u[j] = ((const GT *)S.uc_in)[ubase + gat(min(j0 + j, cnt - 1)) * ustride];
+#pragma unroll
+        for (uint32_t j = 0; j < kBatch; j++) {
+            if (j0 + j >= cnt) break;
+            const double r = node[lat(j0 + j)];
+            ((GT *)S.uc_out)[ubase + gat(j0 + j) * ustride] = (T)(S.epi == kEpiAdd ? (double)u[j] + r : (double)u[j] - r);
+        }
+    }
+}
+
+// Lines longer than those hold (dim 2: more than 18432 nodes; dims 1 / 0: more
+// than 4608): a lane per line runs the
 // Thomas recurrences in node order, the forward sweep writing y in place
 // and the backward sweep reading it back (two passes over the line instead
 // of one). Lines of dims 1 / 0 are indexed as in the strided solve, so a
@@ -1311,6 +1464,33 @@ void set_factors(SolveParams<T> &S, const double *tab_dev, const Factors &F, int
 }
 
 
+// k_solve_wide for a line of m nodes along dim d (the widest runs whose lines
+// fit 148 KB of LDS); false: too long for it
+template <class T>
+bool launch_wide(const SolveParams<T> &S, uint32_t m, uint64_t nlines, int d, hipStream_t s) {
+    if (S.nfix >= kWideFix) return false;  // the table ends with the fixed point
+#define PRODM_WIDE(SEG, LW) \
+    hipLaunchKernelGGL((k_solve_wide<T, SEG, LW>), dim3(div_up(nlines, LW)), dim3(kWideThreads), 0, s, S, m, nlines, d)
+    if (d == 2) {
+        if (m <= 512u * 4) PRODM_WIDE(4, 1);
+        else if (m <= 512u * 36) PRODM_WIDE(36, 1);
+        else return false;
+    } else {
+        // four lines a workgroup while more would leave CUs idle: short
+        // segments and more workgroups count for more than the length of the
+        // runs (769 nodes, 385 lines: 19 -> 13 us)
+        const bool few = nlines < 4 * 256;
+        if (m <= 32u * 36 && !few) PRODM_WIDE(36, 16);
+        else if (m <= 64u * 36 && !few) PRODM_WIDE(36, 8);
+        else if (m <= 128u * 9) PRODM_WIDE(9, 4);
+        else if (m <= 128u * 18) PRODM_WIDE(18, 4);
+        else if (m <= 128u * 36) PRODM_WIDE(36, 4);
+        else return false;
+    }
+#undef PRODM_WIDE
+    return true;
+}
+
 template <class T>
 int solve_all(const LevelGeom &g, int l, double *f, const double *tab_dev, const Factors &F, int epi, const T *uc_in,
               T *uc_out, hipStream_t s) {
@@ -1347,7 +1527,8 @@ int solve_all(const LevelGeom &g, int l, double *f, const double *tab_dev, const
             case 8: PRODM_CONTIG(9, 64); break;
             case 9: PRODM_CONTIG(16, 64); break;
             default:
-                hipLaunchKernelGGL((k_solve_seq<T>), dim3(div_up(nlines, 256)), dim3(256), 0, s, S, m, nlines, d);
+                if (!launch_wide(S, m, nlines, d, s))
+                    hipLaunchKernelGGL((k_solve_seq<T>), dim3(div_up(nlines, 256)), dim3(256), 0, s, S, m, nlines, d);
                 break;
             }
 #undef PRODM_CONTIG
@@ -1368,7 +1549,7 @@ int solve_all(const LevelGeom &g, int l, double *f, const double *tab_dev, const
                 hipLaunchKernelGGL((k_solve_strided<T, 40>), dim3(grid), dim3(64 * nw), 0, s, S, m, nlines, d);
             else if (seg <= 72)
                 hipLaunchKernelGGL((k_solve_strided<T, 72>), dim3(grid), dim3(64 * nw), 0, s, S, m, nlines, d);
-            else
+            else if (!launch_wide(S, m, nlines, d, s))
                 hipLaunchKernelGGL((k_solve_seq<T>), dim3(div_up(nlines, 256)), dim3(256), 0, s, S, m, nlines, d);
         }
         PRODM_CHECK_LAUNCH();
