@@ -203,6 +203,15 @@ template <class S> __device__ __forceinline__ S uniform_load(const S *p) {
     return out;
 }
 
+__device__ inline uint32_t xcd_remap(uint32_t bid, uint32_t nblocks) {
+    // workgroups are dispatched round-robin over the 8 XCDs: give XCD x the
+    // contiguous range [x q, (x + 1) q) of the first 8 q tiles (a bijection;
+    // the remaining tail keeps its index)
+    const uint32_t q = nblocks / 8;
+    if (bid >= 8 * q) return bid;
+    return (bid % 8) * q + bid / 8;
+}
+
 // Entry of a grouped launch that owns virtual workgroup vb: entry e owns
 // [first[e], first[e + 1]), first[0] = 0, first[n] = total > vb.
 __device__ __forceinline__ uint32_t group_entry(const uint32_t *__restrict__ first, uint32_t n, uint32_t vb) {

@@ -152,8 +152,9 @@ size_t adjoint_workspace_bytes(const LevelGeom &g);
 template <class T>
 int mgard_recompose_adjoint(const T *g_in, const uint64_t *in_strides, const LevelGeom &g, T *out,
                             const uint64_t *out_strides, void *ws, size_t ws_bytes, hipStream_t s);
-int mgard_adjoint_coarse(const double *gfine, const LevelGeom &g, int l, double *h_out, void *ws, size_t ws_bytes,
-                         hipStream_t s);
+template <class G>
+int mgard_adjoint_coarse(const G *gfine, const uint64_t *gs, const LevelGeom &g, int l, double *h_out, void *ws,
+                         size_t ws_bytes, hipStream_t s);
 // t = S h of level l (rows of `pitch` doubles) in the workspace
 const double *mgard_adjoint_solution(const LevelGeom &g, int l, void *ws, uint32_t *pitch);
 

@@ -61,6 +61,7 @@ template <class T> struct LoadParams {
     uint32_t ilv_c[3];     // coarse dims used by the interleave index
     T *uc;                 // decompose: coarse nodal values (dense c)
     double *f;             // load vector (c0 x c1 rows of pitch fp)
+    double *h;             // adjoint: the load vector again, dense
     uint32_t fp;           // row pitch of f
     KeyOf<T> *key;         // decompose: level max |W|
     int march;             // coarse planes per workgroup along dim 0
@@ -128,15 +129,6 @@ template <int M1, int M2, int THREADS> struct SweepShape {
 };
 using SweepStd = SweepShape<7, 33, 256>;
 using SweepWide = SweepShape<7, 65, 512>;
-
-__device__ inline uint32_t xcd_remap(uint32_t bid, uint32_t nblocks) {
-    // workgroups are dispatched round-robin over the 8 XCDs: give XCD x the
-    // contiguous range [x q, (x + 1) q) of the first 8 q tiles (a bijection;
-    // the remaining tail keeps its index)
-    const uint32_t q = nblocks / 8;
-    if (bid >= 8 * q) return bid;
-    return (bid % 8) * q + bid / 8;
-}
 
 // Tiles along dim 0: floor(c0 / march), the last one also taking the
 // remainder. Coarse extents are 2^k + 1, so rounding up would leave a last
@@ -421,6 +413,7 @@ __device__ __forceinline__ void load_tile(const LoadParams<T> &P, uint32_t bt, S
     auto in_tile0 = [&](int j0) __attribute__((always_inline)) -> bool { return j0 >= M.js0 && j0 < M.js0 + M.tj0; };
     auto store_f = [&](int j0, double v) __attribute__((always_inline)) {
         ((PRODM_GLOBAL double *)P.f)[((uint64_t)j0 * c1 + j1) * P.fp + j2] = v;
+        if constexpr (MODE == kAdjointPT) P.h[((uint64_t)j0 * c1 + j1) * c2 + j2] = v;
     };
     auto column = [&](int i0, const double *G) __attribute__((always_inline)) {
         if (!has_col) return;
@@ -1781,10 +1774,12 @@ int mgard_recompose(const CoefSink<T> &src, const LevelGeom &g, int tables_ready
     return kOk;
 }
 // Adjoint helpers (adjoint.hip): h = P^T g on the coarse grid of level l
-// (the load kernel with the interpolation-transpose weights), copied to
-// h_out, then t = S h in place in the workspace's load vector.
-int mgard_adjoint_coarse(const double *gfine, const LevelGeom &g, int l, double *h_out, void *ws, size_t ws_bytes,
-                         hipStream_t s) {
+// (the load kernel with the interpolation-transpose weights, which also
+// stores it dense into h_out), then t = S h in place in the workspace's load
+// vector. g may be of either type; sums are FP64.
+template <class G>
+int mgard_adjoint_coarse(const G *gfine, const uint64_t *gs, const LevelGeom &g, int l, double *h_out, void *ws,
+                         size_t ws_bytes, hipStream_t s) {
     const WsLayout w = ws_layout(g, sizeof(double));
     if (ws_bytes < w.total) { set_error("adjoint: workspace too small"); return kErrArg; }
     char *base = static_cast<char *>(ws);
@@ -1793,21 +1788,23 @@ int mgard_adjoint_coarse(const double *gfine, const LevelGeom &g, int l, double 
     const Factors F = make_factors(g);
     if (l == g.L && !F.host.empty())
         PRODM_HIP(hipMemcpyAsync(tab, F.host.data(), F.host.size() * 8, hipMemcpyHostToDevice, s));
-    LoadParams<double> P{};
+    LoadParams<G> P{};
     for (int d = 0; d < 3; d++) { P.n[d] = g.ld[l][d]; P.c[d] = g.ld[l - 1][d]; P.ilv_c[d] = g.ld[l - 1][d]; }
     P.in = gfine;
-    P.is[0] = (uint64_t)P.n[1] * P.n[2];
-    P.is[1] = P.n[2];
+    P.is[0] = gs[0];
+    P.is[1] = gs[1];
     P.is[2] = 1;
     P.f = f;
+    P.h = h_out;
     P.fp = f_pitch(P.c[2]);
-    int rc = launch_load<double, kAdjointPT>(P, false, s);
-    if (rc) return rc;
-    const uint32_t *c = g.ld[l - 1];
-    rc = copy_box<double>(f, (uint64_t)c[1] * P.fp, P.fp, h_out, (uint64_t)c[1] * c[2], c[2], c, s);
+    int rc = launch_load<G, kAdjointPT>(P, false, s);
     if (rc) return rc;
     return solve_all<double>(g, l, f, tab, F, kEpiNone, nullptr, nullptr, s);
 }
+template int mgard_adjoint_coarse<float>(const float *, const uint64_t *, const LevelGeom &, int, double *, void *,
+                                         size_t, hipStream_t);
+template int mgard_adjoint_coarse<double>(const double *, const uint64_t *, const LevelGeom &, int, double *, void *,
+                                          size_t, hipStream_t);
 const double *mgard_adjoint_solution(const LevelGeom &g, int l, void *ws, uint32_t *pitch) {
     *pitch = f_pitch(g.ld[l - 1][2]);
     return reinterpret_cast<const double *>(static_cast<char *>(ws) + ws_layout(g, sizeof(double)).f);
