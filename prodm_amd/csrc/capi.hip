@@ -111,7 +111,7 @@ static int decompose_impl(const T *in, T *out, const uint32_t *dims, int nd, int
     CoefSink<T> sink;
     sink.full = out;
     sink.s[0] = st[0]; sink.s[1] = st[1]; sink.s[2] = 1;
-    return mgard_decompose<T>(in, st, g, sink, nullptr, ws, ws_bytes, s, nullptr, false, hier);
+    return mgard_decompose<T>(in, st, g, sink, nullptr, ws, ws_bytes, s, nullptr, hier);
 }
 
 template <class T>
@@ -125,7 +125,7 @@ static int recompose_impl(const T *in, T *out, const uint32_t *dims, int nd, int
     CoefSink<T> src;
     src.full = const_cast<T *>(in);
     src.s[0] = st[0]; src.s[1] = st[1]; src.s[2] = 1;
-    return mgard_recompose<T>(src, g, 0, out, st, ws, ws_bytes, s, nullptr, hier);
+    return mgard_recompose<T>(src, g, out, st, ws, ws_bytes, s, nullptr, hier);
 }
 
 template <class T>
@@ -341,7 +341,7 @@ template <class T> static int plan_refactor(prodm_mdr_plan *p, const T *in, hipS
     // max are final, beside the decomposition of the coarser levels (also
     // under graph capture: the fork and join become graph edges)
     if (tm) {
-        rc = mgard_decompose<T>(in, st, g, sink, keys, p->ws, p->ws_bytes, s, tm, true, p->hier != 0);
+        rc = mgard_decompose<T>(in, st, g, sink, keys, p->ws, p->ws_bytes, s, tm, p->hier != 0);
         for (int l = g.L; l >= 0 && !rc; l--) rc = encode_level(l, s);
         return rc;
     }
@@ -359,7 +359,7 @@ template <class T> static int plan_refactor(prodm_mdr_plan *p, const T *in, hipS
         return kOk;
     };
     const LevelHook hook{&hook_call<decltype(ready)>, &ready};
-    rc = mgard_decompose<T>(in, st, g, sink, keys, p->ws, p->ws_bytes, s, nullptr, true, p->hier != 0, &hook);
+    rc = mgard_decompose<T>(in, st, g, sink, keys, p->ws, p->ws_bytes, s, nullptr, p->hier != 0, &hook);
     // join the side stream back, also after an error (nothing stays forked)
     const hipError_t e1 = hipEventRecord(p->join_ev, p->side);
     const hipError_t e2 = e1 == hipSuccess ? hipStreamWaitEvent(s, p->join_ev, 0) : e1;
@@ -428,7 +428,7 @@ template <class T> static int plan_retrieve(prodm_mdr_plan *p, const uint8_t *k,
         if (p->capturing) { set_error("retrieve: PerBit decodes on the host and has no graph form"); return kErrUnsupported; }
         const uint64_t st[3] = {(uint64_t)g.dims[1] * g.dims[2], g.dims[2], 1};
         if (int rc = perbit_decode_levels<T>(p, k, s)) return rc;
-        return mgard_recompose<T>(src, g, 1, out, st, p->ws, p->ws_bytes, s, tm, p->hier != 0);
+        return mgard_recompose<T>(src, g, out, st, p->ws, p->ws_bytes, s, tm, p->hier != 0);
     }
     auto decode_level = [&](int l, hipStream_t ds) -> int {
         StageScope sc(tm, l == g.L ? kStDecodeTop : kStDecodeRest);
@@ -446,7 +446,7 @@ template <class T> static int plan_retrieve(prodm_mdr_plan *p, const uint8_t *k,
     if (tm) {
         for (int l = g.L; l >= 0 && !rc; l--) rc = decode_level(l, s);
         if (rc) return rc;
-        return mgard_recompose<T>(src, g, 1, out, st, p->ws, p->ws_bytes, s, tm, p->hier != 0);
+        return mgard_recompose<T>(src, g, out, st, p->ws, p->ws_bytes, s, tm, p->hier != 0);
     }
     // on the side stream, coarsest first: each level's decode and, for the
     // orthogonal decomposer, its recompose load sweep into a per-level load
@@ -455,8 +455,7 @@ template <class T> static int plan_retrieve(prodm_mdr_plan *p, const uint8_t *k,
     // The finest level's decode, load sweep and line solves, the bulk of the
     // bytes, start at once on a second side stream instead of after the
     // coarser levels' short, latency-bound launches (negabinary: its decode
-    // needs no workspace, so the two side streams share nothing but the
-    // read-only factor tables).
+    // needs no workspace, so the two side streams share nothing).
     if ((rc = plan_side(p))) return rc;
     const bool ahead = p->hier == 0 && g.L >= 1;
     double *fl[33] = {nullptr};
@@ -490,7 +489,7 @@ template <class T> static int plan_retrieve(prodm_mdr_plan *p, const uint8_t *k,
         return kOk;
     };
     const LevelHook hook{&hook_call<decltype(need)>, &need};
-    rc = mgard_recompose<T>(src, g, 1, out, st, p->ws, p->ws_bytes, s, nullptr, p->hier != 0, &hook,
+    rc = mgard_recompose<T>(src, g, out, st, p->ws, p->ws_bytes, s, nullptr, p->hier != 0, &hook,
                             ahead ? fl : nullptr, ahead && split);
     // every decode is joined (the last level is waited for before its recomposition)
     if (rc) (void)hipStreamWaitEvent(s, p->lev_ev[g.L], 0);
@@ -756,7 +755,6 @@ int prodm_mdr_plan_create(prodm_mdr_plan **out, const uint32_t *dims, int ndims,
     int rc = kOk;
     p->ws_bytes = mgard_workspace_bytes(g, p->elem);
     if (!rc) rc = plan_alloc(&p->ws, p->ws_bytes, p->device_bytes);
-    if (!rc) rc = mgard_upload_tables(g, p->elem, p->ws, p->ws_bytes);
     if (!rc) rc = plan_alloc(&p->levels, lo * p->elem, p->device_bytes);
     if (!rc) rc = plan_alloc(&p->keys, 8 * (g.L + 1), p->device_bytes);
     if (!rc) rc = plan_alloc(&p->planes, po * sw, p->device_bytes);

@@ -113,10 +113,6 @@ template <class T> struct CoefSink {
 };
 // hier: hierarchical basis (MGARDHierarchicalDecomposer): the same level
 // steps without the L2 correction (no load vector, no line solves).
-// Thomas factor tables live in the workspace. tables_ready: they were
-// uploaded once by mgard_upload_tables (synchronous); otherwise each call
-// uploads them on the stream.
-int mgard_upload_tables(const LevelGeom &g, size_t elem, void *ws, size_t ws_bytes);
 // Level hook: decompose calls it with l once the launches that finish level
 // l's coefficients and max key are on the stream; recompose calls it with l
 // before the first launch that reads level l (for cross-stream events).
@@ -128,15 +124,15 @@ struct LevelHook {
 template <class T>
 int mgard_decompose(const T *in, const uint64_t *in_strides, const LevelGeom &g, const CoefSink<T> &sink,
                     KeyOf<T> *level_keys, void *ws, size_t ws_bytes, hipStream_t s, StageTimer *tm = nullptr,
-                    bool tables_ready = false, bool hier = false, const LevelHook *hook = nullptr);
+                    bool hier = false, const LevelHook *hook = nullptr);
 // f_levels (optional): per level l the load vector of that level, already
 // computed by mgard_recompose_load (so those sweeps can run ahead on another
 // stream); the recompose then only solves and interpolates. top_solved: the
 // finest level's solves also ran ahead (mgard_solve_ahead), so f_levels[L]
 // holds z and the interpolation forms u_c - z itself.
 template <class T>
-int mgard_recompose(const CoefSink<T> &src, const LevelGeom &g, int tables_ready, T *out, const uint64_t *out_strides,
-                    void *ws, size_t ws_bytes, hipStream_t s, StageTimer *tm = nullptr, bool hier = false,
+int mgard_recompose(const CoefSink<T> &src, const LevelGeom &g, T *out, const uint64_t *out_strides, void *ws,
+                    size_t ws_bytes, hipStream_t s, StageTimer *tm = nullptr, bool hier = false,
                     const LevelHook *hook = nullptr, double *const *f_levels = nullptr, bool top_solved = false);
 // the line solves of level l on its load vector f_l (from
 // mgard_recompose_load), z left in f_l; they need no coarse values, so they can
@@ -189,7 +185,7 @@ struct GroupLaunch {
     }
 };
 // One field of a batched decompose: dense input, geometry, interleaved level
-// buffers, L+1 max keys and its own MGARD workspace (factor tables uploaded).
+// buffers, L+1 max keys and its own MGARD workspace.
 struct BatchFieldRef {
     const void *in = nullptr;
     const LevelGeom *g = nullptr;

@@ -517,38 +517,43 @@ __global__ __launch_bounds__(SH::kThreads) void k_load(LoadParams<T> P) {
 }
 
 // ---- line solves -----------------------------------------------------------------
-// Thomas factors (scaled coarse mass matrix tridiag(1, 4, 1), ends 2) for a
-// line of m nodes, stored as inv[0..m) then cp[0..m).
-static void thomas_factors(uint32_t m, double *inv, double *cp) {
-    for (uint32_t i = 0; i < m; i++) {
-        const double b = (i == 0 || i == m - 1) ? 2.0 : 4.0;
-        const double w = (i == 0) ? b : b - cp[i - 1];
-        inv[i] = 1.0 / w;
-        cp[i] = inv[i];
+// Thomas factors of the scaled coarse mass matrix tridiag(1, 4, 1), ends 2:
+// inv[i] = 1 / (b_i - inv[i - 1]). The interior ones depend on the node index
+// alone and reach a bitwise fixed point after a few nodes, so one constant
+// sequence serves the lines of every level and dim (tables per level in the
+// workspace took an upload per call, which waits for the stream).
+constexpr uint32_t kThomasLen = 64;
+struct ThomasSeq {
+    double v[kThomasLen] = {};
+    uint32_t fix = 0;  // v[fix ..] are all equal
+    constexpr ThomasSeq() {
+        v[0] = 1.0 / 2.0;
+        for (uint32_t i = 1; i < kThomasLen; i++) v[i] = 1.0 / (4.0 - v[i - 1]);
+        fix = kThomasLen - 1;
+        while (fix > 0 && v[fix - 1] == v[fix]) fix--;
     }
-}
+};
+constexpr ThomasSeq kThomasHost{};
+static_assert(kThomasHost.fix + 1 < kThomasLen, "the sequence reaches its fixed point");
+__device__ const ThomasSeq kThomas{};
 
 enum Epilogue : int { kEpiNone = 0, kEpiAdd = 1, kEpiSub = 2 };
 
-// The factors of interior nodes depend only on the node index (the end
-// diagonal 2 enters at node 0 and at the last node) and reach a bitwise
-// fixed point after a few nodes: the kernels read the table below nfix and
-// use lim for the interior nodes above it and last for node m - 1, the same
-// values the table holds. cp[i] = inv[i] (the off-diagonal is 1).
+// The kernels read kThomas below nfix (at most m - 1) and use lim for the
+// interior nodes from there on and last for node m - 1. cp[i] = inv[i] (the
+// off-diagonal is 1).
 template <class T> struct SolveParams {
     double *f;            // c0 x c1 rows of pitch fp
     uint32_t fp;
     uint32_t c[3];
-    const double *inv;    // inv[0..m) of the solve dim
     double lim, last;     // inv[i] for nfix <= i < m - 1, inv[m - 1]
     uint32_t nfix;
     int epi;
     const T *uc_in;       // epilogue input (dense c)
     T *uc_out;            // epilogue output (dense c)
 };
-template <class T, class P>
-__device__ __forceinline__ double thomas_factor(const SolveParams<T> &S, P inv, uint32_t m, uint32_t i) {
-    return i < S.nfix ? inv[i] : (i == m - 1 ? S.last : S.lim);
+template <class T> __device__ __forceinline__ double thomas_factor(const SolveParams<T> &S, uint32_t m, uint32_t i) {
+    return i < S.nfix ? kThomas.v[i] : (i == m - 1 ? S.last : S.lim);
 }
 
 // fidx: position in f (padded rows), uidx: position in the dense u_c
@@ -609,7 +614,7 @@ __device__ __forceinline__ void solve_contig_lines(const SolveParams<T> &S, uint
     // kOffNone offsets (narrower groups share one descriptor per wave).
     bool in[SEG];
     double iv[SEG];
-    const auto rinv = buf_rsrc((const void *)S.inv, true);
+    const auto rinv = buf_rsrc((const void *)kThomas.v, true);
 #pragma unroll
     for (int i = 0; i < SEG; i++) {
         const uint32_t k = b + i;
@@ -837,7 +842,7 @@ __device__ __forceinline__ void solve_strided_lines(const SolveParams<T> &S, uin
     for (int r = 0; r < NF; r++) {
         const uint32_t nl = b + 64u * r + lane;
         const bool has = 64u * r + lane < (uint32_t)SEG && nl < e;
-        fl[r] = has ? thomas_factor(S, (const PRODM_GLOBAL double *)S.inv, m, nl) : 0.0;
+        fl[r] = has ? thomas_factor(S, m, nl) : 0.0;
         cl[r] = nl == m - 1 ? 0.0 : fl[r];
     }
     auto fac = [&](int i) __attribute__((always_inline)) -> double { return readlane_f64(fl[i / 64], i % 64); };
@@ -942,7 +947,7 @@ __global__ __launch_bounds__(512) void k_solve_strided(SolveParams<T> S, uint32_
 // 342 us per solve with a lane per line in node order (13 waves on the GPU),
 // 19 us with 16 lines per workgroup (25-node segments), 13 us with 4.
 constexpr int kWideThreads = 512, kWidePitch = kWideThreads + 1;
-constexpr uint32_t kWideFix = 64;  // factors up to the fixed point, kept in LDS
+constexpr uint32_t kWideFix = kThomasLen;  // factors up to the fixed point, kept in LDS
 template <class T, int SEG, int LW>
 __global__ __launch_bounds__(kWideThreads) void k_solve_wide(SolveParams<T> S, uint32_t m, uint64_t nlines, int d) {
     constexpr int NW = kWideThreads / 64, NS = kWideThreads / LW;
@@ -966,7 +971,7 @@ __global__ __launch_bounds__(kWideThreads) void k_solve_wide(SolveParams<T> S, u
         }
     }
     PRODM_GLOBAL double *const f = (PRODM_GLOBAL double *)S.f;
-    if (threadIdx.x < kWideFix) tab[threadIdx.x] = threadIdx.x < S.nfix ? ((const PRODM_GLOBAL double *)S.inv)[threadIdx.x] : S.lim;
+    if (threadIdx.x < kWideFix) tab[threadIdx.x] = threadIdx.x < S.nfix ? kThomas.v[threadIdx.x] : S.lim;
     const uint32_t seg = (m + NS - 1) / NS;
     const uint32_t b = min(m, sg * seg), len = act ? min(m, b + seg) - b : 0u;
     double *const v = node + threadIdx.x;
@@ -1111,7 +1116,6 @@ __global__ __launch_bounds__(256) void k_solve_seq(SolveParams<T> S, uint32_t m,
         }
     }
     PRODM_GLOBAL double *f = (PRODM_GLOBAL double *)S.f;
-    const PRODM_CONST double *inv = (const PRODM_CONST double *)S.inv;
     constexpr uint32_t U = 8;  // loads issued ahead of the dependent chain
     double y = 0.0;
     uint32_t i = 0;
@@ -1121,12 +1125,12 @@ __global__ __launch_bounds__(256) void k_solve_seq(SolveParams<T> S, uint32_t m,
         for (uint32_t k = 0; k < U; k++) t[k] = f[base + (i + k) * stride];
 #pragma unroll
         for (uint32_t k = 0; k < U; k++) {
-            y = (t[k] - y) * thomas_factor(S, inv, m, i + k);
+            y = (t[k] - y) * thomas_factor(S, m, i + k);
             f[base + (i + k) * stride] = y;
         }
     }
     for (; i < m; i++) {
-        y = (f[base + i * stride] - y) * thomas_factor(S, inv, m, i);
+        y = (f[base + i * stride] - y) * thomas_factor(S, m, i);
         f[base + i * stride] = y;
     }
     double z = 0.0;
@@ -1138,14 +1142,14 @@ __global__ __launch_bounds__(256) void k_solve_seq(SolveParams<T> S, uint32_t m,
 #pragma unroll
         for (uint32_t k = 0; k < U; k++) {
             const uint32_t n = e - 1 - k;
-            const double c = (n == m - 1) ? 0.0 : thomas_factor(S, inv, m, n);
+            const double c = (n == m - 1) ? 0.0 : thomas_factor(S, m, n);
             z = t[k] - c * z;
             epilogue(S, base + n * stride, ubase + n * ustride, z);
         }
     }
     for (; e > 0; e--) {
         const uint32_t n = e - 1;
-        const double c = (n == m - 1) ? 0.0 : thomas_factor(S, inv, m, n);
+        const double c = (n == m - 1) ? 0.0 : thomas_factor(S, m, n);
         z = f[base + n * stride] - c * z;
         epilogue(S, base + n * stride, ubase + n * ustride, z);
     }
@@ -1401,27 +1405,8 @@ namespace {
 
 uint64_t points3(const uint32_t *n) { return (uint64_t)n[0] * n[1] * n[2]; }
 
-// factor tables for every (level, dim), packed: offsets[l][d] into the table
-struct Factors {
-    std::vector<double> host;
-    uint64_t off[33][3];
-};
-Factors make_factors(const LevelGeom &g) {
-    Factors F;
-    for (int l = 1; l <= g.L; l++)
-        for (int d = 0; d < 3; d++) {
-            const uint32_t m = g.ld[l - 1][d];
-            F.off[l][d] = F.host.size();
-            std::vector<double> inv(m), cp(m);
-            thomas_factors(m, inv.data(), cp.data());
-            F.host.insert(F.host.end(), inv.begin(), inv.end());
-            F.host.insert(F.host.end(), cp.begin(), cp.end());
-        }
-    return F;
-}
-
 struct WsLayout {
-    size_t xa, xb, f, tab, total;
+    size_t xa, xb, f, total;
 };
 WsLayout ws_layout(const LevelGeom &g, size_t elem) {
     WsLayout w{};
@@ -1432,36 +1417,25 @@ WsLayout ws_layout(const LevelGeom &g, size_t elem) {
     w.xb = al(w.xa + p1 * elem);
     w.f = al(w.xb + std::max(p1, p2) * elem);
     const uint64_t f1 = g.L >= 1 ? (uint64_t)g.ld[g.L - 1][0] * g.ld[g.L - 1][1] * f_pitch(g.ld[g.L - 1][2]) : 1;
-    w.tab = al(w.f + f1 * sizeof(double));
-    size_t tab = 0;
-    for (int l = 1; l <= g.L; l++)
-        for (int d = 0; d < 3; d++) tab += 2 * g.ld[l - 1][d];
-    w.total = al(w.tab + tab * sizeof(double));
+    w.total = al(w.f + f1 * sizeof(double));
     return w;
 }
 
-// factor table of level l, dim d on the device and its fixed-point summary
-template <class T>
-void set_factors(SolveParams<T> &S, const double *tab_dev, const Factors &F, int l, int d, uint32_t m) {
-    const double *h = F.host.data() + F.off[l][d];
-    S.inv = tab_dev + F.off[l][d];
-    S.last = h[m - 1];
-    S.nfix = m;
-    S.lim = 0.0;
-    if (m >= 3) {
-        uint32_t j = m - 2;  // h[j .. m - 2] all equal h[m - 2]
-        while (j > 0 && h[j - 1] == h[m - 2]) j--;
-        S.nfix = j;
-        S.lim = h[m - 2];
-    }
+// the factors of a line of m nodes
+template <class T> void set_factors(SolveParams<T> &S, uint32_t m) {
+    const ThomasSeq &q = kThomasHost;
+    const uint32_t e = m >= 2 ? std::min(m - 2, kThomasLen - 1) : 0;  // node m - 2's entry
+    S.last = m >= 2 ? 1.0 / (2.0 - q.v[e]) : 1.0 / 2.0;
+    S.lim = q.v[e];
+    uint32_t j = m >= 3 ? std::min(e, q.fix) : m - 1;
+    while (m >= 3 && j > 0 && q.v[j - 1] == q.v[e]) j--;
+    S.nfix = j;
 }
-
 
 // k_solve_wide for a line of m nodes along dim d (the widest runs whose lines
 // fit 148 KB of LDS); false: too long for it
 template <class T>
 bool launch_wide(const SolveParams<T> &S, uint32_t m, uint64_t nlines, int d, hipStream_t s) {
-    if (S.nfix >= kWideFix) return false;  // the table ends with the fixed point
 #define PRODM_WIDE(SEG, LW) \
     hipLaunchKernelGGL((k_solve_wide<T, SEG, LW>), dim3(div_up(nlines, LW)), dim3(kWideThreads), 0, s, S, m, nlines, d)
     if (d == 2) {
@@ -1485,8 +1459,7 @@ bool launch_wide(const SolveParams<T> &S, uint32_t m, uint64_t nlines, int d, hi
 }
 
 template <class T>
-int solve_all(const LevelGeom &g, int l, double *f, const double *tab_dev, const Factors &F, int epi, const T *uc_in,
-              T *uc_out, hipStream_t s) {
+int solve_all(const LevelGeom &g, int l, double *f, int epi, const T *uc_in, T *uc_out, hipStream_t s) {
     const uint32_t *c = g.ld[l - 1];
     const uint32_t *n = g.ld[l];
     // solves run dims 2, 1, 0: the last one executed is the smallest active d
@@ -1499,7 +1472,7 @@ int solve_all(const LevelGeom &g, int l, double *f, const double *tab_dev, const
         S.f = f;
         S.fp = f_pitch(c[2]);
         S.c[0] = c[0]; S.c[1] = c[1]; S.c[2] = c[2];
-        set_factors(S, tab_dev, F, l, d, c[d]);
+        set_factors(S, c[d]);
         S.epi = (d == last) ? epi : kEpiNone;
         S.uc_in = uc_in;
         S.uc_out = uc_out;
@@ -1624,19 +1597,10 @@ int launch_load(LoadParams<T> P, bool ilv, hipStream_t s) {
 
 size_t mgard_workspace_bytes(const LevelGeom &g, size_t elem) { return ws_layout(g, elem).total; }
 
-int mgard_upload_tables(const LevelGeom &g, size_t elem, void *ws, size_t ws_bytes) {
-    const WsLayout w = ws_layout(g, elem);
-    if (ws_bytes < w.total) { set_error("workspace too small"); return kErrArg; }
-    const Factors F = make_factors(g);
-    if (!F.host.empty())
-        PRODM_HIP(hipMemcpy(static_cast<char *>(ws) + w.tab, F.host.data(), F.host.size() * 8, hipMemcpyHostToDevice));
-    return kOk;
-}
-
 template <class T>
 int mgard_decompose(const T *in, const uint64_t *in_strides, const LevelGeom &g, const CoefSink<T> &sink,
-                    KeyOf<T> *level_keys, void *ws, size_t ws_bytes, hipStream_t s, StageTimer *tm, bool tables_ready,
-                    bool hier, const LevelHook *hook) {
+                    KeyOf<T> *level_keys, void *ws, size_t ws_bytes, hipStream_t s, StageTimer *tm, bool hier,
+                    const LevelHook *hook) {
     const LevelHook none{nullptr, nullptr};
     const LevelHook &ready = hook ? *hook : none;
     const WsLayout w = ws_layout(g, sizeof(T));
@@ -1644,12 +1608,6 @@ int mgard_decompose(const T *in, const uint64_t *in_strides, const LevelGeom &g,
     char *base = static_cast<char *>(ws);
     T *xa = reinterpret_cast<T *>(base + w.xa), *xb = reinterpret_cast<T *>(base + w.xb);
     double *f = reinterpret_cast<double *>(base + w.f);
-    double *tab = reinterpret_cast<double *>(base + w.tab);
-    const Factors F = make_factors(g);
-    // a copy from pageable memory blocks the host until the stream drains:
-    // plans upload the tables once (mgard_upload_tables)
-    if (!tables_ready && !F.host.empty())
-        PRODM_HIP(hipMemcpyAsync(tab, F.host.data(), F.host.size() * 8, hipMemcpyHostToDevice, s));
     const bool ilv = sink.full == nullptr;
     const T *cur = in;
     uint64_t cs[3] = {in_strides[0], in_strides[1], 1};
@@ -1674,7 +1632,7 @@ int mgard_decompose(const T *in, const uint64_t *in_strides, const LevelGeom &g,
         if (rc) return rc;
         if (!hier) {
             StageScope sc(tm, l == g.L ? kStDecSolveTop : kStDecSolveRest);
-            rc = solve_all<T>(g, l, f, tab, F, kEpiAdd, uc, uc, s);
+            rc = solve_all<T>(g, l, f, kEpiAdd, uc, uc, s);
         }
         if (rc) return rc;
         cur = uc;
@@ -1703,14 +1661,14 @@ int mgard_decompose(const T *in, const uint64_t *in_strides, const LevelGeom &g,
     return kOk;
 }
 template int mgard_decompose<float>(const float *, const uint64_t *, const LevelGeom &, const CoefSink<float> &,
-                                    uint32_t *, void *, size_t, hipStream_t, StageTimer *, bool, bool,
+                                    uint32_t *, void *, size_t, hipStream_t, StageTimer *, bool,
                                     const LevelHook *);
 template int mgard_decompose<double>(const double *, const uint64_t *, const LevelGeom &, const CoefSink<double> &,
-                                     unsigned long long *, void *, size_t, hipStream_t, StageTimer *, bool, bool,
+                                     unsigned long long *, void *, size_t, hipStream_t, StageTimer *, bool,
                                      const LevelHook *);
 
 template <class T>
-int mgard_recompose(const CoefSink<T> &src, const LevelGeom &g, int tables_ready, T *out, const uint64_t *out_strides,
+int mgard_recompose(const CoefSink<T> &src, const LevelGeom &g, T *out, const uint64_t *out_strides,
                     void *ws, size_t ws_bytes, hipStream_t s, StageTimer *tm, bool hier, const LevelHook *hook,
                     double *const *f_levels, bool top_solved) {
     const LevelHook none{nullptr, nullptr};
@@ -1720,10 +1678,6 @@ int mgard_recompose(const CoefSink<T> &src, const LevelGeom &g, int tables_ready
     char *base = static_cast<char *>(ws);
     T *bufs[2] = {reinterpret_cast<T *>(base + w.xa), reinterpret_cast<T *>(base + w.xb)};
     double *f = reinterpret_cast<double *>(base + w.f);
-    double *tab = reinterpret_cast<double *>(base + w.tab);
-    const Factors F = make_factors(g);
-    if (!tables_ready && !F.host.empty())
-        PRODM_HIP(hipMemcpyAsync(tab, F.host.data(), F.host.size() * 8, hipMemcpyHostToDevice, s));
     const bool ilv = src.full == nullptr;
     const uint32_t *c0 = g.ld[0];
     if (int rc = need(0)) return rc;
@@ -1752,7 +1706,7 @@ int mgard_recompose(const CoefSink<T> &src, const LevelGeom &g, int tables_ready
             }
             if (rc) return rc;
             StageScope sc(tm, l == g.L ? kStRecSolveTop : kStRecSolveRest);
-            rc = solve_all<T>(g, l, fl, tab, F, kEpiSub, cur, cur, s);  // u_c = u_c' - z, in place
+            rc = solve_all<T>(g, l, fl, kEpiSub, cur, cur, s);  // u_c = u_c' - z, in place
             if (rc) return rc;
         }
         const uint32_t *n = g.ld[l];
@@ -1784,10 +1738,6 @@ int mgard_adjoint_coarse(const G *gfine, const uint64_t *gs, const LevelGeom &g,
     if (ws_bytes < w.total) { set_error("adjoint: workspace too small"); return kErrArg; }
     char *base = static_cast<char *>(ws);
     double *f = reinterpret_cast<double *>(base + w.f);
-    double *tab = reinterpret_cast<double *>(base + w.tab);
-    const Factors F = make_factors(g);
-    if (l == g.L && !F.host.empty())
-        PRODM_HIP(hipMemcpyAsync(tab, F.host.data(), F.host.size() * 8, hipMemcpyHostToDevice, s));
     LoadParams<G> P{};
     for (int d = 0; d < 3; d++) { P.n[d] = g.ld[l][d]; P.c[d] = g.ld[l - 1][d]; P.ilv_c[d] = g.ld[l - 1][d]; }
     P.in = gfine;
@@ -1799,7 +1749,7 @@ int mgard_adjoint_coarse(const G *gfine, const uint64_t *gs, const LevelGeom &g,
     P.fp = f_pitch(P.c[2]);
     int rc = launch_load<G, kAdjointPT>(P, false, s);
     if (rc) return rc;
-    return solve_all<double>(g, l, f, tab, F, kEpiNone, nullptr, nullptr, s);
+    return solve_all<double>(g, l, f, kEpiNone, nullptr, nullptr, s);
 }
 template int mgard_adjoint_coarse<float>(const float *, const uint64_t *, const LevelGeom &, int, double *, void *,
                                          size_t, hipStream_t);
@@ -1810,18 +1760,16 @@ const double *mgard_adjoint_solution(const LevelGeom &g, int l, void *ws, uint32
     return reinterpret_cast<const double *>(static_cast<char *>(ws) + ws_layout(g, sizeof(double)).f);
 }
 
-template int mgard_recompose<float>(const CoefSink<float> &, const LevelGeom &, int, float *, const uint64_t *, void *,
-                                    size_t, hipStream_t, StageTimer *, bool, const LevelHook *, double *const *, bool);
-template int mgard_recompose<double>(const CoefSink<double> &, const LevelGeom &, int, double *, const uint64_t *,
-                                     void *, size_t, hipStream_t, StageTimer *, bool, const LevelHook *,
+template int mgard_recompose<float>(const CoefSink<float> &, const LevelGeom &, float *, const uint64_t *, void *, size_t,
+                                    hipStream_t, StageTimer *, bool, const LevelHook *, double *const *, bool);
+template int mgard_recompose<double>(const CoefSink<double> &, const LevelGeom &, double *, const uint64_t *, void *,
+                                     size_t, hipStream_t, StageTimer *, bool, const LevelHook *,
                                      double *const *, bool);
 
 template <class T> int mgard_solve_ahead(const LevelGeom &g, int l, double *f_l, void *ws, size_t ws_bytes, hipStream_t s) {
     const WsLayout w = ws_layout(g, sizeof(T));
     if (l < 1 || l > g.L || !f_l || ws_bytes < w.total) { set_error("solve ahead: bad level or workspace"); return kErrArg; }
-    const double *tab = reinterpret_cast<const double *>(static_cast<const char *>(ws) + w.tab);
-    const Factors F = make_factors(g);
-    return solve_all<T>(g, l, f_l, tab, F, kEpiNone, (const T *)nullptr, (T *)nullptr, s);
+    return solve_all<T>(g, l, f_l, kEpiNone, (const T *)nullptr, (T *)nullptr, s);
 }
 template int mgard_solve_ahead<float>(const LevelGeom &, int, double *, void *, size_t, hipStream_t);
 template int mgard_solve_ahead<double>(const LevelGeom &, int, double *, void *, size_t, hipStream_t);
@@ -1923,7 +1871,6 @@ int mgard_batched_launches(const std::vector<BatchFieldRef> &fields, const std::
             char *base = static_cast<char *>(f.ws);
             T *bufs[2] = {reinterpret_cast<T *>(base + w.xa), reinterpret_cast<T *>(base + w.xb)};
             double *fv = reinterpret_cast<double *>(base + w.f);
-            const double *tab = reinterpret_cast<const double *>(base + w.tab);
             CoefSink<T> sink;
             for (int k = 0; k <= g.L; k++) sink.level[k] = static_cast<T *>(f.level[k]);
             State &s = st[i];
@@ -1948,14 +1895,13 @@ int mgard_batched_launches(const std::vector<BatchFieldRef> &fields, const std::
                 int last = -1;
                 for (int d = 0; d < 3; d++)
                     if (n[d] > 1) { last = d; break; }
-                const Factors F = make_factors(g);
                 for (int d = 2; d >= 0; d--) {
                     if (n[d] == 1) continue;
                     SolveEntry<T> E{};
                     E.S.f = fv;
                     E.S.fp = f_pitch(c[2]);
                     E.S.c[0] = c[0]; E.S.c[1] = c[1]; E.S.c[2] = c[2];
-                    set_factors(E.S, tab, F, l, d, c[d]);
+                    set_factors(E.S, c[d]);
                     E.S.epi = (d == last) ? kEpiAdd : kEpiNone;
                     E.S.uc_in = uc;
                     E.S.uc_out = uc;
