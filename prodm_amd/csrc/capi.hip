@@ -253,12 +253,7 @@ static int collect_squared_impl(const T *x, uint64_t n, int nb, T maxerr, double
                                 hipStream_t s) {
     if (nb < 1 || nb > Traits<T>::kBlock || !h_out) { set_error("squared collector: bad arguments"); return kErrArg; }
     if (ws_bytes < sq_workspace_bytes<T>(n, nb)) { set_error("squared collector: workspace too small"); return kErrArg; }
-    int rc = launch_collect_squared<T>(x, n, nb, maxerr, ws, ws_bytes, s);
-    if (rc) return rc;
-    std::vector<uint8_t> host(sq_result_bytes<T>(nb));
-    PRODM_HIP(hipMemcpyAsync(host.data(), ws, host.size(), hipMemcpyDeviceToHost, s));
-    PRODM_HIP(hipStreamSynchronize(s));
-    return finish_collect_squared<T>(host.data(), nb, maxerr, h_out);
+    return squared_errors<T>(x, n, nb, maxerr, h_out, ws, s);
 }
 
 }  // namespace prodm

@@ -1,18 +1,12 @@
-// collect.hip -- SquaredErrorCollector (SquaredErrorCollector.hpp:23-65) on gfx950.
+// collect.hip -- SquaredErrorCollector (SquaredErrorCollector.hpp:23-65) and the
+// encoders' level errors on gfx950.
 //
 // The reference adds, per element, the squared truncation error of every
 // bitplane prefix (computed in T) into a double table, sequentially. A
 // parallel FP64 sum cannot reproduce that order, so each table entry is
 // defined as the EXACTLY ROUNDED sum of the same terms: order independent,
-// and identical between this kernel and the CPU restatement.
-//
-// Exactness: every truncation term is a multiple of Q = max(q^2, min_sub)
-// with q = 2^(le - nb - prec) (the finest mantissa step of any element whose
-// planes are truncated), and is at most 2^(2 le). Terms are accumulated as
-// integers in units of Q in per-thread multi-limb registers, reduced across
-// the wave and workgroup with carries, and summed exactly on the host. The
-// rare squares x^2 of elements far below the level maximum that are not
-// multiples of Q go to a per-(bin, exponent) histogram of mantissa sums.
+// and identical between these kernels and the CPU restatement.
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <vector>
@@ -20,23 +14,6 @@
 #include "internal.hpp"
 
 namespace prodm {
-
-template <class T> struct SqCfg;
-template <> struct SqCfg<float> {
-    static constexpr int kLimbs = 2;      // 2^128 > 2^(2*32+46) * 2^12 terms per wave chunk
-    static constexpr int kExpBuckets = 256;
-    static constexpr int kEmin = -149;
-    static constexpr int kMantBits = 23;
-};
-template <> struct SqCfg<double> {
-    static constexpr int kLimbs = 4;      // 2^256 > 2^(2*64+104) * 2^12
-    static constexpr int kExpBuckets = 2048;
-    static constexpr int kEmin = -1074;
-    static constexpr int kMantBits = 52;
-};
-
-constexpr int kSqThreads = 256;
-constexpr int kSqEPT = 16;  // elements per thread
 
 template <class T> __device__ inline typename Traits<T>::Bits to_bits(T v) {
     typename Traits<T>::Bits b;
@@ -48,6 +25,281 @@ template <class T> __device__ inline T from_bits(typename Traits<T>::Bits b) {
     __builtin_memcpy(&v, &b, sizeof(v));
     return v;
 }
+
+// ---- exact host summation and rounding ---------------------------------------------
+namespace {
+struct Big {
+    std::vector<uint64_t> w;  // little endian
+    explicit Big(size_t limbs) : w(limbs, 0) {}
+    void add_shifted(uint64_t v, int shift) {  // v << shift, shift >= 0
+        if (!v) return;
+        const size_t li = (size_t)shift / 64;
+        const int off = shift % 64;
+        uint64_t parts[2] = {v << off, off ? (v >> (64 - off)) : 0};
+        uint64_t carry = 0;
+        for (size_t j = li; j < w.size(); j++) {
+            const uint64_t add = (j - li < 2) ? parts[j - li] : 0;
+            if (j - li >= 2 && !carry) break;
+            const uint64_t s1 = w[j] + add;
+            const uint64_t c1 = s1 < add;
+            const uint64_t s2 = s1 + carry;
+            const uint64_t c2 = s2 < carry;
+            w[j] = s2;
+            carry = c1 | c2;
+        }
+    }
+    void sub_shifted(uint64_t v, int shift) {  // the total stays >= 0
+        if (!v) return;
+        const size_t li = (size_t)shift / 64;
+        const int off = shift % 64;
+        const uint64_t parts[2] = {v << off, off ? (v >> (64 - off)) : 0};
+        uint64_t borrow = 0;
+        for (size_t j = li; j < w.size(); j++) {
+            if (j - li >= 2 && !borrow) break;
+            const uint64_t sub = (j - li < 2) ? parts[j - li] : 0;
+            const uint64_t s1 = w[j] - sub, s2 = s1 - borrow;
+            borrow = (w[j] < sub) | (s1 < borrow);
+            w[j] = s2;
+        }
+    }
+    void add128(__int128 v, int shift, bool negatives) {  // the value, or nothing if its sign is not asked for
+        if ((v < 0) != negatives) return;
+        const unsigned __int128 m = negatives ? (unsigned __int128)(-v) : (unsigned __int128)v;
+        const uint64_t lo = (uint64_t)m, hi = (uint64_t)(m >> 64);
+        if (negatives) { sub_shifted(lo, shift); sub_shifted(hi, shift + 64); }
+        else { add_shifted(lo, shift); add_shifted(hi, shift + 64); }
+    }
+    int bit(long i) const { return i < 0 ? 0 : (int)((w[(size_t)i / 64] >> (i % 64)) & 1u); }
+    // value * 2^scale rounded to nearest even
+    double to_double(int scale) const {
+        long top = -1;
+        for (long i = (long)w.size() - 1; i >= 0; i--)
+            if (w[i]) { top = i * 64 + 63 - __builtin_clzll(w[i]); break; }
+        if (top < 0) return 0.0;
+        if (top <= 52) return std::ldexp((double)w[0], scale);
+        const long lsb = top - 52;
+        uint64_t mant = 0;
+        for (long b = top; b >= lsb; b--) mant = (mant << 1) | (uint64_t)bit(b);
+        const int rb = bit(lsb - 1);
+        int sticky = 0;
+        for (long b = lsb - 2; b >= 0 && !sticky; b--) sticky = bit(b);
+        if (rb && (sticky || (mant & 1u))) mant++;
+        return std::ldexp((double)mant, (int)(scale + lsb));
+    }
+};
+}  // namespace
+
+
+// ---- exact sums in FP64 (float data) --------------------------------------------
+// A term below 2^T and a multiple of 2^Q is added to up to three accumulators
+// of decreasing grid 2^u. An accumulator starts at 1.5 2^(u + 52), so that it
+// stays in one binade, whose numbers are the multiples of 2^u: adding a term
+// rounds it to the grid, the rounding error is exact and goes to the next one,
+// and the last grid is 2^Q itself. The sum in units of 2^u is the difference of
+// the bit patterns, an integer. 32 terms per accumulator, then the integers go to
+// LDS (a slot per lane pair), to one partial sum per workgroup, and to 96-bit
+// totals that the host adds and rounds once. A term costs 3 operations per
+// accumulator but the last, which costs 1; the tables' lower entries need
+// three, most two (carrying integers over the words of the same window took
+// some 50 operations, a wave reduction of them per 16 terms, and a host sum
+// over every workgroup's partials: 257^3 finest level, both tables 2.94 ms, now
+// 0.43 ms).
+namespace {
+
+constexpr int kExThreads = 256, kExEPT = 32, kExChunk = kExThreads * kExEPT;
+constexpr int kExMaxChunks = 8;  // 2^16 terms below 2^(u + 45) per workgroup: sums stay in 63 bits
+constexpr int kExSlots = 32;     // LDS words per accumulator
+constexpr int kExBins = 35;      // nb + 1 entries and two for the tiny elements
+constexpr int kExBuckets = 2048;
+
+struct Grid3 {
+    int n;     // accumulators used
+    int u[3];  // exponents of their grids; the last is [2]
+};
+// grids of terms of at most 2^T, multiples of 2^Q
+__host__ __device__ inline Grid3 grid3(int T, int Q) {
+    Grid3 g;
+    // 32 terms of at most 2^T in the first, remainders of at most 2^(T - 46),
+    // 2^(T - 92) in the others, each sum below half of the bias's binade
+    g.n = T - Q <= 45 ? 1 : T - Q <= 91 ? 2 : 3;
+    g.u[0] = T - 45;
+    g.u[1] = T - 91;
+    g.u[2] = Q;
+    return g;
+}
+// the tiny elements' grids: no Q, what the third does not hold is refused
+__host__ __device__ inline Grid3 grid3_open(int T) {
+    Grid3 g{3, {T - 45, T - 91, T - 137}};
+    return g;
+}
+__device__ __forceinline__ double grid_bias(int u) { return ldexp(1.5, u + 52); }
+
+struct Acc3 {
+    double a[3], b[3];
+    __device__ __forceinline__ void start(const Grid3 &g) {
+#pragma unroll
+        for (int i = 0; i < 3; i++) a[i] = b[i] = grid_bias(g.u[i]);
+    }
+    template <int N> __device__ __forceinline__ void add(double t) {
+        if constexpr (N >= 2) { const double n = a[0] + t; t -= n - a[0]; a[0] = n; }
+        if constexpr (N >= 3) { const double n = a[1] + t; t -= n - a[1]; a[1] = n; }
+        a[2] += t;
+    }
+    // adds t if the three grids hold it
+    __device__ __forceinline__ bool add_open(double t) {
+        const double n0 = a[0] + t, t1 = t - (n0 - a[0]);
+        const double n1 = a[1] + t1, t2 = t1 - (n1 - a[1]);
+        const double n2 = a[2] + t2;
+        if (t2 - (n2 - a[2]) != 0.0) return false;
+        a[0] = n0; a[1] = n1; a[2] = n2;
+        return true;
+    }
+    __device__ __forceinline__ void flush(unsigned long long *slot) const {
+#pragma unroll
+        for (int i = 0; i < 3; i++) {
+            // unconditional: behind a test, the second and third chains of the
+            // sums would sink to their uses, with all terms held until then
+            const uint64_t d = to_bits(a[i]) - to_bits(b[i]);
+            atomicAdd(slot + i * kExSlots + (threadIdx.x % kExSlots), (unsigned long long)d);
+        }
+    }
+};
+
+// one finite term outside the grids, into the 128-bit sum of its exponent
+__device__ __forceinline__ void add_under(double t, int bin, unsigned long long *under, uint32_t *flag) {
+    const uint64_t tb = to_bits(t);
+    const int be = (int)((tb >> 52) & 0x7ff);
+    if (!(tb << 1) || be == 0x7ff) return;  // zero; infinite and NaN terms have no sum
+    const unsigned long long M = (tb & ((1ull << 52) - 1)) | (be ? (1ull << 52) : 0);
+    unsigned long long *bk = under + ((size_t)bin * kExBuckets + (be ? be : 1)) * 2;
+    const unsigned long long old = atomicAdd(bk, M);
+    if (old + M < old) atomicAdd(bk + 1, 1ull);
+    *flag = 1u;
+}
+
+// the workgroup's sums of every accumulator (kExBins * 3 of kExSlots words)
+__device__ __forceinline__ void store_partials(const unsigned long long *acc, int bins, uint64_t *__restrict__ partial) {
+    for (int s = threadIdx.x; s < bins * 3; s += kExThreads) {
+        uint64_t v = 0;
+#pragma unroll
+        for (int i = 0; i < kExSlots; i++) v += acc[s * kExSlots + ((i + threadIdx.x) % kExSlots)];
+        partial[(uint64_t)s * gridDim.x + blockIdx.x] = v;
+    }
+}
+// total of accumulator blockIdx.x over the workgroups: out[2 s] low and
+// out[2 s + 1] high parts in units of 1 and 2^32
+__global__ __launch_bounds__(kExThreads) void k_exact_totals(const uint64_t *__restrict__ partial, uint32_t nwg,
+                                                             uint64_t *__restrict__ out) {
+    __shared__ uint64_t red[2][kExThreads / 64];
+    uint64_t lo = 0, hi = 0;
+    for (uint32_t i = threadIdx.x; i < nwg; i += kExThreads) {
+        const int64_t v = (int64_t)partial[(uint64_t)blockIdx.x * nwg + i];
+        lo += (uint32_t)v;
+        hi += (uint64_t)(v >> 32);
+    }
+    for (int o = 32; o >= 1; o >>= 1) { lo += __shfl_xor(lo, o, 64); hi += __shfl_xor(hi, o, 64); }
+    if (lane_id() == 0) { red[0][threadIdx.x / 64] = lo; red[1][threadIdx.x / 64] = hi; }
+    __syncthreads();
+    if (threadIdx.x < 2) {
+        uint64_t v = 0;
+        for (int w = 0; w < kExThreads / 64; w++) v += red[threadIdx.x][w];
+        out[2 * blockIdx.x + threadIdx.x] = v;
+    }
+}
+
+// workspace: [totals: bins * 3 * 2 words][flag][partials][exponent buckets]
+struct ExLayout {
+    uint32_t nwg;
+    int bins;
+    size_t flag, partial, under, total;
+};
+ExLayout ex_layout(uint64_t n, int nb) {
+    ExLayout L;
+    const uint64_t chunks = std::max<uint64_t>(1, (n + kExChunk - 1) / kExChunk);
+    // one chunk per workgroup up to 4 workgroups per CU, then up to kExMaxChunks
+    const uint64_t per = std::min<uint64_t>(kExMaxChunks, std::max<uint64_t>(1, chunks / 1024));
+    L.nwg = (uint32_t)((chunks + per - 1) / per);
+    L.bins = nb + 3;
+    L.flag = (size_t)L.bins * 3 * 16;
+    L.partial = L.flag + 16;
+    L.under = L.partial + (size_t)L.bins * 3 * 8 * L.nwg;
+    L.total = L.under + (size_t)L.bins * kExBuckets * 16;
+    return L;
+}
+
+// Sums the totals of the kernel's accumulators: out[k] = main k + the tiny
+// sums that tiny(k) names (bit 0: entry nb + 1, bit 1: entry nb + 2), times
+// 2^scale. grid(i): the grids of entry i.
+template <class GridOf, class TinyOf>
+int exact_finish(const ExLayout &L, int nb, GridOf grid, TinyOf tiny, int scale, double *out, void *ws, hipStream_t s) {
+    char *base = static_cast<char *>(ws);
+    hipLaunchKernelGGL(k_exact_totals, dim3(L.bins * 3), dim3(kExThreads), 0, s,
+                       reinterpret_cast<const uint64_t *>(base + L.partial), L.nwg, reinterpret_cast<uint64_t *>(base));
+    PRODM_CHECK_LAUNCH();
+    std::vector<uint64_t> tot((L.flag + 16) / 8), under;
+    PRODM_HIP(hipMemcpyAsync(tot.data(), base, tot.size() * 8, hipMemcpyDeviceToHost, s));
+    PRODM_HIP(hipStreamSynchronize(s));
+    if (tot[L.flag / 8]) {
+        under.resize((L.total - L.under) / 8);
+        PRODM_HIP(hipMemcpyAsync(under.data(), base + L.under, under.size() * 8, hipMemcpyDeviceToHost, s));
+        PRODM_HIP(hipStreamSynchronize(s));
+    }
+    constexpr int kEmin = -1074;
+    for (int k = 0; k <= nb; k++) {
+        Big b((2048 + 128 + 64 * 4 + 64) / 64 + 2);
+        const int from[3] = {k, tiny(k) & 1 ? nb + 1 : -1, tiny(k) & 2 ? nb + 2 : -1};
+        for (int neg = 0; neg < 2; neg++)
+            for (int i : from) {
+                if (i < 0) continue;
+                const Grid3 g = grid(i);
+                for (int a = 0; a < 3; a++) {
+                    const uint64_t *t = tot.data() + ((size_t)i * 3 + a) * 2;
+                    b.add128(((__int128)(int64_t)t[1] << 32) + (__int128)t[0], g.u[a] - kEmin, neg);
+                }
+                if (!neg && !under.empty())
+                    for (int e = 1; e < kExBuckets; e++) {
+                        b.add_shifted(under[((size_t)i * kExBuckets + e) * 2], e - 1);
+                        b.add_shifted(under[((size_t)i * kExBuckets + e) * 2 + 1], e - 1 + 64);
+                    }
+            }
+        out[k] = std::ldexp(b.to_double(kEmin), scale);
+    }
+    return kOk;
+}
+
+// The thread's elements of chunk c (0 past n): i-th at i * kExThreads + its
+// index. A buffer descriptor ends with the data, so no address is per lane
+// and all loads are in flight together.
+__device__ __forceinline__ void load_chunk(const float *x, uint64_t n, uint64_t c, float (&v)[kExEPT]) {
+    const uint64_t e0 = c * kExChunk;
+    const uint32_t bytes = (uint32_t)min((uint64_t)kExChunk, n - e0) * 4u;
+    const auto r = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(x + e0), 0, bytes, 0x00020000);
+#pragma unroll
+    for (int i = 0; i < kExEPT; i++)
+        v[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, (int)threadIdx.x * 4, i * kExThreads * 4, 0));
+}
+
+// adds term(i), i < kExEPT, in N accumulators and flushes them
+template <int N, class Fn>
+__device__ __forceinline__ void sum_terms(const Grid3 &g, unsigned long long *slot, Fn &&term) {
+    Acc3 A;
+    A.start(g);
+#pragma unroll
+    for (int i = 0; i < kExEPT; i++) {
+        A.add<N>(term(i));
+        // the scheduler would form all terms before the serial sums (256
+        // VGPRs, one wave per SIMD)
+        if (i % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+    }
+    A.flush(slot);
+}
+template <class Fn> __device__ __forceinline__ void sum_bin(const Grid3 &g, unsigned long long *slot, Fn &&term) {
+    if (g.n == 1) sum_terms<1>(g, slot, term);
+    else if (g.n == 2) sum_terms<2>(g, slot, term);
+    else sum_terms<3>(g, slot, term);
+}
+
+}  // namespace
 
 // term of bin k for element x, restating the reference loop (:326-356):
 // bins s_idx, s_idx-1, ... get the squared residual after clearing mantissa
@@ -70,13 +322,106 @@ __device__ inline T sq_term(T x, int de, int le, int nb, int k) {
     return x * x;
 }
 
-template <class T>
-__global__ __launch_bounds__(kSqThreads) void k_collect_squared(const T *__restrict__ x, uint64_t n, int nb, int le,
+// SquaredErrorCollector, float. An element of exponent de has the term
+// (x - x cleared of mantissa bits 0 .. b)^2 in entry k, b = le + 23 - de - k
+// (x^2 from b = 23 on, 0 below b = 0). With le - nb < de <= le its terms are at
+// most 2^(2 (le - k)) and multiples of 2^(2 (le - nb - 23)). Smaller elements
+// have the term x^2 in every entry and are summed once; subnormal ones above
+// that (whose bits do not shift with de) and ones past the bound go term by
+// term to the buckets.
+__host__ __device__ inline Grid3 sq_grid(int k, int le, int nb) {
+    if (k > nb) return grid3_open(2 * (le - nb));
+    const int q = 2 * (le - nb - 23);
+    return grid3(2 * (le - k), q > -149 ? q : -149);
+}
+__global__ __launch_bounds__(kExThreads) void k_collect_squared_f32(const float *__restrict__ x, uint64_t n, int nb,
+                                                                    int le, uint64_t *__restrict__ partial,
+                                                                    unsigned long long *__restrict__ under,
+                                                                    uint32_t *__restrict__ flag) {
+    __shared__ unsigned long long acc[kExBins * 3 * kExSlots];
+    for (int i = threadIdx.x; i < (nb + 3) * 3 * kExSlots; i += kExThreads) acc[i] = 0;
+    __syncthreads();
+    for (uint64_t c = blockIdx.x; c * kExChunk < n; c += gridDim.x) {
+        float v[kExEPT];
+        int cut[kExEPT];  // mantissa bits cleared in entry 0
+        load_chunk(x, n, c, v);
+        uint32_t rest = 0;  // elements not summed by the loops over entries, element 0 in bit 31
+#pragma unroll
+        for (int i = 0; i < kExEPT; i++) {
+            const int de = dev_frexp_exp(v[i]);
+            const float a = fabsf(v[i]);
+            cut[i] = le + 24 - de;
+            const bool main = de > le - nb && de <= le && a >= 1.17549435e-38f && a < __builtin_inff();
+            rest = 2 * rest + (!main && v[i] != 0.0f);
+            v[i] = main ? v[i] : 0.0f;
+            // formed here: left to the loop below, the selects and what they
+            // read would both stay live (256 VGPRs instead of 111)
+            asm volatile("" : "+v"(v[i]), "+v"(cut[i]));
+        }
+        if (__any(rest != 0)) {
+            Acc3 tiny;
+            tiny.start(sq_grid(nb + 1, le, nb));
+            while (rest) {
+                const int i = __clz(rest);  // element 0 is bit 31
+                rest ^= 0x80000000u >> i;
+                const float t = x[c * kExChunk + (uint64_t)i * kExThreads + threadIdx.x];
+                const int de = dev_frexp_exp(t);
+                if (de <= le - nb && fabsf(t) < __builtin_inff()) {
+                    const float tt = t * t;
+                    if (!tiny.add_open((double)tt)) add_under((double)tt, nb + 1, under, flag);
+                } else {
+                    for (int k = 0; k <= nb; k++) add_under((double)sq_term<float>(t, de, le, nb, k), k, under, flag);
+                }
+            }
+            tiny.flush(acc + (nb + 1) * 3 * kExSlots);
+        }
+        for (int k = 0; k <= nb; k++) {
+            sum_bin(sq_grid(k, le, nb), acc + k * 3 * kExSlots, [&](int i) __attribute__((always_inline)) -> double {
+                const int b = cut[i] - k;
+                const uint32_t keep = 0xffffffffu << (b > 23 ? 31 : max(b, 0));
+                const float d = v[i] - from_bits<float>(to_bits(v[i]) & keep);
+                const float t = d * d;
+                return (double)t;
+            });
+        }
+    }
+    __syncthreads();
+    store_partials(acc, nb + 3, partial);
+}
+
+size_t sq_workspace_bytes_f32(uint64_t n, int nb) { return ex_layout(n, nb).total; }
+static int squared_errors_f32(const float *x, uint64_t n, int nb, float maxerr, double *out, void *ws, hipStream_t s) {
+    int le = 0;
+    std::frexp(maxerr, &le);
+    const ExLayout L = ex_layout(n, nb);
+    char *base = static_cast<char *>(ws);
+    uint32_t *flag = reinterpret_cast<uint32_t *>(base + L.flag);
+    if (int rc = launch_fill_u32(flag, 4, 0u, s)) return rc;
+    if (int rc = launch_fill_u64(reinterpret_cast<uint64_t *>(base + L.under), (L.total - L.under) / 8, 0ull, s)) return rc;
+    hipLaunchKernelGGL(k_collect_squared_f32, dim3(L.nwg), dim3(kExThreads), 0, s, x, n, nb, le,
+                       reinterpret_cast<uint64_t *>(base + L.partial),
+                       reinterpret_cast<unsigned long long *>(base + L.under), flag);
+    PRODM_CHECK_LAUNCH();
+    return exact_finish(L, nb, [&](int i) { return sq_grid(i, le, nb); }, [](int) { return 1; }, 0, out, ws, s);
+}
+
+// ---- SquaredErrorCollector, double -------------------------------------------------
+// Terms are doubles over a window of up to 232 bits, accumulated as integers
+// in units of Q = max(q^2, min_sub), q = 2^(le - nb - 52), in per-thread
+// multi-limb registers, reduced across the wave and workgroup with carries,
+// and summed exactly on the host. The rare squares of elements far below
+// the level maximum that are not multiples of Q go to a per-(entry, exponent)
+// histogram of mantissa sums.
+constexpr int kSqLimbs = 4;  // 2^256 > 2^(2 * 64 + 104) * 2^12 terms per workgroup
+constexpr int kSqExpBuckets = 2048, kSqEmin = -1074;
+constexpr int kSqThreads = 256;
+constexpr int kSqEPT = 16;  // elements per thread
+__global__ __launch_bounds__(kSqThreads) void k_collect_squared_f64(const double *__restrict__ x, uint64_t n, int nb, int le,
                                                                 int log2q, uint64_t *__restrict__ partial,
                                                                 unsigned long long *__restrict__ under) {
-    constexpr int LM = SqCfg<T>::kLimbs;
-    constexpr int MB = SqCfg<T>::kMantBits;
+    using T = double;
     using Bits = typename Traits<T>::Bits;
+    constexpr int LM = kSqLimbs, MB = 52;
     __shared__ uint64_t wacc[kSqThreads / 64][65][LM];
     const uint32_t lane = lane_id(), wv = threadIdx.x / 64;
     const uint64_t base = (uint64_t)blockIdx.x * kSqThreads * kSqEPT;
@@ -98,12 +443,12 @@ __global__ __launch_bounds__(kSqThreads) void k_collect_squared(const T *__restr
             const T t = sq_term<T>(v[i], de[i], le, nb, k);
             if (t == (T)0) continue;
             const Bits tb = to_bits<T>(t);
-            const int be = (int)((tb >> MB) & ((1u << (8 * sizeof(T) == 32 ? 8 : 11)) - 1));
+            const int be = (int)((tb >> MB) & ((1u << 11) - 1));
             const uint64_t M = (uint64_t)(tb & (((Bits)1 << MB) - 1)) | (be ? ((uint64_t)1 << MB) : 0);
-            const int E = (be ? be : 1) - 1 + SqCfg<T>::kEmin;  // t = M * 2^E
+            const int E = (be ? be : 1) - 1 + kSqEmin;  // t = M * 2^E
             const int s = E - log2q;
             if (s < 0) {
-                atomicAdd(&under[(size_t)k * SqCfg<T>::kExpBuckets + (be ? be : 1)], (unsigned long long)M);
+                atomicAdd(&under[(size_t)k * kSqExpBuckets + (be ? be : 1)], (unsigned long long)M);
                 continue;
             }
             const int li = s >> 6, off = s & 63;
@@ -165,122 +510,55 @@ __global__ __launch_bounds__(kSqThreads) void k_collect_squared(const T *__restr
     }
 }
 
-// workspace: [header: nwg][partials][underflow histogram]
-template <class T> static uint32_t sq_nwg(uint64_t n) { return (uint32_t)std::max<uint64_t>(1, (n + kSqThreads * kSqEPT - 1) / (kSqThreads * kSqEPT)); }
-template <class T> size_t sq_result_bytes_n(uint64_t n, int nb) {
-    return 64 + (size_t)sq_nwg<T>(n) * (nb + 1) * SqCfg<T>::kLimbs * 8 + (size_t)(nb + 1) * SqCfg<T>::kExpBuckets * 8;
-}
-template <class T> size_t sq_workspace_bytes(uint64_t n, int nb) { return sq_result_bytes_n<T>(n, nb); }
-template size_t sq_workspace_bytes<float>(uint64_t, int);
-template size_t sq_workspace_bytes<double>(uint64_t, int);
 
-// the host copies the whole result area; its size depends on n, so it is
-// encoded in the header written by the launch
-static thread_local size_t g_sq_last_bytes = 0;
-template <class T> size_t sq_result_bytes(int) { return g_sq_last_bytes; }
-template size_t sq_result_bytes<float>(int);
-template size_t sq_result_bytes<double>(int);
-
-template <class T> static int log2_quantum(int le, int nb) {
-    const long q2 = 2L * ((long)le - nb - Traits<T>::kPrec);
-    return (int)std::max<long>(q2, SqCfg<T>::kEmin);
-}
-
-template <class T>
-int launch_collect_squared(const T *x, uint64_t n, int nb, T maxerr, void *ws, size_t ws_bytes, hipStream_t s) {
+// workspace: [partials][underflow histogram]
+static uint32_t sq_nwg(uint64_t n) { return (uint32_t)std::max<uint64_t>(1, (n + kSqThreads * kSqEPT - 1) / (kSqThreads * kSqEPT)); }
+static size_t sq_partial_bytes(uint64_t n, int nb) { return (size_t)sq_nwg(n) * (nb + 1) * kSqLimbs * 8; }
+static size_t sq_under_bytes(int nb) { return (size_t)(nb + 1) * kSqExpBuckets * 8; }
+static int squared_errors_f64(const double *x, uint64_t n, int nb, double maxerr, double *out, void *ws,
+                              hipStream_t s) {
     int le = 0;
     std::frexp(maxerr, &le);
-    const uint32_t nwg = sq_nwg<T>(n);
-    const size_t bytes = sq_result_bytes_n<T>(n, nb);
-    if (ws_bytes < bytes) { set_error("squared collector: workspace too small"); return kErrArg; }
-    g_sq_last_bytes = bytes;
-    char *base = static_cast<char *>(ws);
-    uint64_t *hdr = reinterpret_cast<uint64_t *>(base);
-    uint64_t *partial = reinterpret_cast<uint64_t *>(base + 64);
-    unsigned long long *under =
-        reinterpret_cast<unsigned long long *>(base + 64 + (size_t)nwg * (nb + 1) * SqCfg<T>::kLimbs * 8);
-    int rc = launch_fill_u64(hdr, 8, 0ull, s);
-    if (!rc) rc = launch_fill_u64(hdr, 1, (uint64_t)nwg, s);
-    if (!rc) rc = launch_fill_u64(reinterpret_cast<uint64_t *>(under), (size_t)(nb + 1) * SqCfg<T>::kExpBuckets, 0ull, s);
-    if (rc) return rc;
+    const int log2q = (int)std::max<long>(2L * ((long)le - nb - 52), kSqEmin);
+    const uint32_t nwg = sq_nwg(n);
+    const size_t pb = sq_partial_bytes(n, nb), ub = sq_under_bytes(nb);
+    uint64_t *partial = static_cast<uint64_t *>(ws);
+    unsigned long long *under = reinterpret_cast<unsigned long long *>(static_cast<char *>(ws) + pb);
+    if (int rc = launch_fill_u64(reinterpret_cast<uint64_t *>(under), ub / 8, 0ull, s)) return rc;
     if (n == 0) {
-        return launch_fill_u64(partial, (size_t)nwg * (nb + 1) * SqCfg<T>::kLimbs, 0ull, s);
+        if (int rc = launch_fill_u64(partial, pb / 8, 0ull, s)) return rc;
+    } else {
+        hipLaunchKernelGGL(k_collect_squared_f64, dim3(nwg), dim3(kSqThreads), 0, s, x, n, nb, le, log2q, partial, under);
+        PRODM_CHECK_LAUNCH();
     }
-    hipLaunchKernelGGL(k_collect_squared<T>, dim3(nwg), dim3(kSqThreads), 0, s, x, n, nb, le, log2_quantum<T>(le, nb),
-                       partial, under);
-    PRODM_CHECK_LAUNCH();
-    return kOk;
-}
-template int launch_collect_squared<float>(const float *, uint64_t, int, float, void *, size_t, hipStream_t);
-template int launch_collect_squared<double>(const double *, uint64_t, int, double, void *, size_t, hipStream_t);
-
-// ---- exact host summation and rounding ---------------------------------------------
-namespace {
-struct Big {
-    std::vector<uint64_t> w;  // little endian
-    explicit Big(size_t limbs) : w(limbs, 0) {}
-    void add_shifted(uint64_t v, int shift) {  // v << shift, shift >= 0
-        if (!v) return;
-        const size_t li = (size_t)shift / 64;
-        const int off = shift % 64;
-        uint64_t parts[2] = {v << off, off ? (v >> (64 - off)) : 0};
-        uint64_t carry = 0;
-        for (size_t j = li; j < w.size(); j++) {
-            const uint64_t add = (j - li < 2) ? parts[j - li] : 0;
-            if (j - li >= 2 && !carry) break;
-            const uint64_t s1 = w[j] + add;
-            const uint64_t c1 = s1 < add;
-            const uint64_t s2 = s1 + carry;
-            const uint64_t c2 = s2 < carry;
-            w[j] = s2;
-            carry = c1 | c2;
-        }
-    }
-    int bit(long i) const { return i < 0 ? 0 : (int)((w[(size_t)i / 64] >> (i % 64)) & 1u); }
-    // value * 2^scale rounded to nearest even
-    double to_double(int scale) const {
-        long top = -1;
-        for (long i = (long)w.size() - 1; i >= 0; i--)
-            if (w[i]) { top = i * 64 + 63 - __builtin_clzll(w[i]); break; }
-        if (top < 0) return 0.0;
-        if (top <= 52) return std::ldexp((double)w[0], scale);
-        const long lsb = top - 52;
-        uint64_t mant = 0;
-        for (long b = top; b >= lsb; b--) mant = (mant << 1) | (uint64_t)bit(b);
-        const int rb = bit(lsb - 1);
-        int sticky = 0;
-        for (long b = lsb - 2; b >= 0 && !sticky; b--) sticky = bit(b);
-        if (rb && (sticky || (mant & 1u))) mant++;
-        return std::ldexp((double)mant, (int)(scale + lsb));
-    }
-};
-}  // namespace
-
-template <class T> int finish_collect_squared(const void *h, int nb, T maxerr, double *out) {
-    constexpr int LM = SqCfg<T>::kLimbs;
-    constexpr int NE = SqCfg<T>::kExpBuckets;
-    int le = 0;
-    std::frexp(maxerr, &le);
-    const int log2q = log2_quantum<T>(le, nb);
-    const uint8_t *base = static_cast<const uint8_t *>(h);
-    uint64_t nwg;
-    std::memcpy(&nwg, base, 8);
-    const uint64_t *partial = reinterpret_cast<const uint64_t *>(base + 64);
-    const uint64_t *under = partial + nwg * (nb + 1) * LM;
+    std::vector<uint64_t> host((pb + ub) / 8);
+    PRODM_HIP(hipMemcpyAsync(host.data(), ws, pb + ub, hipMemcpyDeviceToHost, s));
+    PRODM_HIP(hipStreamSynchronize(s));
+    const uint64_t *hp = host.data(), *hu = host.data() + pb / 8;
     // common scale: 2^emin; window terms sit at 2^log2q = 2^emin * 2^(log2q - emin)
-    const int wshift = log2q - SqCfg<T>::kEmin;
-    const size_t limbs = (size_t)(wshift + 64 * LM + 64 + 64 + 2 * 1100) / 64 + 2;
+    const int wshift = log2q - kSqEmin;
+    const size_t limbs = (size_t)(wshift + 64 * kSqLimbs + 64 + 64 + 2 * 1100) / 64 + 2;
     for (int k = 0; k <= nb; k++) {
         Big b(limbs);
         for (uint64_t g = 0; g < nwg; g++)
-            for (int j = 0; j < LM; j++) b.add_shifted(partial[(g * (nb + 1) + k) * LM + j], wshift + 64 * j);
-        for (int e = 1; e < NE; e++) b.add_shifted(under[(size_t)k * NE + e], e - 1);
-        out[k] = b.to_double(SqCfg<T>::kEmin);
+            for (int j = 0; j < kSqLimbs; j++) b.add_shifted(hp[(g * (nb + 1) + k) * kSqLimbs + j], wshift + 64 * j);
+        for (int e = 1; e < kSqExpBuckets; e++) b.add_shifted(hu[(size_t)k * kSqExpBuckets + e], e - 1);
+        out[k] = b.to_double(kSqEmin);
     }
     return kOk;
 }
-template int finish_collect_squared<float>(const void *, int, float, double *);
-template int finish_collect_squared<double>(const void *, int, double, double *);
+
+template <class T> size_t sq_workspace_bytes(uint64_t n, int nb) {
+    return sizeof(T) == 4 ? sq_workspace_bytes_f32(n, nb) : 64 + sq_partial_bytes(n, nb) + sq_under_bytes(nb);
+}
+template size_t sq_workspace_bytes<float>(uint64_t, int);
+template size_t sq_workspace_bytes<double>(uint64_t, int);
+template <> int squared_errors<float>(const float *x, uint64_t n, int nb, float maxerr, double *out, void *ws, hipStream_t s) {
+    return squared_errors_f32(x, n, nb, maxerr, out, ws, s);
+}
+template <> int squared_errors<double>(const double *x, uint64_t n, int nb, double maxerr, double *out, void *ws, hipStream_t s) {
+    return squared_errors_f64(x, n, nb, maxerr, out, ws, s);
+}
 
 // ---- encoder-fused level errors ------------------------------------------------------
 // NegaBinaryBPEncoder::encode(..., level_errors) (NegaBinaryBPEncoder.hpp:65-125,
@@ -293,19 +571,13 @@ template int finish_collect_squared<double>(const void *, int, double, double *)
 // reference does. Each entry is the exactly rounded sum over elements, then
 // scaled by 2^(2 (e - nb)).
 //
-// Exactness: in shifted units every term of an element with |s| >= 1 is a
-// multiple of 2^-46 (the fraction's step is at least 2^-23) and every term
-// of an element with 2^-32 <= |s| < 1 a multiple of 2^-110, so terms are
-// integers in units of Q = 2^-110 below 2^176 (3 limbs, 2^13 terms per
-// workgroup). Terms of smaller elements go to a per-(bin, exponent)
-// histogram of 128-bit mantissa sums.
+// Exactness: an element with 1 <= |s| < 2^min(nb, 31) has terms of at most
+// 2^(2 (nb - k) + 2) in entry k that are multiples of 2^-46 (the fraction's step
+// is at least 2^-23). One with |s| < 1 has no digit: its term is s^2 in every
+// entry, as a double, or squared in float where the reference squares in
+// float; both are summed once. Larger ones (an exponent below the data's) go
+// term by term to the buckets.
 namespace {
-constexpr int kFeLimbs = 3;
-constexpr int kFeLog2Q = -110;
-constexpr int kFeThreads = 256;
-constexpr int kFeEPT = 32;
-constexpr int kFeExpBuckets = 2048;
-
 __device__ __forceinline__ uint32_t fe_mask(int k) { return k >= 31 ? 0x7fffffffu : ((1u << k) - 1u); }
 
 template <int ENC>
@@ -325,163 +597,123 @@ __device__ __forceinline__ double fe_term(float s, float m, uint32_t bits, int n
     return d * d;
 }
 
+
+// an element's shifted value (its magnitude for GroupedBP), fraction and digits
 template <int ENC>
-__global__ __launch_bounds__(kFeThreads) void k_fused_errors(const float *__restrict__ x, uint64_t n, int shift,
-                                                             int nb, uint64_t *__restrict__ partial,
-                                                             unsigned long long *__restrict__ under) {
-    constexpr int LM = kFeLimbs;
-    __shared__ uint64_t wacc[kFeThreads / 64][33][LM];
-    const uint32_t lane = lane_id(), wv = threadIdx.x / 64;
-    const uint64_t base = (uint64_t)blockIdx.x * kFeThreads * kFeEPT;
-    float s[kFeEPT], m[kFeEPT];
-    uint32_t bits[kFeEPT];
-#pragma unroll
-    for (int i = 0; i < kFeEPT; i++) {
-        const uint64_t e = base + (uint64_t)i * kFeThreads + threadIdx.x;
-        // unconditional load (past n: element 0, discarded), so that the
-        // loads of all elements are in flight together
-        const float x0 = x[e < n ? e : 0];
-        const float v = e < n ? x0 : 0.0f;
-        const float sh = ldexpf(v, shift);
-        if (ENC == 0) {
-            // (int32) shifted as in the reference (in range: |x| < 2^e)
-            const int32_t q = (sh == sh && fabsf(sh) < 2147483648.0f) ? (int32_t)sh : (int32_t)0x80000000;
-            bits[i] = ((uint32_t)q + 0xaaaaaaaau) ^ 0xaaaaaaaau;
-            s[i] = sh;
-            m[i] = sh - (float)q;
-        } else {
-            const float a = fabsf(sh);
-            const uint32_t fp = (a == a && a < 4294967296.0f) ? (uint32_t)a : 0u;
-            bits[i] = fp;
-            s[i] = a;
-            m[i] = a - (float)fp;
-        }
+__device__ __forceinline__ void fe_split(float x, int shift, float &s, float &m, uint32_t &bits) {
+    const float sh = ldexpf(x, shift);
+    const float a = fabsf(sh);
+    if (ENC == 0) {
+        // (int32) shifted as in the reference (in range: |x| < 2^e)
+        const int32_t q = (sh == sh && a < 2147483648.0f) ? (int32_t)sh : (int32_t)0x80000000;
+        bits = ((uint32_t)q + 0xaaaaaaaau) ^ 0xaaaaaaaau;
+        s = sh;
+        m = sh - (float)q;
+    } else {
+        const uint32_t fp = (a == a && a < 4294967296.0f) ? (uint32_t)a : 0u;
+        bits = fp;
+        s = a;
+        m = a - (float)fp;
     }
-    for (int bin = 0; bin <= nb; bin++) {
-        uint64_t a[LM];
+}
+
+constexpr int kFeQ = -46;
+__host__ __device__ inline Grid3 fe_grid(int k, int nb) {
+    return k > nb ? grid3_open(0) : grid3(2 * (nb - k) + 2, kFeQ);
+}
+
+template <int ENC>
+__global__ __launch_bounds__(kExThreads) void k_fused_errors(const float *__restrict__ x, uint64_t n, int shift,
+                                                             int nb, uint64_t *__restrict__ partial,
+                                                             unsigned long long *__restrict__ under,
+                                                             uint32_t *__restrict__ flag) {
+    __shared__ unsigned long long acc[kExBins * 3 * kExSlots];
+    for (int i = threadIdx.x; i < (nb + 3) * 3 * kExSlots; i += kExThreads) acc[i] = 0;
+    __syncthreads();
+    const float top = ldexpf(1.0f, min(nb, 31));
+    for (uint64_t c = blockIdx.x; c * kExChunk < n; c += gridDim.x) {
+        float m[kExEPT];
+        uint32_t bits[kExEPT];
+        load_chunk(x, n, c, m);
+        uint32_t rest = 0;  // elements not summed by the loops over entries, element 0 in bit 31
 #pragma unroll
-        for (int j = 0; j < LM; j++) a[j] = 0;
-#pragma unroll 4
-        for (int i = 0; i < kFeEPT; i++) {
-            const double t = fe_term<ENC>(s[i], m[i], bits[i], nb, bin);
-            if (t == 0.0) continue;
-            uint64_t tb;
-            __builtin_memcpy(&tb, &t, 8);
-            const int be = (int)((tb >> 52) & 0x7ff);
-            const uint64_t M = (tb & ((1ull << 52) - 1)) | (be ? (1ull << 52) : 0);
-            const int E = (be ? be : 1) - 1075;  // t = M 2^E
-            const int sft = E - kFeLog2Q;
-            if (sft < 0) {
-                // 128-bit bucket: low word with carry into the high word
-                unsigned long long *bk = under + ((size_t)bin * kFeExpBuckets + (be ? be : 1)) * 2;
-                const unsigned long long old = atomicAdd(bk, (unsigned long long)M);
-                if (old + M < old) atomicAdd(bk + 1, 1ull);
-                continue;
-            }
-            const int li = sft >> 6, off = sft & 63;
-            const uint64_t plo = M << off;
-            const uint64_t phi = off ? (M >> (64 - off)) : 0;
-            uint64_t carry = 0;
-#pragma unroll
-            for (int j = 0; j < LM; j++) {
-                const uint64_t add = (j == li ? plo : 0) + (j == li + 1 ? phi : 0);
-                const uint64_t s1 = a[j] + add;
-                const uint64_t c1 = s1 < add;
-                const uint64_t s2 = s1 + carry;
-                const uint64_t c2 = s2 < carry;
-                a[j] = s2;
-                carry = c1 | c2;
-            }
+        for (int i = 0; i < kExEPT; i++) {
+            float s;
+            fe_split<ENC>(m[i], shift, s, m[i], bits[i]);
+            const float a = fabsf(s);
+            const bool main = a >= 1.0f && a < top;
+            rest = 2 * rest + (!main && s != 0.0f);
+            m[i] = main ? m[i] : 0.0f;
+            bits[i] = main ? bits[i] : 0u;
+            asm volatile("" : "+v"(m[i]), "+v"(bits[i]));  // as above
         }
-        for (int o = 32; o >= 1; o >>= 1) {
-            uint64_t b[LM];
-#pragma unroll
-            for (int j = 0; j < LM; j++) b[j] = __shfl_xor(a[j], o, 64);
-            uint64_t carry = 0;
-#pragma unroll
-            for (int j = 0; j < LM; j++) {
-                const uint64_t s1 = a[j] + b[j];
-                const uint64_t c1 = s1 < b[j];
-                const uint64_t s2 = s1 + carry;
-                const uint64_t c2 = s2 < carry;
-                a[j] = s2;
-                carry = c1 | c2;
+        if (__any(rest != 0)) {
+            Acc3 tinyd, tinyf;
+            tinyd.start(fe_grid(nb + 1, nb));
+            tinyf.start(fe_grid(nb + 2, nb));
+            while (rest) {
+                const int i = __clz(rest);  // element 0 is bit 31
+                rest ^= 0x80000000u >> i;
+                float s, mm;
+                uint32_t bb;
+                fe_split<ENC>(x[c * kExChunk + (uint64_t)i * kExThreads + threadIdx.x], shift, s, mm, bb);
+                if (fabsf(s) < 1.0f) {
+                    const double d = (double)s * (double)s;
+                    const float ff = s * s;
+                    if (!tinyd.add_open(d)) add_under(d, nb + 1, under, flag);
+                    if (!tinyf.add_open((double)ff)) add_under((double)ff, nb + 2, under, flag);
+                } else {
+                    for (int k = 0; k <= nb; k++) add_under(fe_term<ENC>(s, mm, bb, nb, k), k, under, flag);
+                }
             }
+            tinyd.flush(acc + (nb + 1) * 3 * kExSlots);
+            tinyf.flush(acc + (nb + 2) * 3 * kExSlots);
         }
-        if (lane == 0) {
-#pragma unroll
-            for (int j = 0; j < LM; j++) wacc[wv][bin][j] = a[j];
+        // entries 0 and nb: s = digits + fraction again, exactly
+        sum_bin(fe_grid(0, nb), acc, [&](int i) __attribute__((always_inline)) -> double {
+            const float q = ENC == 0 ? (float)(int32_t)((bits[i] ^ 0xaaaaaaaau) - 0xaaaaaaaau) : (float)bits[i];
+            return fe_term<ENC>(q + m[i], m[i], bits[i], nb, 0);
+        });
+        sum_bin(fe_grid(nb, nb), acc + nb * 3 * kExSlots,
+                [&](int i) __attribute__((always_inline)) -> double { return fe_term<ENC>(0.0f, m[i], bits[i], nb, nb); });
+        for (int k = 1; k < nb; k++) {
+            const uint32_t mask = fe_mask(nb - k);
+            sum_bin(fe_grid(k, nb), acc + k * 3 * kExSlots, [&](int i) __attribute__((always_inline)) -> double {
+                const uint32_t low = bits[i] & mask;
+                const double v = ENC == 0 ? (double)(int32_t)((low ^ 0xaaaaaaaau) - 0xaaaaaaaau) : (double)low;
+                const double d = v + (double)m[i];
+                return d * d;
+            });
         }
     }
     __syncthreads();
-    for (int bin = threadIdx.x; bin <= nb; bin += kFeThreads) {
-        uint64_t a[LM];
-#pragma unroll
-        for (int j = 0; j < LM; j++) a[j] = 0;
-        for (int w = 0; w < kFeThreads / 64; w++) {
-            uint64_t carry = 0;
-#pragma unroll
-            for (int j = 0; j < LM; j++) {
-                const uint64_t bj = wacc[w][bin][j];
-                const uint64_t s1 = a[j] + bj;
-                const uint64_t c1 = s1 < bj;
-                const uint64_t s2 = s1 + carry;
-                const uint64_t c2 = s2 < carry;
-                a[j] = s2;
-                carry = c1 | c2;
-            }
-        }
-#pragma unroll
-        for (int j = 0; j < LM; j++) partial[((uint64_t)blockIdx.x * (nb + 1) + bin) * LM + j] = a[j];
-    }
+    store_partials(acc, nb + 3, partial);
 }
-
-uint32_t fe_nwg(uint64_t n) { return (uint32_t)std::max<uint64_t>(1, (n + kFeThreads * kFeEPT - 1) / (kFeThreads * kFeEPT)); }
-size_t fe_partial_bytes(uint64_t n, int nb) { return (size_t)fe_nwg(n) * (nb + 1) * kFeLimbs * 8; }
-size_t fe_under_bytes(int nb) { return (size_t)(nb + 1) * kFeExpBuckets * 16; }
 }  // namespace
 
-size_t fused_errors_workspace_bytes(uint64_t n, int nb) {
-    return fe_partial_bytes(n, nb) + fe_under_bytes(nb);
-}
+size_t fused_errors_workspace_bytes(uint64_t n, int nb) { return ex_layout(n, nb).total; }
 
 int fused_level_errors(int enc, const float *x, uint64_t n, int32_t exp, int nb, double *out, void *ws,
                        size_t ws_bytes, hipStream_t s) {
     if (nb < 1 || nb > 32 || !out || (enc != 0 && enc != 1)) { set_error("level errors: bad arguments"); return kErrArg; }
     if (n > 0 && !x) { set_error("level errors: null input"); return kErrArg; }
-    const size_t pb = fe_partial_bytes(n, nb), ub = fe_under_bytes(nb);
-    if (ws_bytes < pb + ub || !ws) { set_error("level errors: workspace too small"); return kErrArg; }
+    const ExLayout L = ex_layout(n, nb);
+    if (ws_bytes < L.total || !ws) { set_error("level errors: workspace too small"); return kErrArg; }
     const int e = enc == 0 ? exp + 2 : exp;  // NegaBinaryBPEncoder.hpp:68
-    uint64_t *partial = static_cast<uint64_t *>(ws);
-    unsigned long long *under = reinterpret_cast<unsigned long long *>(static_cast<char *>(ws) + pb);
-    const uint32_t nwg = fe_nwg(n);
-    int rc = launch_fill_u64(reinterpret_cast<uint64_t *>(under), ub / 8, 0ull, s);
-    if (!rc && n == 0) rc = launch_fill_u64(partial, pb / 8, 0ull, s);
-    if (rc) return rc;
-    if (n) {
-        if (enc == 0)
-            hipLaunchKernelGGL(k_fused_errors<0>, dim3(nwg), dim3(kFeThreads), 0, s, x, n, nb - e, nb, partial, under);
-        else
-            hipLaunchKernelGGL(k_fused_errors<1>, dim3(nwg), dim3(kFeThreads), 0, s, x, n, nb - e, nb, partial, under);
-        PRODM_CHECK_LAUNCH();
-    }
-    std::vector<uint64_t> host((pb + ub) / 8);
-    PRODM_HIP(hipMemcpyAsync(host.data(), ws, pb + ub, hipMemcpyDeviceToHost, s));
-    PRODM_HIP(hipStreamSynchronize(s));
-    const uint64_t *hp = host.data(), *hu = host.data() + pb / 8;
-    const int wshift = kFeLog2Q - (-1074);
-    const size_t limbs = (size_t)(2048 + 128 + 64 * kFeLimbs + 64) / 64 + 2;
-    for (int k = 0; k <= nb; k++) {
-        Big b(limbs);
-        for (uint32_t g = 0; g < nwg; g++)
-            for (int j = 0; j < kFeLimbs; j++) b.add_shifted(hp[((uint64_t)g * (nb + 1) + k) * kFeLimbs + j], wshift + 64 * j);
-        for (int slot = 1; slot < kFeExpBuckets; slot++) {
-            b.add_shifted(hu[((size_t)k * kFeExpBuckets + slot) * 2], slot - 1);
-            b.add_shifted(hu[((size_t)k * kFeExpBuckets + slot) * 2 + 1], slot - 1 + 64);
-        }
-        out[k] = std::ldexp(b.to_double(-1074), 2 * (e - nb));
-    }
-    return kOk;
+    char *base = static_cast<char *>(ws);
+    uint64_t *partial = reinterpret_cast<uint64_t *>(base + L.partial);
+    unsigned long long *under = reinterpret_cast<unsigned long long *>(base + L.under);
+    uint32_t *flag = reinterpret_cast<uint32_t *>(base + L.flag);
+    if (int rc = launch_fill_u32(flag, 4, 0u, s)) return rc;
+    if (int rc = launch_fill_u64(reinterpret_cast<uint64_t *>(under), (L.total - L.under) / 8, 0ull, s)) return rc;
+    if (enc == 0)
+        hipLaunchKernelGGL(k_fused_errors<0>, dim3(L.nwg), dim3(kExThreads), 0, s, x, n, nb - e, nb, partial, under, flag);
+    else
+        hipLaunchKernelGGL(k_fused_errors<1>, dim3(L.nwg), dim3(kExThreads), 0, s, x, n, nb - e, nb, partial, under, flag);
+    PRODM_CHECK_LAUNCH();
+    // entries whose terms of tiny elements are squared in float take the second sum
+    return exact_finish(L, nb, [&](int i) { return fe_grid(i, nb); },
+                        [&](int k) { return k == 0 || (enc == 0 && k == nb) ? 2 : 1; }, 2 * (e - nb), out, ws, s);
 }
 
 }  // namespace prodm

@@ -87,13 +87,10 @@ int launch_interleave(const T *data, const uint64_t *strides3, const uint32_t *f
                       bool reposition, hipStream_t s);
 
 // ---- squared error collector (SquaredErrorCollector.hpp:23-65) ---------------
+// Exactly rounded table of nb + 1 doubles on the host; synchronizes.
 template <class T> size_t sq_workspace_bytes(uint64_t n, int nb);
 template <class T>
-int launch_collect_squared(const T *x, uint64_t n, int nb, T max_level_error, void *ws, size_t ws_bytes,
-                           hipStream_t s);
-// finishes on the host after the stream is synchronized: exact rounding
-template <class T> int finish_collect_squared(const void *h_ws_copy, int nb, T max_level_error, double *out);
-template <class T> size_t sq_result_bytes(int nb);
+int squared_errors(const T *x, uint64_t n, int nb, T max_level_error, double *out, void *ws, hipStream_t s);
 
 // ---- encoder-fused level errors (NegaBinaryBPEncoder.hpp:65-125,231-239,
 // GroupedBPEncoder.hpp:76-145,324-335), fp32: enc 0 NegaBinary, 1 GroupedBP.
