@@ -31,7 +31,7 @@ FLAGS = [
 ]
 
 
-HOST_FLAGS = ["-O2", "-std=c++17", "-fPIC", "-Wall"]
+HOST_FLAGS = ["-O3", "-std=c++17", "-fPIC", "-Wall", "-pthread"]
 
 
 def _compile(src):

@@ -275,6 +275,8 @@ static void plan_free(prodm_mdr_plan *p) {
     for (hipEvent_t e : p->lev_ev)
         if (e) (void)hipEventDestroy(e);
     if (p->join_ev) (void)hipEventDestroy(p->join_ev);
+    if (p->pin) (void)hipHostFree(p->pin);
+    if (p->pin_ev) (void)hipEventDestroy(p->pin_ev);
     if (p->side) (void)hipStreamDestroy(p->side);
     if (p->side2) (void)hipStreamDestroy(p->side2);
     void *ptrs[] = {p->ws, p->levels, p->keys, p->planes, p->rb, p->words, p->signs, p->gbws, p->flev};
@@ -363,47 +365,98 @@ template <class T> static int plan_refactor(prodm_mdr_plan *p, const T *in, hipS
     return kOk;
 }
 
+// Pinned staging of a plan's host decode, at most kPinMax bytes (allocated on
+// first use, freed with the plan).
+constexpr size_t kPinMax = size_t(64) << 20;
+static int plan_pin(prodm_mdr_plan *p, size_t bytes) {
+    if (p->pin_bytes >= bytes) return kOk;
+    if (!p->pin_ev) PRODM_HIP(hipEventCreateWithFlags(&p->pin_ev, hipEventDisableTiming));
+    if (p->pin) { PRODM_HIP(hipHostFree(p->pin)); p->pin = nullptr; p->pin_bytes = 0; }
+    PRODM_HIP(hipHostMalloc(&p->pin, bytes, hipHostMallocDefault));
+    p->pin_bytes = bytes;
+    return kOk;
+}
+
 // PerBit planes [0, k[l]) of every level decoded on the host (the streams
 // have no index of where an element's bits begin) into the level buffers.
-// Synchronizes the stream.
+// Plane bytes and values go through the pinned staging, so that every copy of
+// the retrieval is queued before the one wait for it, and the values of a
+// level travel back while the next is decoded; a retrieval that does not fit
+// it copies level by level through pageable memory. Waits for the stream.
 template <class T> static int perbit_decode_levels(prodm_mdr_plan *p, const uint8_t *k, hipStream_t s) {
     const LevelGeom &g = p->g;
+    if (p->pin_ev) PRODM_HIP(hipEventSynchronize(p->pin_ev));  // the last call's uploads have left the staging
+    const size_t nsizes = (size_t)(g.L + 1) * p->nb;
+    std::vector<uint32_t> sizes(nsizes);
+    std::vector<KeyOf<T>> keys(g.L + 1);
+    PRODM_HIP(hipMemcpyAsync(sizes.data(), p->words, nsizes * 4, hipMemcpyDeviceToHost, s));
+    PRODM_HIP(hipMemcpyAsync(keys.data(), p->keys, keys.size() * sizeof(T), hipMemcpyDeviceToHost, s));
     PRODM_HIP(hipStreamSynchronize(s));
-    std::vector<uint32_t> sizes((size_t)(g.L + 1) * p->nb);
-    PRODM_HIP(hipMemcpy(sizes.data(), p->words, sizes.size() * 4, hipMemcpyDeviceToHost));
+    // a small level's planes come as they lie, in one copy; a large one's each
+    // by itself, without the unused ends
+    auto whole = [&](int l) { return k[l] * p->plane_stride[l] * p->elem <= (size_t(1) << 20); };
+    auto level_bytes = [&](int l) -> size_t {
+        size_t b = (g.elems[l] * sizeof(T) + 255) & ~(size_t)255;
+        if (whole(l)) return b + k[l] * p->plane_stride[l] * p->elem;
+        for (int i = 0; i < k[l]; i++) b += ((size_t)sizes[(size_t)l * p->nb + i] + 7) / 8 * 8;
+        return b;
+    };
+    size_t need = 0;
+    for (int l = 0; l <= g.L; l++) need += (level_bytes(l) + 255) & ~(size_t)255;
+    const bool pinned = need <= kPinMax;
+    if (pinned)
+        if (int rc = plan_pin(p, need)) return rc;
+    std::vector<uint8_t> paged;
+    std::vector<std::vector<const uint64_t *>> ptrs(g.L + 1);
+    std::vector<T *> vals(g.L + 1);
+    // places of level l's values and planes in `at`, and the copies of its planes
+    auto fetch = [&](int l, char *at) -> int {
+        vals[l] = reinterpret_cast<T *>(at);
+        at += (g.elems[l] * sizeof(T) + 255) & ~(size_t)255;
+        const size_t pitch = p->plane_stride[l] * p->elem;
+        const char *base = static_cast<const char *>(p->planes) + p->elem * p->plane_off[l];
+        ptrs[l].assign(k[l] ? k[l] : 1, nullptr);
+        if (whole(l) && k[l]) PRODM_HIP(hipMemcpyAsync(at, base, k[l] * pitch, hipMemcpyDeviceToHost, s));
+        for (int i = 0; i < k[l]; i++) {
+            const size_t bytes = sizes[(size_t)l * p->nb + i];
+            if (bytes > pitch) { set_error("retrieve: plane larger than its storage"); return kErrState; }
+            ptrs[l][i] = reinterpret_cast<const uint64_t *>(at);
+            if (!whole(l) && bytes) PRODM_HIP(hipMemcpyAsync(at, base + i * pitch, bytes, hipMemcpyDeviceToHost, s));
+            at += whole(l) ? pitch : (bytes + 7) / 8 * 8;
+        }
+        return kOk;
+    };
+    if (pinned) {
+        char *at = static_cast<char *>(p->pin);
+        for (int l = 0; l <= g.L; l++) {
+            if (int rc = fetch(l, at)) return rc;
+            at += (level_bytes(l) + 255) & ~(size_t)255;
+        }
+        PRODM_HIP(hipStreamSynchronize(s));
+    }
     prodm_perbit_state *st = nullptr;
     if (int rc = prodm_perbit_state_create(&st)) return rc;
     int rc = kOk;
-    std::vector<T> vals;
-    std::vector<std::vector<uint64_t>> words;
     for (int l = 0; l <= g.L && !rc; l++) {
         const uint64_t n = g.elems[l];
-        double mx;
-        int32_t e;
-        if ((rc = prodm_mdr_level_info(p, l, &mx, &e, nullptr))) break;
-        words.assign(k[l], {});
-        std::vector<const uint64_t *> ptrs(k[l] ? k[l] : 1);
-        const char *base = static_cast<const char *>(p->planes) + p->elem * p->plane_off[l];
-        for (int i = 0; i < k[l]; i++) {
-            const uint32_t bytes = sizes[(size_t)l * p->nb + i];
-            words[i].resize(bytes / 8 + 1);
-            if (bytes)
-                if (hipMemcpy(words[i].data(), base + p->elem * p->plane_stride[l] * i, bytes, hipMemcpyDeviceToHost) !=
-                    hipSuccess) { set_error("retrieve: plane copy"); rc = kErrHip; break; }
-            ptrs[i] = words[i].data();
+        if (!pinned) {
+            paged.resize(level_bytes(l) + 256);
+            if ((rc = fetch(l, reinterpret_cast<char *>(paged.data())))) break;
+            if (hipStreamSynchronize(s) != hipSuccess) { set_error("retrieve: plane copy"); rc = kErrHip; break; }
         }
-        if (rc) break;
-        vals.resize(n ? n : 1);
-        std::vector<uint32_t> sz(k[l] ? k[l] : 1);
-        for (int i = 0; i < k[l]; i++) sz[i] = sizes[(size_t)l * p->nb + i];
-        rc = sizeof(T) == 4 ? prodm_perbit_decode_f32(st, l, ptrs.data(), sz.data(), (uint32_t)n, e, 0, k[l],
-                                                      reinterpret_cast<float *>(vals.data()))
-                            : prodm_perbit_decode_f64(st, l, ptrs.data(), sz.data(), (uint32_t)n, e, 0, k[l],
-                                                      reinterpret_cast<double *>(vals.data()));
+        int e = 0;
+        std::frexp(key_to_value<T>((uint64_t)keys[l]), &e);
+        const uint32_t *sz = sizes.data() + (size_t)l * p->nb;
+        rc = sizeof(T) == 4 ? prodm_perbit_decode_f32(st, l, ptrs[l].data(), sz, (uint32_t)n, e, 0, k[l],
+                                                      reinterpret_cast<float *>(vals[l]))
+                            : prodm_perbit_decode_f64(st, l, ptrs[l].data(), sz, (uint32_t)n, e, 0, k[l],
+                                                      reinterpret_cast<double *>(vals[l]));
+        T *dst = static_cast<T *>(p->levels) + p->level_off[l];
         if (!rc && n &&
-            hipMemcpy(static_cast<T *>(p->levels) + p->level_off[l], vals.data(), n * sizeof(T), hipMemcpyHostToDevice) !=
-                hipSuccess) { set_error("retrieve: level upload"); rc = kErrHip; }
+            (hipMemcpyAsync(dst, vals[l], n * sizeof(T), hipMemcpyHostToDevice, s) != hipSuccess ||
+             (!pinned && hipStreamSynchronize(s) != hipSuccess))) { set_error("retrieve: level upload"); rc = kErrHip; }
     }
+    if (pinned && hipEventRecord(p->pin_ev, s) != hipSuccess && !rc) { set_error("retrieve: event record"); rc = kErrHip; }
     prodm_perbit_state_destroy(st);
     return rc;
 }

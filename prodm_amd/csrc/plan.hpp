@@ -40,6 +40,9 @@ struct prodm_mdr_plan {
     hipStream_t side2 = nullptr;  // retrieve: the finest level's decode and load sweep
     hipEvent_t lev_ev[33] = {};
     hipEvent_t join_ev = nullptr;
+    void *pin = nullptr;          // pinned staging of the PerBit retrieve's host decode
+    size_t pin_bytes = 0;
+    hipEvent_t pin_ev = nullptr;  // its last upload
     bool capturing = false;  // a graph capture is in progress (the PerBit retrieve has no graph form)
     // per-level load vectors of the retrieve pipeline (allocated on first use)
     void *flev = nullptr;
