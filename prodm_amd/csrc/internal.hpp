@@ -159,7 +159,7 @@ const double *mgard_adjoint_solution(const LevelGeom &g, int l, void *ws, uint32
 enum GroupKind : int { kGrpLoad = 0, kGrpContig = 1, kGrpStrided = 2, kGrpLevel0 = 3, kGrpNbEncode = 4, kGrpZero = 5 };
 // Shape knobs of one grouped launch; none changes any result.
 struct GroupShape {
-    int a = 0;         // load: coarse planes per tile march (0: per-entry default);
+    int a = 0;         // load: coarse planes per tile march (0: by the tiles of the launch);
                        // contig solve: lines (waves) per workgroup (0: 4)
     uint32_t cap = 0;  // workgroups of the launch (0: one per virtual workgroup)
 };
