@@ -74,6 +74,54 @@ template <class T> int launch_maxabs(const T *x, uint64_t n, KeyOf<T> *key, hipS
 template int launch_maxabs<float>(const float *, uint64_t, uint32_t *, hipStream_t);
 template int launch_maxabs<double>(const double *, uint64_t, unsigned long long *, hipStream_t);
 
+// The maximum for the host: every workgroup stores its own into out[its
+// index] (pinned host memory, no initial value, no atomics on one address:
+// 2350 workgroups' atomics had taken 24 us for 4.9 M floats, now 4 us).
+template <class T>
+__global__ __launch_bounds__(kThreads) void k_maxabs_blocks(const T *__restrict__ x, uint64_t n, KeyOf<T> *out) {
+    using K = KeyOf<T>;
+    constexpr int C = 16 / (int)sizeof(T);
+    __shared__ K red[kThreads / 64];
+    const uint64_t t0 = (uint64_t)blockIdx.x * kThreads + threadIdx.x, step = (uint64_t)gridDim.x * kThreads;
+    K m = 0;
+    auto take = [&](T v) __attribute__((always_inline)) {
+        const K k = v == v ? (K)abs_key(v) : (K)0;
+        m = k > m ? k : m;
+    };
+    uint64_t done = 0;
+    if (((uintptr_t)x & 15) == 0) {  // 16-byte loads of the aligned part
+        const uint64_t nv = n / C;
+#pragma unroll 4
+        for (uint64_t i = t0; i < nv; i += step) {
+            T v[C];
+            const float4 q = reinterpret_cast<const float4 *>(x)[i];
+            __builtin_memcpy(v, &q, 16);
+#pragma unroll
+            for (int c = 0; c < C; c++) take(v[c]);
+        }
+        done = nv * C;
+    }
+#pragma unroll 4
+    for (uint64_t i = done + t0; i < n; i += step) take(x[i]);
+    for (int off = 32; off >= 1; off >>= 1) {
+        const K o = __shfl_xor(m, off, 64);
+        m = o > m ? o : m;
+    }
+    if (lane_id() == 0) red[threadIdx.x / 64] = m;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < kThreads / 64; w++) m = red[w] > m ? red[w] : m;
+        out[blockIdx.x] = m;
+    }
+}
+template <class T> int launch_maxabs_blocks(const T *x, uint64_t n, KeyOf<T> *out, uint32_t blocks, hipStream_t s) {
+    hipLaunchKernelGGL(k_maxabs_blocks<T>, dim3(blocks), dim3(kThreads), 0, s, x, n, out);
+    PRODM_CHECK_LAUNCH();
+    return kOk;
+}
+template int launch_maxabs_blocks<float>(const float *, uint64_t, uint32_t *, uint32_t, hipStream_t);
+template int launch_maxabs_blocks<double>(const double *, uint64_t, unsigned long long *, uint32_t, hipStream_t);
+
 template <class T> __device__ inline int level_exp(int32_t exp, const KeyOf<T> *key) {
     return key ? dev_frexp_exp(key_to_value<T>((uint64_t)*key)) : exp;
 }

@@ -1,6 +1,7 @@
 // capi.hip -- extern "C" entry points of libprodm_mdr.so (include/prodm_mdr.h).
 #include <algorithm>
 #include <cstring>
+#include <mutex>
 #include <vector>
 
 #include "internal.hpp"
@@ -156,22 +157,56 @@ static int interleave_impl(const T *data, const uint32_t *dims, int nd, const ui
     return launch_interleave<T>(data, st, f3, c3, buf, repos, s);
 }
 
+// Pinned result slots (kSlotBytes each) of calls that return a value to the
+// host: taken and given back under a lock, at most kSlotsKept kept between
+// calls (for the life of the process), so that a call neither allocates nor
+// copies. Any thread and stream may hold one.
+constexpr size_t kSlotBytes = 4096;
+constexpr size_t kSlotsKept = 16;
+struct PinnedSlot {
+    static std::mutex mu;
+    static std::vector<void *> kept;
+    void *p = nullptr;
+    int take() {
+        {
+            std::lock_guard<std::mutex> lock(mu);
+            if (!kept.empty()) { p = kept.back(); kept.pop_back(); return kOk; }
+        }
+        PRODM_HIP(hipHostMalloc(&p, kSlotBytes, hipHostMallocPortable));
+        return kOk;
+    }
+    ~PinnedSlot() {
+        if (!p) return;
+        {
+            std::lock_guard<std::mutex> lock(mu);
+            if (kept.size() < kSlotsKept) { kept.push_back(p); return; }
+        }
+        (void)hipHostFree(p);
+    }
+};
+std::mutex PinnedSlot::mu;
+std::vector<void *> PinnedSlot::kept = [] { std::vector<void *> v; v.reserve(kSlotsKept); return v; }();
+
 template <class T>
 static int maxabs_impl(const T *x, uint64_t n, T *h_out, hipStream_t s) {
-    KeyOf<T> *key = nullptr;
-    PRODM_HIP(hipMallocAsync((void **)&key, sizeof(KeyOf<T>), s));
-    int rc = (sizeof(T) == 4) ? launch_fill_u32(reinterpret_cast<uint32_t *>(key), 1, 0u, s)
-                              : launch_fill_u64(reinterpret_cast<uint64_t *>(key), 1, 0ull, s);
-    if (!rc) rc = launch_maxabs<T>(x, n, key, s);
-    KeyOf<T> hk = 0;
-    if (!rc) {
-        hipError_t e = hipMemcpyAsync(&hk, key, sizeof(hk), hipMemcpyDeviceToHost, s);
-        if (e == hipSuccess) e = hipStreamSynchronize(s);
-        if (e != hipSuccess) { set_error(hipGetErrorString(e)); rc = kErrHip; }
+    KeyOf<T> best = 0;
+    if (n) {
+        PinnedSlot slot;
+        if (int rc = slot.take()) return rc;
+        // 16 elements per thread up to two workgroups per CU, which loop
+        const uint32_t blocks = (uint32_t)std::min<uint64_t>(kSlotBytes / 8, div_up(n, 256 * 16));
+        KeyOf<T> *keys = static_cast<KeyOf<T> *>(slot.p);
+        const int rc = launch_maxabs_blocks<T>(x, n, keys, blocks, s);
+        // no slot goes back before the stream is done with it
+        const hipError_t e = hipStreamSynchronize(s);
+        if (rc) return rc;
+        if (e != hipSuccess) { set_error(hipGetErrorString(e)); return kErrHip; }
+        for (uint32_t i = 0; i < blocks; i++) best = std::max(best, keys[i]);
+    } else {
+        PRODM_HIP(hipStreamSynchronize(s));
     }
-    (void)hipFreeAsync(key, s);
-    if (!rc) *h_out = key_to_value<T>((uint64_t)hk);
-    return rc;
+    *h_out = key_to_value<T>((uint64_t)best);
+    return kOk;
 }
 
 // ---- grouped decode state -------------------------------------------------------

@@ -44,6 +44,8 @@ int launch_fill_u64(uint64_t *dst, uint64_t count, uint64_t value, hipStream_t s
 // ---- max-abs (RefactorUtils.hpp:68-76) into an order key (atomicMax) --------
 template <class T> using KeyOf = typename std::conditional<sizeof(T) == 4, uint32_t, unsigned long long>::type;
 template <class T> int launch_maxabs(const T *x, uint64_t n, KeyOf<T> *key, hipStream_t s);
+// the same into one key per workgroup (every out[0 .. blocks) is written)
+template <class T> int launch_maxabs_blocks(const T *x, uint64_t n, KeyOf<T> *out, uint32_t blocks, hipStream_t s);
 
 // ---- NegaBinary (NegaBinaryBPEncoder.hpp:18-62, 132-192) ---------------------
 // planes: plane p at planes + p * stride (stride even for u32 words, and
