@@ -22,6 +22,7 @@
 #include "internal.hpp"
 
 #include <algorithm>
+#include <atomic>
 #include <cstring>
 #include <string>
 #include <type_traits>
@@ -521,7 +522,10 @@ __global__ __launch_bounds__(SH::kThreads) void k_load(LoadParams<T> P) {
 // inv[i] = 1 / (b_i - inv[i - 1]). The interior ones depend on the node index
 // alone and reach a bitwise fixed point after a few nodes, so one constant
 // sequence serves the lines of every level and dim (tables per level in the
-// workspace took an upload per call, which waits for the stream).
+// workspace took an upload per call, which waits for the stream). The kernels
+// take its address as a parameter: named in the kernel it costs registers that
+// the 40-node strided solve, at its limit, then spills (finest solves 173 -> 179
+// us at 513^3).
 constexpr uint32_t kThomasLen = 64;
 struct ThomasSeq {
     double v[kThomasLen] = {};
@@ -535,25 +539,45 @@ struct ThomasSeq {
 };
 constexpr ThomasSeq kThomasHost{};
 static_assert(kThomasHost.fix + 1 < kThomasLen, "the sequence reaches its fixed point");
-__device__ const ThomasSeq kThomas{};
+static __device__ ThomasSeq kThomas{};
+
+// device address of kThomas on the current device, looked up on first use
+static int thomas_table(const double **out) {
+    constexpr int kMaxDevices = 64;
+    static std::atomic<const double *> table[kMaxDevices];
+    int dev = -1;
+    PRODM_HIP(hipGetDevice(&dev));
+    if (dev < 0 || dev >= kMaxDevices) { set_error("line solves: no such device"); return kErrHip; }
+    const double *t = table[dev].load(std::memory_order_acquire);
+    if (!t) {
+        void *p = nullptr;
+        PRODM_HIP(hipGetSymbolAddress(&p, HIP_SYMBOL(kThomas)));
+        t = reinterpret_cast<const ThomasSeq *>(p)->v;
+        table[dev].store(t, std::memory_order_release);
+    }
+    *out = t;
+    return kOk;
+}
 
 enum Epilogue : int { kEpiNone = 0, kEpiAdd = 1, kEpiSub = 2 };
 
-// The kernels read kThomas below nfix (at most m - 1) and use lim for the
+// The kernels read inv (kThomas) below nfix (at most m - 1) and use lim for the
 // interior nodes from there on and last for node m - 1. cp[i] = inv[i] (the
 // off-diagonal is 1).
 template <class T> struct SolveParams {
     double *f;            // c0 x c1 rows of pitch fp
     uint32_t fp;
     uint32_t c[3];
+    const double *inv;    // inv[0..nfix)
     double lim, last;     // inv[i] for nfix <= i < m - 1, inv[m - 1]
     uint32_t nfix;
     int epi;
     const T *uc_in;       // epilogue input (dense c)
     T *uc_out;            // epilogue output (dense c)
 };
-template <class T> __device__ __forceinline__ double thomas_factor(const SolveParams<T> &S, uint32_t m, uint32_t i) {
-    return i < S.nfix ? kThomas.v[i] : (i == m - 1 ? S.last : S.lim);
+template <class T, class P>
+__device__ __forceinline__ double thomas_factor(const SolveParams<T> &S, P inv, uint32_t m, uint32_t i) {
+    return i < S.nfix ? inv[i] : (i == m - 1 ? S.last : S.lim);
 }
 
 // fidx: position in f (padded rows), uidx: position in the dense u_c
@@ -614,7 +638,7 @@ __device__ __forceinline__ void solve_contig_lines(const SolveParams<T> &S, uint
     // kOffNone offsets (narrower groups share one descriptor per wave).
     bool in[SEG];
     double iv[SEG];
-    const auto rinv = buf_rsrc((const void *)kThomas.v, true);
+    const auto rinv = buf_rsrc((const void *)S.inv, true);
 #pragma unroll
     for (int i = 0; i < SEG; i++) {
         const uint32_t k = b + i;
@@ -842,7 +866,7 @@ __device__ __forceinline__ void solve_strided_lines(const SolveParams<T> &S, uin
     for (int r = 0; r < NF; r++) {
         const uint32_t nl = b + 64u * r + lane;
         const bool has = 64u * r + lane < (uint32_t)SEG && nl < e;
-        fl[r] = has ? thomas_factor(S, m, nl) : 0.0;
+        fl[r] = has ? thomas_factor(S, (const PRODM_GLOBAL double *)S.inv, m, nl) : 0.0;
         cl[r] = nl == m - 1 ? 0.0 : fl[r];
     }
     auto fac = [&](int i) __attribute__((always_inline)) -> double { return readlane_f64(fl[i / 64], i % 64); };
@@ -971,7 +995,7 @@ __global__ __launch_bounds__(kWideThreads) void k_solve_wide(SolveParams<T> S, u
         }
     }
     PRODM_GLOBAL double *const f = (PRODM_GLOBAL double *)S.f;
-    if (threadIdx.x < kWideFix) tab[threadIdx.x] = threadIdx.x < S.nfix ? kThomas.v[threadIdx.x] : S.lim;
+    if (threadIdx.x < kWideFix) tab[threadIdx.x] = threadIdx.x < S.nfix ? ((const PRODM_GLOBAL double *)S.inv)[threadIdx.x] : S.lim;
     const uint32_t seg = (m + NS - 1) / NS;
     const uint32_t b = min(m, sg * seg), len = act ? min(m, b + seg) - b : 0u;
     double *const v = node + threadIdx.x;
@@ -1116,6 +1140,7 @@ __global__ __launch_bounds__(256) void k_solve_seq(SolveParams<T> S, uint32_t m,
         }
     }
     PRODM_GLOBAL double *f = (PRODM_GLOBAL double *)S.f;
+    const PRODM_CONST double *inv = (const PRODM_CONST double *)S.inv;
     constexpr uint32_t U = 8;  // loads issued ahead of the dependent chain
     double y = 0.0;
     uint32_t i = 0;
@@ -1125,12 +1150,12 @@ __global__ __launch_bounds__(256) void k_solve_seq(SolveParams<T> S, uint32_t m,
         for (uint32_t k = 0; k < U; k++) t[k] = f[base + (i + k) * stride];
 #pragma unroll
         for (uint32_t k = 0; k < U; k++) {
-            y = (t[k] - y) * thomas_factor(S, m, i + k);
+            y = (t[k] - y) * thomas_factor(S, inv, m, i + k);
             f[base + (i + k) * stride] = y;
         }
     }
     for (; i < m; i++) {
-        y = (f[base + i * stride] - y) * thomas_factor(S, m, i);
+        y = (f[base + i * stride] - y) * thomas_factor(S, inv, m, i);
         f[base + i * stride] = y;
     }
     double z = 0.0;
@@ -1142,14 +1167,14 @@ __global__ __launch_bounds__(256) void k_solve_seq(SolveParams<T> S, uint32_t m,
 #pragma unroll
         for (uint32_t k = 0; k < U; k++) {
             const uint32_t n = e - 1 - k;
-            const double c = (n == m - 1) ? 0.0 : thomas_factor(S, m, n);
+            const double c = (n == m - 1) ? 0.0 : thomas_factor(S, inv, m, n);
             z = t[k] - c * z;
             epilogue(S, base + n * stride, ubase + n * ustride, z);
         }
     }
     for (; e > 0; e--) {
         const uint32_t n = e - 1;
-        const double c = (n == m - 1) ? 0.0 : thomas_factor(S, m, n);
+        const double c = (n == m - 1) ? 0.0 : thomas_factor(S, inv, m, n);
         z = f[base + n * stride] - c * z;
         epilogue(S, base + n * stride, ubase + n * ustride, z);
     }
@@ -1422,7 +1447,8 @@ WsLayout ws_layout(const LevelGeom &g, size_t elem) {
 }
 
 // the factors of a line of m nodes
-template <class T> void set_factors(SolveParams<T> &S, uint32_t m) {
+template <class T> void set_factors(SolveParams<T> &S, const double *inv, uint32_t m) {
+    S.inv = inv;
     const ThomasSeq &q = kThomasHost;
     const uint32_t e = m >= 2 ? std::min(m - 2, kThomasLen - 1) : 0;  // node m - 2's entry
     S.last = m >= 2 ? 1.0 / (2.0 - q.v[e]) : 1.0 / 2.0;
@@ -1462,6 +1488,8 @@ template <class T>
 int solve_all(const LevelGeom &g, int l, double *f, int epi, const T *uc_in, T *uc_out, hipStream_t s) {
     const uint32_t *c = g.ld[l - 1];
     const uint32_t *n = g.ld[l];
+    const double *inv = nullptr;
+    if (int rc = thomas_table(&inv)) return rc;
     // solves run dims 2, 1, 0: the last one executed is the smallest active d
     int last = -1;
     for (int d = 0; d < 3; d++)
@@ -1472,7 +1500,7 @@ int solve_all(const LevelGeom &g, int l, double *f, int epi, const T *uc_in, T *
         S.f = f;
         S.fp = f_pitch(c[2]);
         S.c[0] = c[0]; S.c[1] = c[1]; S.c[2] = c[2];
-        set_factors(S, c[d]);
+        set_factors(S, inv, c[d]);
         S.epi = (d == last) ? epi : kEpiNone;
         S.uc_in = uc_in;
         S.uc_out = uc_out;
@@ -1852,6 +1880,8 @@ int mgard_batched_launches(const std::vector<BatchFieldRef> &fields, const std::
         int which;
     };
     std::vector<State> st(fields.size());
+    const double *inv = nullptr;
+    if (int rc = thomas_table(&inv)) return rc;
     int Lmax = 0;
     for (size_t i = 0; i < fields.size(); i++) {
         const BatchFieldRef &f = fields[i];
@@ -1916,7 +1946,7 @@ int mgard_batched_launches(const std::vector<BatchFieldRef> &fields, const std::
                     E.S.f = fv;
                     E.S.fp = f_pitch(c[2]);
                     E.S.c[0] = c[0]; E.S.c[1] = c[1]; E.S.c[2] = c[2];
-                    set_factors(E.S, c[d]);
+                    set_factors(E.S, inv, c[d]);
                     E.S.epi = (d == last) ? kEpiAdd : kEpiNone;
                     E.S.uc_in = uc;
                     E.S.uc_out = uc;
