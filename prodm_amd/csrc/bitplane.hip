@@ -539,15 +539,16 @@ template int launch_nb_encode<float>(const float *, uint32_t, int32_t, const uin
 template int launch_nb_encode<double>(const double *, uint32_t, int32_t, const unsigned long long *, int, uint64_t *,
                                       uint64_t, hipStream_t);
 
-template <class T>
-__global__ __launch_bounds__(BlkStage<T>::kTPB) void k_nb_decode(PlanePtrs pl, uint32_t n, int32_t exp,
-                                                              const KeyOf<T> *key, int start, int k,
-                                                              T *__restrict__ out) {
+// workgroup bid decodes its blocks from planes [start, start + k), plane(i)
+// giving the words of plane start + i
+template <class T, class PlaneFn>
+__device__ __forceinline__ void nb_decode_blocks(PlaneFn &&plane, uint32_t n, int32_t exp, const KeyOf<T> *key,
+                                                 int start, int k, T *__restrict__ out, uint32_t bid) {
     using S = typename Traits<T>::Stream;
     using SF = typename Traits<T>::SFixed;
     constexpr int TPB = BlkStage<T>::kTPB, B = BlkStage<T>::kB, PI = BlkStage<T>::kPitch;
     __shared__ T sx[TPB * PI];
-    const uint64_t b0 = (uint64_t)blockIdx.x * TPB;
+    const uint64_t b0 = (uint64_t)bid * TPB;
     const uint64_t b = b0 + threadIdx.x;
     const uint64_t nw = ((uint64_t)n + B - 1) / B;
     const int e2 = level_exp<T>(exp, key) + 2;
@@ -559,7 +560,7 @@ __global__ __launch_bounds__(BlkStage<T>::kTPB) void k_nb_decode(PlanePtrs pl, u
 #pragma unroll
         for (int r = 0; r < 32; r++) {
             const int i = k - 1 - r;
-            a[r] = (i >= 0 && b < nw) ? static_cast<const S *>(pl.p[i])[b] : 0u;
+            a[r] = (i >= 0 && b < nw) ? plane(i)[b] : 0u;
         }
         transpose32(a);
 #pragma unroll
@@ -573,7 +574,7 @@ __global__ __launch_bounds__(BlkStage<T>::kTPB) void k_nb_decode(PlanePtrs pl, u
         static_for<0, 64>([&](auto rc) {
             constexpr int r = decltype(rc)::value;
             const int i = k - 1 - r;
-            const uint64_t w = (i >= 0 && b < nw) ? static_cast<const S *>(pl.p[i])[b] : 0ull;
+            const uint64_t w = (i >= 0 && b < nw) ? plane(i)[b] : 0ull;
             word64_set<r>(lo, hi, w);
         });
         transpose64(lo, hi);
@@ -587,6 +588,15 @@ __global__ __launch_bounds__(BlkStage<T>::kTPB) void k_nb_decode(PlanePtrs pl, u
     }
     __syncthreads();
     stage_out<T>(out, n, b0 * B, sx);
+}
+
+template <class T>
+__global__ __launch_bounds__(BlkStage<T>::kTPB) void k_nb_decode(PlanePtrs pl, uint32_t n, int32_t exp,
+                                                              const KeyOf<T> *key, int start, int k,
+                                                              T *__restrict__ out) {
+    using S = typename Traits<T>::Stream;
+    nb_decode_blocks<T>([&](int i) __attribute__((always_inline)) { return static_cast<const S *>(pl.p[i]); }, n, exp,
+                        key, start, k, out, blockIdx.x);
 }
 
 template <class T>
@@ -610,6 +620,55 @@ template int launch_nb_decode<float>(const PlanePtrs &, uint32_t, int32_t, const
                                      hipStream_t);
 template int launch_nb_decode<double>(const PlanePtrs &, uint32_t, int32_t, const unsigned long long *, int, int,
                                       double *, hipStream_t);
+
+// ---- small levels of a plan together ---------------------------------------------
+// A plan's small levels take one launch per kernel (LevelSet by value) instead
+// of one each: a launch costs some 3 us of host time and 3 to 6 us on the GPU
+// whatever its size, and a 33^3 refactor + retrieve was 40 of them.
+template <class T>
+__global__ __launch_bounds__(BlkStage<T>::kTPB) void k_nb_encode_set(LevelSet<NbLevel<T>> L, int nb) {
+    const uint32_t i = set_entry(L, blockIdx.x);
+    const NbLevel<T> &E = L.e[i];
+    nb_encode_blocks<T>(E.x, E.n, 0, E.key, nb, E.planes, E.stride, blockIdx.x - L.first[i]);
+}
+template <class T>
+__global__ __launch_bounds__(BlkStage<T>::kTPB) void k_nb_decode_set(LevelSet<NbLevel<T>> L) {
+    const uint32_t i = set_entry(L, blockIdx.x);
+    const NbLevel<T> &E = L.e[i];
+    const typename Traits<T>::Stream *planes = E.planes;
+    const uint64_t stride = E.stride;
+    nb_decode_blocks<T>([&](int p) __attribute__((always_inline)) { return planes + (uint64_t)p * stride; }, E.n, 0,
+                        E.key, 0, E.k, E.x, blockIdx.x - L.first[i]);
+}
+template <class T> static uint32_t nb_workgroups(uint32_t n) {
+    return div_up(((uint64_t)n + Traits<T>::kBlock - 1) / Traits<T>::kBlock, BlkStage<T>::kTPB);
+}
+template <class T> int launch_nb_encode_set(LevelSet<NbLevel<T>> L, int nb, hipStream_t s) {
+    if (!L.n) return kOk;
+    for (uint32_t i = 0; i < L.n; i++)
+        if (L.e[i].n == 0 || nb < 1 || nb > Traits<T>::kBlock) {
+            set_error("negabinary encode: bad n or num_bitplanes");
+            return kErrArg;
+        }
+    set_sizes(L, [](const NbLevel<T> &e) { return nb_workgroups<T>(e.n); });
+    hipLaunchKernelGGL(k_nb_encode_set<T>, dim3(L.first[L.n]), dim3(BlkStage<T>::kTPB), 0, s, L, nb);
+    PRODM_CHECK_LAUNCH();
+    return kOk;
+}
+template <class T> int launch_nb_decode_set(LevelSet<NbLevel<T>> L, hipStream_t s) {
+    if (!L.n) return kOk;
+    for (uint32_t i = 0; i < L.n; i++)
+        if (L.e[i].k < 0 || L.e[i].k > Traits<T>::kBlock) { set_error("negabinary decode: bad plane range"); return kErrArg; }
+    set_sizes(L, [](const NbLevel<T> &e) { return nb_workgroups<T>(e.n); });
+    if (!L.first[L.n]) return kOk;
+    hipLaunchKernelGGL(k_nb_decode_set<T>, dim3(L.first[L.n]), dim3(BlkStage<T>::kTPB), 0, s, L);
+    PRODM_CHECK_LAUNCH();
+    return kOk;
+}
+template int launch_nb_encode_set<float>(LevelSet<NbLevel<float>>, int, hipStream_t);
+template int launch_nb_encode_set<double>(LevelSet<NbLevel<double>>, int, hipStream_t);
+template int launch_nb_decode_set<float>(LevelSet<NbLevel<float>>, hipStream_t);
+template int launch_nb_decode_set<double>(LevelSet<NbLevel<double>>, hipStream_t);
 
 // ------------------------------------------------------------------------------
 // GroupedBP
@@ -672,9 +731,9 @@ __device__ __forceinline__ void gb_row(const uint32_t *h, int pstart, int k, uin
 // it through 16-byte loads and the pass reads at the memory's rate. Blocks
 // with a larger value (an exponent below the level's, infinities) take the OR.
 template <class T>
-__global__ __launch_bounds__(kGbTPB) void k_gb_rb(const T *__restrict__ x, uint32_t n, int32_t exp,
-                                                  const KeyOf<T> *key, int nb, int compat, uint8_t *__restrict__ rb,
-                                                  uint32_t *__restrict__ rowsum) {
+__device__ __forceinline__ void gb_rb_blocks(const T *__restrict__ x, uint32_t n, int32_t exp, const KeyOf<T> *key,
+                                             int nb, int compat, uint8_t *__restrict__ rb,
+                                             uint32_t *__restrict__ rowsum, uint32_t bid) {
     using F = typename Traits<T>::Fixed;
     using K = KeyOf<T>;
     constexpr int B = Traits<T>::kBlock, C = 16 / (int)sizeof(T);
@@ -685,7 +744,7 @@ __global__ __launch_bounds__(kGbTPB) void k_gb_rb(const T *__restrict__ x, uint3
     if (threadIdx.x < 128) h[threadIdx.x] = 0;
     __syncthreads();
     const uint32_t lane = lane_id(), wv = threadIdx.x / 64;
-    const uint64_t b0 = (uint64_t)blockIdx.x * gb_wg_blocks<T>() + (uint64_t)wv * WaveRows<T>::kBlocks;
+    const uint64_t b0 = (uint64_t)bid * gb_wg_blocks<T>() + (uint64_t)wv * WaveRows<T>::kBlocks;
     const uint64_t e0 = b0 * B;
     const uint64_t nblk = ((uint64_t)n - 1) / B + 1;
     const int shift = nb - level_exp<T>(exp, key);
@@ -748,7 +807,14 @@ __global__ __launch_bounds__(kGbTPB) void k_gb_rb(const T *__restrict__ x, uint3
         atomicAdd(&h[r], 1u);
     }
     __syncthreads();
-    if (wv == 0) gb_row(h, 0, nb, rowsum + (uint64_t)blockIdx.x * nb);
+    if (wv == 0) gb_row(h, 0, nb, rowsum + (uint64_t)bid * nb);
+}
+
+template <class T>
+__global__ __launch_bounds__(kGbTPB) void k_gb_rb(const T *__restrict__ x, uint32_t n, int32_t exp,
+                                                  const KeyOf<T> *key, int nb, int compat, uint8_t *__restrict__ rb,
+                                                  uint32_t *__restrict__ rowsum) {
+    gb_rb_blocks<T>(x, n, exp, key, nb, compat, rb, rowsum, blockIdx.x);
 }
 
 // Offsets: rows of k words are scanned down the workgroups, a lane per plane
@@ -835,15 +901,16 @@ struct GbWaveLds {
 };
 template <class T>
 __device__ __forceinline__ uint32_t gb_wave_base(int r, const uint32_t *__restrict__ rows, int pstart, int k,
-                                                 uint32_t *__restrict__ totals, GbWaveLds &lds) {
+                                                 uint32_t *__restrict__ totals, GbWaveLds &lds, uint32_t bid,
+                                                 uint32_t nwg) {
     const uint32_t lane = lane_id(), wv = threadIdx.x / 64;
-    const bool on = (int)lane < k, direct = gridDim.x <= (uint32_t)kGbScanRows;
+    const bool on = (int)lane < k, direct = nwg <= (uint32_t)kGbScanRows;
     lds.hw[wv][lane] = 0;
     if (r < 64 && lane < (uint32_t)WaveRows<T>::kBlocks) atomicAdd(&lds.hw[wv][r], 1u);
     uint32_t b = 0;
     if (direct && on) {
 #pragma unroll 8
-        for (uint32_t c = wv; c < blockIdx.x; c += kGbWaves) b += rows[(uint64_t)c * k + lane];
+        for (uint32_t c = wv; c < bid; c += kGbWaves) b += rows[(uint64_t)c * k + lane];
     }
     lds.below[wv][lane] = b;
     __syncthreads();
@@ -852,10 +919,10 @@ __device__ __forceinline__ uint32_t gb_wave_base(int r, const uint32_t *__restri
     const uint32_t words = __ockl_wfscan_add_u32(hb, true) + hb;  // lane p: plane p
     // window lane i <- plane pstart + i
     const uint32_t shifted = __shfl(words, (int)((lane + (uint32_t)pstart) & 63u), 64);
-    uint32_t own = on && (!direct || totals) ? rows[(uint64_t)blockIdx.x * k + lane] : 0u;
+    uint32_t own = on && (!direct || totals) ? rows[(uint64_t)bid * k + lane] : 0u;
     if (direct) {
         const uint32_t o = (lds.below[0][lane] + lds.below[1][lane]) + (lds.below[2][lane] + lds.below[3][lane]);
-        if (totals && on && wv == 0 && blockIdx.x == gridDim.x - 1) totals[lane] = o + own;
+        if (totals && on && wv == 0 && bid == nwg - 1) totals[lane] = o + own;
         own = o;
     }
     return on ? own + shifted : 0u;
@@ -875,22 +942,22 @@ __device__ __forceinline__ uint32_t gb_pos(uint32_t base, int i, uint64_t le, ui
 // Pass 2: plane words, compacted per plane. The positions need no barrier
 // inside the plane loop (gb_wave_base).
 template <class T>
-__global__ __launch_bounds__(kGbTPB) void k_gb_write(const T *__restrict__ x, uint32_t n, int32_t exp,
-                                                     const KeyOf<T> *key, int nb, int compat,
-                                                     const uint8_t *__restrict__ rb, const uint32_t *__restrict__ off,
-                                                     typename Traits<T>::Stream *__restrict__ planes, uint64_t stride,
-                                                     uint32_t *__restrict__ totals) {
+__device__ __forceinline__ void gb_write_blocks(const T *__restrict__ x, uint32_t n, int32_t exp, const KeyOf<T> *key,
+                                                int nb, int compat, const uint8_t *__restrict__ rb,
+                                                const uint32_t *__restrict__ off,
+                                                typename Traits<T>::Stream *__restrict__ planes, uint64_t stride,
+                                                uint32_t *__restrict__ totals, uint32_t bid, uint32_t nwg) {
     using R = WaveRows<T>;
     constexpr int B = Traits<T>::kBlock, W = 8 * (int)sizeof(T);
     __shared__ __align__(16) uint32_t rows[kGbWaves][64 * kRowPitch];
     __shared__ GbWaveLds wl;
     const uint32_t lane = lane_id(), wv = threadIdx.x / 64;
-    const uint64_t b0 = (uint64_t)blockIdx.x * gb_wg_blocks<T>() + (uint64_t)wv * R::kBlocks;
+    const uint64_t b0 = (uint64_t)bid * gb_wg_blocks<T>() + (uint64_t)wv * R::kBlocks;
     const uint32_t bl = lane % R::kBlocks, half = lane / R::kBlocks;
     const uint64_t b = b0 + bl, nblk = ((uint64_t)n - 1) / B + 1;
     const int r = b < nblk ? rb[b] : 255;
     // before the elements: its loop over rows would hold registers beside them
-    const uint32_t base = gb_wave_base<T>(r, off, 0, nb, totals, wl);
+    const uint32_t base = gb_wave_base<T>(r, off, 0, nb, totals, wl, bid, nwg);
     const int shift = nb - level_exp<T>(exp, key);
     uint32_t w[W], sg = 0;
     rows_in<T>(x, n, b0 * B, rows[wv], [&](int j, T v) __attribute__((always_inline)) {
@@ -912,6 +979,15 @@ __global__ __launch_bounds__(kGbTPB) void k_gb_write(const T *__restrict__ x, ui
             if (r <= p) dst[(uint64_t)pos * R::kHalves] = w[k];
         }
     });
+}
+
+template <class T>
+__global__ __launch_bounds__(kGbTPB) void k_gb_write(const T *__restrict__ x, uint32_t n, int32_t exp,
+                                                     const KeyOf<T> *key, int nb, int compat,
+                                                     const uint8_t *__restrict__ rb, const uint32_t *__restrict__ off,
+                                                     typename Traits<T>::Stream *__restrict__ planes, uint64_t stride,
+                                                     uint32_t *__restrict__ totals) {
+    gb_write_blocks<T>(x, n, exp, key, nb, compat, rb, off, planes, stride, totals, blockIdx.x, gridDim.x);
 }
 
 // workgroups of the formula the workspace sizes were first given out with;
@@ -967,18 +1043,24 @@ template int launch_gb_encode<double>(const double *, uint32_t, int32_t, const u
 // ---- GroupedBP progressive decode ----------------------------------------------
 // words rows of planes [start, start + k) from the recording planes
 template <class T>
-__global__ __launch_bounds__(kGbTPB) void k_gb_rbrows(const uint8_t *__restrict__ rb, uint32_t nblk, int start, int k,
-                                                      uint32_t *__restrict__ rows) {
+__device__ __forceinline__ void gb_rbrows_blocks(const uint8_t *__restrict__ rb, uint32_t nblk, int start, int k,
+                                                 uint32_t *__restrict__ rows, uint32_t bid) {
     __shared__ uint32_t h[64];
     if (threadIdx.x < 64) h[threadIdx.x] = 0;
     __syncthreads();
-    const uint64_t b = (uint64_t)blockIdx.x * gb_wg_blocks<T>() + threadIdx.x;
+    const uint64_t b = (uint64_t)bid * gb_wg_blocks<T>() + threadIdx.x;
     if (threadIdx.x < gb_wg_blocks<T>() && b < nblk) {
         const int r = rb[b];
         if (r < 64) atomicAdd(&h[r], 1u);
     }
     __syncthreads();
-    if (threadIdx.x < 64) gb_row(h, start, k, rows + (uint64_t)blockIdx.x * k);
+    if (threadIdx.x < 64) gb_row(h, start, k, rows + (uint64_t)bid * k);
+}
+
+template <class T>
+__global__ __launch_bounds__(kGbTPB) void k_gb_rbrows(const uint8_t *__restrict__ rb, uint32_t nblk, int start, int k,
+                                                      uint32_t *__restrict__ rows) {
+    gb_rbrows_blocks<T>(rb, nblk, start, k, rows, blockIdx.x);
 }
 
 // 32-bit word at any byte offset (stream 0's words follow its header)
@@ -990,18 +1072,18 @@ __device__ __forceinline__ uint32_t load_bytes32(const uint8_t *p) {
 // planes are loaded without branches: a lane without a word in a plane (rb
 // above it) takes the offset past the buffer's range and reads 0. A plane
 // holds at most 2 words per block, 2^30 bytes at 2^32 elements.
-template <class T>
-__global__ __launch_bounds__(kGbTPB) void k_gb_decode(PlanePtrs pl, uint32_t n, int32_t exp, const KeyOf<T> *key,
-                                                      int start, int k, const uint8_t *__restrict__ rb,
-                                                      typename Traits<T>::Stream *__restrict__ signs,
-                                                      const uint32_t *__restrict__ off, T *__restrict__ out,
-                                                      uint64_t hdr0) {
+template <class T, class PlaneFn>
+__device__ __forceinline__ void gb_decode_blocks(PlaneFn &&plane, uint32_t n, int32_t exp, const KeyOf<T> *key,
+                                                 int start, int k, const uint8_t *__restrict__ rb,
+                                                 typename Traits<T>::Stream *__restrict__ signs,
+                                                 const uint32_t *__restrict__ off, T *__restrict__ out, uint64_t hdr0,
+                                                 uint32_t bid, uint32_t nwg) {
     using R = WaveRows<T>;
     constexpr int B = Traits<T>::kBlock, W = 8 * (int)sizeof(T);
     __shared__ __align__(16) uint32_t rows[kGbWaves][64 * kRowPitch];
     __shared__ GbWaveLds wl;
     const uint32_t lane = lane_id(), wv = threadIdx.x / 64;
-    const uint64_t b0 = (uint64_t)blockIdx.x * gb_wg_blocks<T>() + (uint64_t)wv * R::kBlocks;
+    const uint64_t b0 = (uint64_t)bid * gb_wg_blocks<T>() + (uint64_t)wv * R::kBlocks;
     const uint32_t bl = lane % R::kBlocks, half = lane / R::kBlocks;
     const uint64_t b = b0 + bl, nblk = ((uint64_t)n - 1) / B + 1;
     const bool valid = b < nblk;
@@ -1010,7 +1092,7 @@ __global__ __launch_bounds__(kGbTPB) void k_gb_decode(PlanePtrs pl, uint32_t n, 
     const int r = valid ? rb[b] : 255;
     uint32_t *const sgw = reinterpret_cast<uint32_t *>(signs) + b * R::kHalves + half;
     uint32_t sg = valid ? *sgw : 0u;
-    const uint32_t base = gb_wave_base<T>(r, off, start, k, nullptr, wl);
+    const uint32_t base = gb_wave_base<T>(r, off, start, k, nullptr, wl, bid, nwg);
     // acc bit (end - 1 - p) comes from plane p; planes below rb are zero
     const uint8_t *sgat = nullptr;
     uint32_t w[W];
@@ -1021,7 +1103,7 @@ __global__ __launch_bounds__(kGbTPB) void k_gb_decode(PlanePtrs pl, uint32_t n, 
         if (i >= 0) {
             const uint64_t le = ballot64(r <= p), eq = ballot64(r == p);
             const uint32_t pos = gb_pos<T>(base, i, le, eq), at = (pos * R::kHalves + half) * 4;
-            const uint8_t *sb = static_cast<const uint8_t *>(pl.p[i]) + (i == 0 ? hdr0 : 0);
+            const uint8_t *sb = plane(i) + (i == 0 ? hdr0 : 0);
             if (eq && r == p) sgat = sb + at;
             const uint32_t word = at + (r == p ? 4 * R::kHalves : 0);
             if (i == 0 && (hdr0 & 3)) {
@@ -1046,6 +1128,16 @@ __global__ __launch_bounds__(kGbTPB) void k_gb_decode(PlanePtrs pl, uint32_t n, 
         v[j] = (r >= end) ? (T)0 : y;
     }
     rows_out<T>(out, n, b0 * B, rows[wv], v);
+}
+
+template <class T>
+__global__ __launch_bounds__(kGbTPB) void k_gb_decode(PlanePtrs pl, uint32_t n, int32_t exp, const KeyOf<T> *key,
+                                                      int start, int k, const uint8_t *__restrict__ rb,
+                                                      typename Traits<T>::Stream *__restrict__ signs,
+                                                      const uint32_t *__restrict__ off, T *__restrict__ out,
+                                                      uint64_t hdr0) {
+    gb_decode_blocks<T>([&](int i) __attribute__((always_inline)) { return static_cast<const uint8_t *>(pl.p[i]); }, n,
+                        exp, key, start, k, rb, signs, off, out, hdr0, blockIdx.x, gridDim.x);
 }
 
 template <class T>
@@ -1087,6 +1179,72 @@ template <class T> size_t gb_decode_workspace_bytes(uint32_t n, int start, int k
 }
 template size_t gb_decode_workspace_bytes<float>(uint32_t, int, int);
 template size_t gb_decode_workspace_bytes<double>(uint32_t, int, int);
+
+// ---- small levels of a plan together (at most kGbScanRows workgroups each) -------
+template <class T> __global__ __launch_bounds__(kGbTPB) void k_gb_rb_set(LevelSet<GbLevel<T>> L, int nb) {
+    const uint32_t i = set_entry(L, blockIdx.x);
+    const GbLevel<T> &E = L.e[i];
+    gb_rb_blocks<T>(E.x, E.n, 0, E.key, nb, 0, E.rb, E.rows, blockIdx.x - L.first[i]);
+}
+template <class T> __global__ __launch_bounds__(kGbTPB) void k_gb_write_set(LevelSet<GbLevel<T>> L, int nb) {
+    const uint32_t i = set_entry(L, blockIdx.x);
+    const GbLevel<T> &E = L.e[i];
+    gb_write_blocks<T>(E.x, E.n, 0, E.key, nb, 0, E.rb, E.rows, E.planes, E.stride, E.words, blockIdx.x - L.first[i],
+                       L.first[i + 1] - L.first[i]);
+}
+template <class T> __global__ __launch_bounds__(kGbTPB) void k_gb_rbrows_set(LevelSet<GbLevel<T>> L) {
+    const uint32_t i = set_entry(L, blockIdx.x);
+    const GbLevel<T> &E = L.e[i];
+    gb_rbrows_blocks<T>(E.rb, (E.n - 1) / Traits<T>::kBlock + 1, 0, E.k, E.rows, blockIdx.x - L.first[i]);
+}
+template <class T> __global__ __launch_bounds__(kGbTPB) void k_gb_decode_set(LevelSet<GbLevel<T>> L) {
+    const uint32_t i = set_entry(L, blockIdx.x);
+    const GbLevel<T> &E = L.e[i];
+    const typename Traits<T>::Stream *planes = E.planes;
+    const uint64_t stride = E.stride;
+    gb_decode_blocks<T>(
+        [&](int p) __attribute__((always_inline)) { return reinterpret_cast<const uint8_t *>(planes + (uint64_t)p * stride); },
+        E.n, 0, E.key, 0, E.k, E.rb, E.signs, E.rows, E.x, 0, blockIdx.x - L.first[i], L.first[i + 1] - L.first[i]);
+}
+template <class T> size_t gb_set_row_words(uint32_t n, int nb) {
+    const uint32_t nwg = gb_nwg<T>(n);
+    return nwg <= (uint32_t)kGbScanRows ? (size_t)nwg * nb : 0;
+}
+template size_t gb_set_row_words<float>(uint32_t, int);
+template size_t gb_set_row_words<double>(uint32_t, int);
+template <class T> int launch_gb_encode_set(LevelSet<GbLevel<T>> L, int nb, hipStream_t s) {
+    if (!L.n) return kOk;
+    for (uint32_t i = 0; i < L.n; i++)
+        if (L.e[i].n == 0 || nb < 1 || nb > Traits<T>::kBlock || !gb_set_row_words<T>(L.e[i].n, nb)) {
+            set_error("grouped encode: bad n or num_bitplanes");
+            return kErrArg;
+        }
+    set_sizes(L, [](const GbLevel<T> &e) { return gb_nwg<T>(e.n); });
+    hipLaunchKernelGGL(k_gb_rb_set<T>, dim3(L.first[L.n]), dim3(kGbTPB), 0, s, L, nb);
+    PRODM_CHECK_LAUNCH();
+    hipLaunchKernelGGL(k_gb_write_set<T>, dim3(L.first[L.n]), dim3(kGbTPB), 0, s, L, nb);
+    PRODM_CHECK_LAUNCH();
+    return kOk;
+}
+template <class T> int launch_gb_decode_set(LevelSet<GbLevel<T>> L, hipStream_t s) {
+    if (!L.n) return kOk;
+    for (uint32_t i = 0; i < L.n; i++)
+        if (L.e[i].k < 0 || L.e[i].k > Traits<T>::kBlock || (L.e[i].n && !gb_set_row_words<T>(L.e[i].n, 1))) {
+            set_error("grouped decode: bad plane range or level size");
+            return kErrArg;
+        }
+    set_sizes(L, [](const GbLevel<T> &e) { return e.n ? gb_nwg<T>(e.n) : 0; });
+    if (!L.first[L.n]) return kOk;
+    hipLaunchKernelGGL(k_gb_rbrows_set<T>, dim3(L.first[L.n]), dim3(kGbTPB), 0, s, L);
+    PRODM_CHECK_LAUNCH();
+    hipLaunchKernelGGL(k_gb_decode_set<T>, dim3(L.first[L.n]), dim3(kGbTPB), 0, s, L);
+    PRODM_CHECK_LAUNCH();
+    return kOk;
+}
+template int launch_gb_encode_set<float>(LevelSet<GbLevel<float>>, int, hipStream_t);
+template int launch_gb_encode_set<double>(LevelSet<GbLevel<double>>, int, hipStream_t);
+template int launch_gb_decode_set<float>(LevelSet<GbLevel<float>>, hipStream_t);
+template int launch_gb_decode_set<double>(LevelSet<GbLevel<double>>, hipStream_t);
 
 // ------------------------------------------------------------------------------
 // PerBit

@@ -74,6 +74,51 @@ int launch_gb_decode(const PlanePtrs &streams, uint32_t n, int32_t exp, const Ke
                      uint64_t hdr0_bytes, hipStream_t s);
 template <class T> size_t gb_decode_workspace_bytes(uint32_t n, int start, int k);
 
+// ---- small levels of a plan in one launch --------------------------------------
+// Entry i of a set, passed to a kernel by value, owns workgroups
+// [first[i], first[i + 1]).
+constexpr int kSetMax = 16;
+template <class E> struct LevelSet {
+    uint32_t n = 0;
+    uint32_t first[kSetMax + 1] = {0};
+    E e[kSetMax];
+};
+template <class E, class Fn> void set_sizes(LevelSet<E> &L, Fn &&workgroups) {
+    for (uint32_t i = 0; i < L.n; i++) L.first[i + 1] = L.first[i] + workgroups(L.e[i]);
+}
+template <class E> __device__ __forceinline__ uint32_t set_entry(const LevelSet<E> &L, uint32_t bid) {
+    uint32_t i = 0;
+    while (i + 1 < L.n && L.first[i + 1] <= bid) i++;
+    return i;
+}
+// a plan level's coefficients x (encoded from or decoded to), planes and max
+// key; decode reads planes [0, k)
+template <class T> struct NbLevel {
+    T *x;
+    const KeyOf<T> *key;
+    typename Traits<T>::Stream *planes;
+    uint64_t stride;
+    uint32_t n;
+    int32_t k;
+};
+template <class T> int launch_nb_encode_set(LevelSet<NbLevel<T>> L, int nb, hipStream_t s);
+template <class T> int launch_nb_decode_set(LevelSet<NbLevel<T>> L, hipStream_t s);
+// GroupedBP: rows holds gb_set_row_words(n, nb) words (0: the level is too
+// large for a set)
+template <class T> struct GbLevel {
+    T *x;
+    const KeyOf<T> *key;
+    uint8_t *rb;
+    typename Traits<T>::Stream *planes, *signs;
+    uint32_t *rows, *words;
+    uint64_t stride;
+    uint32_t n;
+    int32_t k;
+};
+template <class T> size_t gb_set_row_words(uint32_t n, int nb);
+template <class T> int launch_gb_encode_set(LevelSet<GbLevel<T>> L, int nb, hipStream_t s);
+template <class T> int launch_gb_decode_set(LevelSet<GbLevel<T>> L, hipStream_t s);
+
 // ---- PerBit (PerBitBPEncoder.hpp:81-143) -------------------------------------
 // Stream p (64-bit words) at streams + p * stride, stride >= pb_stream_words(n);
 // sizes[p] (device) = its bytes, whole words.
@@ -141,6 +186,10 @@ template <class T> int mgard_solve_ahead(const LevelGeom &g, int l, double *f_l,
 // into f_l (rows of pitch round16(c2)); bytes of such a buffer
 template <class T> int mgard_recompose_load(const CoefSink<T> &src, const LevelGeom &g, int l, double *f_l, hipStream_t s);
 size_t mgard_level_f_bytes(const LevelGeom &g, int l);
+// the same of levels lo..hi (interleaved buffers) in one launch, into f_levels[l]
+template <class T>
+int mgard_recompose_load_set(const CoefSink<T> &src, const LevelGeom &g, int lo, int hi, double *const *f_levels,
+                             hipStream_t s);
 // Transpose of recompose (adjoint.hip): g_in = dJ/du on the level-L box
 // (strides in_strides), out = dJ/dcoefficients in the decompose layout.
 size_t adjoint_workspace_bytes(const LevelGeom &g);

@@ -1581,7 +1581,7 @@ template <class T, class SH> uint32_t sweep_tiles(const LoadParams<T> &P, int ma
     return t2n * t1n * march_tiles0(P.n[0], P.c[0], march);
 }
 
-template <class T, int MODE, class SH> void launch_sweep(LoadParams<T> P, bool ilv, hipStream_t s) {
+template <class T, int MODE, class SH> int sweep_march(const LoadParams<T> &P) {
     // march length: 16 coarse planes per workgroup, shorter when the level
     // has too few tiles to fill the 256 CUs (short marches = more
     // parallelism). Measured at 513^3, 6 levels: the decompose sweep keeps
@@ -1591,8 +1591,11 @@ template <class T, int MODE, class SH> void launch_sweep(LoadParams<T> P, bool i
     int march = 16;
     const uint64_t want = MODE == kDecompose ? 256 : 2048;
     while (march > 2 && sweep_tiles<T, SH>(P, march) < want) march /= 2;
-    P.march = march;
-    const uint32_t grid = sweep_tiles<T, SH>(P, march);
+    return march;
+}
+template <class T, int MODE, class SH> void launch_sweep(LoadParams<T> P, bool ilv, hipStream_t s) {
+    P.march = sweep_march<T, MODE, SH>(P);
+    const uint32_t grid = sweep_tiles<T, SH>(P, P.march);
     const bool a3 = P.n[0] > 1 && P.n[1] > 1 && P.n[2] > 1;
     const dim3 blk(SH::kThreads);
     if (ilv && a3) hipLaunchKernelGGL((k_load<T, MODE, true, true, SH>), dim3(grid), blk, 0, s, P);
@@ -1645,7 +1648,8 @@ int mgard_decompose(const T *in, const uint64_t *in_strides, const LevelGeom &g,
         LoadParams<T> P = load_params(g, l, sink);
         P.in = cur;
         P.is[0] = cs[0]; P.is[1] = cs[1]; P.is[2] = 1;
-        T *uc = bufs[which];
+        // the coarsest grid is the level-0 buffer itself (both dense)
+        T *uc = ilv && l == 1 ? sink.level[0] : bufs[which];
         P.uc = uc;
         P.f = f;
         P.fp = f_pitch(P.c[2]);
@@ -1672,11 +1676,10 @@ int mgard_decompose(const T *in, const uint64_t *in_strides, const LevelGeom &g,
     StageScope sc0(tm, kStDecCopy);
     const uint32_t *c0 = g.ld[0];
     if (ilv) {
-        int rc;
+        int rc = kOk;
         // a kernel rather than a copy node, so that the sequence captures
         // into a graph as kernel nodes only
         if (g.L == 0) rc = copy_box<T>(in, in_strides[0], in_strides[1], sink.level[0], (uint64_t)c0[1] * c0[2], c0[2], c0, s);
-        else rc = copy_box<T>(cur, cs[0], cs[1], sink.level[0], (uint64_t)c0[1] * c0[2], c0[2], c0, s);
         if (!rc && level_keys) rc = launch_maxabs<T>(sink.level[0], points3(c0), level_keys + 0, s);
         return rc ? rc : ready(0);
     }
@@ -1713,12 +1716,12 @@ int mgard_recompose(const CoefSink<T> &src, const LevelGeom &g, T *out, const ui
         if (ilv) return copy_box<T>(src.level[0], (uint64_t)c0[1] * c0[2], c0[2], out, out_strides[0], out_strides[1], c0, s);
         return copy_box<T>(src.full, src.s[0], src.s[1], out, out_strides[0], out_strides[1], c0, s);
     }
-    // coarsest grid into a dense buffer
+    // the coarsest grid: the level-0 buffer as it is, or the box of a full
+    // array into a dense buffer
     int which = 0;
-    T *cur = bufs[which];
-    int rc;
-    if (ilv) rc = copy_box<T>(src.level[0], (uint64_t)c0[1] * c0[2], c0[2], cur, (uint64_t)c0[1] * c0[2], c0[2], c0, s);
-    else rc = copy_box<T>(src.full, src.s[0], src.s[1], cur, (uint64_t)c0[1] * c0[2], c0[2], c0, s);
+    const T *cur = ilv ? src.level[0] : bufs[which];
+    int rc = kOk;
+    if (!ilv) rc = copy_box<T>(src.full, src.s[0], src.s[1], bufs[which], (uint64_t)c0[1] * c0[2], c0[2], c0, s);
     if (rc) return rc;
     for (int l = 1; l <= g.L; l++) {
         if ((rc = need(l))) return rc;
@@ -1734,8 +1737,10 @@ int mgard_recompose(const CoefSink<T> &src, const LevelGeom &g, T *out, const ui
             }
             if (rc) return rc;
             StageScope sc(tm, l == g.L ? kStRecSolveTop : kStRecSolveRest);
-            rc = solve_all<T>(g, l, fl, kEpiSub, cur, cur, s);  // u_c = u_c' - z, in place
+            // u_c = u_c' - z, in place but for the level-0 buffer
+            rc = solve_all<T>(g, l, fl, kEpiSub, cur, bufs[which], s);
             if (rc) return rc;
+            if (g.points[l] > 1) cur = bufs[which];  // a single point has no line
         }
         const uint32_t *n = g.ld[l];
         T *dst;
@@ -1807,6 +1812,41 @@ size_t mgard_level_f_bytes(const LevelGeom &g, int l) {
     const uint32_t *c = g.ld[l - 1];
     return (size_t)c[0] * c[1] * f_pitch(c[2]) * sizeof(double);
 }
+
+template <class T, bool A3>
+__global__ __launch_bounds__(SweepStd::kThreads) void k_load_set(LevelSet<LoadParams<T>> L) {
+    __shared__ SweepLds<T, kRecompose> lds;
+    const uint32_t i = set_entry(L, blockIdx.x);
+    load_tile<T, kRecompose, true, A3>(L.e[i], xcd_remap(blockIdx.x - L.first[i], L.first[i + 1] - L.first[i]), lds);
+}
+template <class T>
+int mgard_recompose_load_set(const CoefSink<T> &src, const LevelGeom &g, int lo, int hi, double *const *f_levels,
+                             hipStream_t s) {
+    if (lo < 1 || hi > g.L || hi - lo >= kSetMax || src.full) { set_error("recompose load set: bad levels"); return kErrArg; }
+    LevelSet<LoadParams<T>> L;
+    static_assert(sizeof(L) <= 4096, "kernel argument limit");
+    for (int l = lo; l <= hi; l++) {
+        LoadParams<T> P = load_params(g, l, src);
+        P.f = f_levels[l];
+        P.fp = f_pitch(P.c[2]);
+        if (!sweep_planes_fit(P)) {
+            set_error("a fine plane of this level spans 2 GiB or more; the sweeps address planes with 31-bit offsets");
+            return kErrUnsupported;
+        }
+        P.march = sweep_march<T, kRecompose, SweepStd>(P);
+        L.e[L.n++] = P;
+    }
+    if (!L.n) return kOk;
+    set_sizes(L, [](const LoadParams<T> &P) { return load_tiles(P); });
+    // a dim of more than one node stays so at every level above 0
+    const bool a3 = g.dims[0] > 1 && g.dims[1] > 1 && g.dims[2] > 1;
+    if (a3) hipLaunchKernelGGL((k_load_set<T, true>), dim3(L.first[L.n]), dim3(SweepStd::kThreads), 0, s, L);
+    else hipLaunchKernelGGL((k_load_set<T, false>), dim3(L.first[L.n]), dim3(SweepStd::kThreads), 0, s, L);
+    PRODM_CHECK_LAUNCH();
+    return kOk;
+}
+template int mgard_recompose_load_set<float>(const CoefSink<float> &, const LevelGeom &, int, int, double *const *, hipStream_t);
+template int mgard_recompose_load_set<double>(const CoefSink<double> &, const LevelGeom &, int, int, double *const *, hipStream_t);
 
 template <class T> int mgard_recompose_load(const CoefSink<T> &src, const LevelGeom &g, int l, double *f_l, hipStream_t s) {
     if (l < 1 || l > g.L || !f_l) { set_error("recompose load: bad level"); return kErrArg; }

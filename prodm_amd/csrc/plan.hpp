@@ -24,6 +24,7 @@ struct prodm_mdr_plan {
     void *signs = nullptr;           // GroupedBP decode signs
     void *gbws = nullptr;
     size_t gbws_bytes = 0;
+    uint32_t *gbrows = nullptr;      // GroupedBP: words rows of the small levels
     uint64_t device_bytes = 0;
     prodm::StageTimer timer;
     int hier = 0;  // PRODM_DECOMP_HIERARCHICAL
