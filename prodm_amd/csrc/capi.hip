@@ -342,13 +342,15 @@ static int plan_flev(prodm_mdr_plan *p) {
 
 template <class F> static int hook_call(void *ctx, int level) { return (*static_cast<F *>(ctx))(level); }
 
-// Levels 0 .. small_top(p) (-1: none) are small: at most kSmallLevel elements,
-// 1 MB or 2 MB, 2 us of HBM traffic. Their encodes, decodes and recompose load
-// sweeps are launched together, and a plan of small levels only runs on the
-// caller's stream alone: there a launch or an event costs more than it would
-// overlap. Refactor + retrieve of 33^3: 240 -> 141 us; of 65^3, GroupedBP: 336
-// -> 216; fp64 161 x 257, GroupedBP: 480 -> 189.
-constexpr uint64_t kSmallLevel = uint64_t(1) << 18;
+// Levels 0 .. small_top(p) (-1: none) are small: at most kSmallLevel elements.
+// Their encodes, decodes and recompose load sweeps are launched together, and a
+// plan of small levels only runs on the caller's stream alone: there a launch
+// or an event costs more than it would overlap. 2^21 is also the largest level
+// whose GroupedBP rows a workgroup adds up by itself (kGbScanRows of them).
+// Refactor + retrieve of 33^3: 240 -> 141 us; 129^3: 318 -> 244, GroupedBP
+// 357 -> 263 (its finest level, 1.87e6, launched by itself on a second stream:
+// 290, 309); 1025^2: 400 -> 346; 257^3 GroupedBP f64: 742 -> 696.
+constexpr uint64_t kSmallLevel = uint64_t(1) << 21;
 static int small_top(const prodm_mdr_plan *p) {
     int top = -1;
     while (top < p->g.L && top + 1 < kSetMax && p->g.elems[top + 1] <= kSmallLevel) top++;
