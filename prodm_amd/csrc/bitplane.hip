@@ -1484,7 +1484,7 @@ __global__ __launch_bounds__(kPbTPB) void k_pb_write(const T *__restrict__ x, ui
     PbLane<T> P;
     P.load(x, ((uint64_t)blockIdx.x * kPbTPB + threadIdx.x) * B, n, nb - level_exp<T>(exp, key), compat,
            ((uintptr_t)x & 15) == 0);
-    const uint32_t S = P.sg;  // sign bits of the lane's elements
+    const uint32_t S = P.sg, S1 = S << 1;  // sign bits of the lane's elements
     // first-1 flags of the lanes below and of the wave: for f32 two planes
     // per scan, computed before the plane loop (16 words); f64's 64 planes
     // would hold 32 of them, so it scans per plane
@@ -1512,17 +1512,25 @@ __global__ __launch_bounds__(kPbTPB) void k_pb_write(const T *__restrict__ x, ui
             flags = readlane_u32(pre + c, 63);
         }
         const uint32_t q = (uint32_t)(o & 63) + below + pre;
-        // insert each flagged element's sign after its bit, highest first
-        uint64_t r = D;
-        uint32_t ff = F;
+        // insert each flagged element's sign after its bit, highest first:
+        // adding the bits above an element to themselves moves them up by
+        // one (the low word's carry is the high word's new bit 0). c = the bit
+        // above the element; element 31, whose c is in the high word, first. The
+        // loop runs as often as the lane with the most flags needs and is what
+        // bounds the kernel: with 64-bit masks and shifts 2^27 - 2^24 fp32
+        // elements took 431 us, the whole encode 580 -> 513
+        uint32_t lo = D, hi = (S & F) >> 31;
+        uint32_t ff = F << 1;
         while (ff) {
-            const int j = 31 - __clz(ff);
-            ff ^= 1u << j;
-            const uint64_t low = (2ull << j) - 1;
-            r = (r & low) | ((uint64_t)((S >> j) & 1u) << (j + 1)) | ((r & ~low) << 1);
+            const uint32_t c = 0x80000000u >> __clz(ff);
+            ff ^= c;
+            const uint64_t up = (uint64_t)lo + (lo & (0u - c));
+            hi = hi + hi + (uint32_t)(up >> 32);
+            lo = (uint32_t)up | (S1 & c);
         }
+        const uint64_t r = ((uint64_t)hi << 32) | lo;
         const uint32_t wi = q >> 6, sh = q & 63;
-        const uint64_t w0 = r << sh, w1 = sh ? r >> (64 - sh) : 0;
+        const uint64_t w0 = r << sh, w1 = (r >> 1) >> (63 - sh);
         atomicOr(&buf[wi], w0);  // unconditional: OR-ing zero is harmless and needs no branch
         atomicOr(&buf[wi + 1], w1);
         // whole words of this run are stored; a first word shared with the
