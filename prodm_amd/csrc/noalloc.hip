@@ -3,15 +3,15 @@
 // device allocation, for callers that cannot allocate (code under HIP graph
 // capture, serving loops, harnesses that forbid hipMalloc).
 //
-// The encode's kernels (k_gb_rb, k_gb_scan, k_gb_write) keep per-workgroup
-// recording-plane histograms and the scanned plane offsets in a scratch
-// buffer. Here that buffer is `scratch`, a file-scope device array of
+// The encode's kernels (k_gb_rb, k_gb_sums, k_gb_offsets, k_gb_write) keep a
+// row of words per plane for each workgroup, and its scanned offsets, in a
+// scratch buffer. Here that buffer is `scratch`, a file-scope device array of
 // kScratchBytes that every GPU the library runs on holds until the process
 // ends. Its device address is looked up once per device
 // (hipGetSymbolAddress, with that device current) and passed to the kernels
 // as the workspace; the host-side name `scratch` is never used as an address.
-// Each call overwrites the part it uses before reading it (every histogram
-// and offset is written by the call itself), so nothing needs clearing.
+// Each call overwrites the part it uses before reading it (every row and
+// offset is written by the call itself), so nothing needs clearing.
 // Calls that overlap on one GPU (two streams at once) share the array and
 // race; serialize them.
 #include <mutex>
