@@ -127,7 +127,15 @@ def negabinary_encode(x, exp, nb):
     B = _BLOCK[x.dtype]
     nw = (n + B - 1) // B
     stride = (nw + 1) & ~1
-    planes = torch.zeros((nb, stride), dtype=_WORD[x.dtype], device=x.device)
+    # the encoder writes every plane's nw words, so only a pad column has to be
+    # cleared: a fill of all planes is a pass over memory (118 M float32
+    # elements: 437 us with it, 353 without). Up to 2^20 words the fill costs
+    # less than the strided clear's slicing (20,000 elements: 45 against 47 us)
+    pad = stride > nw
+    make = torch.zeros if pad and nb * stride <= 1 << 20 else torch.empty
+    planes = make((nb, stride), dtype=_WORD[x.dtype], device=x.device)
+    if pad and make is torch.empty:
+        planes[:, nw:].zero_()
     check(_fn("prodm_negabinary_encode", x.dtype)(_ptr(x), n, exp, nb, _ptr(planes), stride, _stream()),
           "negabinary encode")
     return planes
@@ -154,9 +162,10 @@ def grouped_encode(x, exp, nb, compat=False):
     B = _BLOCK[x.dtype]
     nblk = (n - 1) // B + 1
     stride = 2 * nblk
-    rb = torch.zeros(nblk, dtype=torch.uint8, device=x.device)
+    # rb and words are written whole, a plane's row only up to its words
+    rb = torch.empty(nblk, dtype=torch.uint8, device=x.device)
     planes = torch.zeros((nb, stride), dtype=_WORD[x.dtype], device=x.device)
-    words = torch.zeros(nb, dtype=torch.int32, device=x.device)
+    words = torch.empty(nb, dtype=torch.int32, device=x.device)
     wsb = lib().prodm_grouped_workspace_bytes(n, nb, _TDT[x.dtype])
     ws = _ws(wsb)
     check(_fn("prodm_grouped_encode", x.dtype)(_ptr(x), n, exp, nb, int(compat), _ptr(rb), _ptr(planes), stride,
