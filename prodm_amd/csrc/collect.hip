@@ -165,11 +165,17 @@ struct Acc3 {
     }
 };
 
-// one finite term outside the grids, into the 128-bit sum of its exponent
-__device__ __forceinline__ void add_under(double t, int bin, unsigned long long *under, uint32_t *flag) {
+// one term outside the grids, into the 128-bit sum of its exponent. A term that
+// is infinite or NaN has no sum and is left out, or (over) counts as its float's
+// bits read as a number: infinity is 2^128.
+__device__ __forceinline__ void add_under(double t, int bin, unsigned long long *under, uint32_t *flag, bool over) {
     const uint64_t tb = to_bits(t);
-    const int be = (int)((tb >> 52) & 0x7ff);
-    if (!(tb << 1) || be == 0x7ff) return;  // zero; infinite and NaN terms have no sum
+    int be = (int)((tb >> 52) & 0x7ff);
+    if (!(tb << 1)) return;
+    if (be == 0x7ff) {
+        if (!over) return;
+        be = 1023 + 128;
+    }
     const unsigned long long M = (tb & ((1ull << 52) - 1)) | (be ? (1ull << 52) : 0);
     unsigned long long *bk = under + ((size_t)bin * kExBuckets + (be ? be : 1)) * 2;
     const unsigned long long old = atomicAdd(bk, M);
@@ -329,10 +335,17 @@ __device__ inline T sq_term(T x, int de, int le, int nb, int k) {
 // have the term x^2 in every entry and are summed once; subnormal ones above
 // that (whose bits do not shift with de) and ones past the bound go term by
 // term to the buckets.
+// Squares are float. One past the largest float counts as 2^128, as in the CPU
+// restatement (infinity's bits read as a number), so that no term is above 2^128
+// and 2^128 is on the grid of any step up to it. Only entries with le - k > 64
+// reach it and take the minimum. Elements past the bound, infinite or NaN have
+// such terms too: theirs count where a 128-bit window from 2^q reaches 2^128
+// (le > nb + 23), and are left out elsewhere.
+constexpr double kSqOver = 0x1p128;
 __host__ __device__ inline Grid3 sq_grid(int k, int le, int nb) {
     if (k > nb) return grid3_open(2 * (le - nb));
-    const int q = 2 * (le - nb - 23);
-    return grid3(2 * (le - k), q > -149 ? q : -149);
+    const int q = 2 * (le - nb - 23), t = 2 * (le - k);
+    return grid3(t < 128 ? t : 128, q < -149 ? -149 : q > 128 ? 128 : q);
 }
 __global__ __launch_bounds__(kExThreads) void k_collect_squared_f32(const float *__restrict__ x, uint64_t n, int nb,
                                                                     int le, uint64_t *__restrict__ partial,
@@ -368,21 +381,29 @@ __global__ __launch_bounds__(kExThreads) void k_collect_squared_f32(const float 
                 const int de = dev_frexp_exp(t);
                 if (de <= le - nb && fabsf(t) < __builtin_inff()) {
                     const float tt = t * t;
-                    if (!tiny.add_open((double)tt)) add_under((double)tt, nb + 1, under, flag);
+                    const double td = fmin((double)tt, kSqOver);
+                    if (!tiny.add_open(td)) add_under(td, nb + 1, under, flag, false);
                 } else {
-                    for (int k = 0; k <= nb; k++) add_under((double)sq_term<float>(t, de, le, nb, k), k, under, flag);
+                    for (int k = 0; k <= nb; k++)
+                        add_under((double)sq_term<float>(t, de, le, nb, k), k, under, flag, le > nb + 23);
                 }
             }
             tiny.flush(acc + (nb + 1) * 3 * kExSlots);
         }
         for (int k = 0; k <= nb; k++) {
-            sum_bin(sq_grid(k, le, nb), acc + k * 3 * kExSlots, [&](int i) __attribute__((always_inline)) -> double {
+            auto term = [&](int i) __attribute__((always_inline)) -> double {
                 const int b = cut[i] - k;
                 const uint32_t keep = 0xffffffffu << (b > 23 ? 31 : max(b, 0));
                 const float d = v[i] - from_bits<float>(to_bits(v[i]) & keep);
                 const float t = d * d;
                 return (double)t;
-            });
+            };
+            const Grid3 g = sq_grid(k, le, nb);
+            unsigned long long *const slot = acc + k * 3 * kExSlots;
+            if (le - k > 64)
+                sum_bin(g, slot, [&](int i) __attribute__((always_inline)) -> double { return fmin(term(i), kSqOver); });
+            else
+                sum_bin(g, slot, term);
         }
     }
     __syncthreads();
@@ -660,10 +681,10 @@ __global__ __launch_bounds__(kExThreads) void k_fused_errors(const float *__rest
                 if (fabsf(s) < 1.0f) {
                     const double d = (double)s * (double)s;
                     const float ff = s * s;
-                    if (!tinyd.add_open(d)) add_under(d, nb + 1, under, flag);
-                    if (!tinyf.add_open((double)ff)) add_under((double)ff, nb + 2, under, flag);
+                    if (!tinyd.add_open(d)) add_under(d, nb + 1, under, flag, false);
+                    if (!tinyf.add_open((double)ff)) add_under((double)ff, nb + 2, under, flag, false);
                 } else {
-                    for (int k = 0; k <= nb; k++) add_under(fe_term<ENC>(s, mm, bb, nb, k), k, under, flag);
+                    for (int k = 0; k <= nb; k++) add_under(fe_term<ENC>(s, mm, bb, nb, k), k, under, flag, false);
                 }
             }
             tinyd.flush(acc + (nb + 1) * 3 * kExSlots);
