@@ -351,6 +351,7 @@ template <class F> static int hook_call(void *ctx, int level) { return (*static_
 // 357 -> 263 (its finest level, 1.87e6, launched by itself on a second stream:
 // 290, 309); 1025^2: 400 -> 346; 257^3 GroupedBP f64: 742 -> 696.
 constexpr uint64_t kSmallLevel = uint64_t(1) << 21;
+constexpr uint64_t kBehindFinest = uint64_t(3) << 24;  // see plan_retrieve
 static int small_top(const prodm_mdr_plan *p) {
     int top = -1;
     while (top < p->g.L && top + 1 < kSetMax && p->g.elems[top + 1] <= kSmallLevel) top++;
@@ -630,11 +631,23 @@ template <class T> static int plan_retrieve(prodm_mdr_plan *p, const uint8_t *k,
     // is the one such level
     const bool split = g.L >= 1 && (p->encoder == PRODM_ENC_NEGABINARY || top == g.L - 1);
     if (split) PRODM_HIP(hipStreamWaitEvent(p->side2, p->join_ev, 0));
+    // Levels between the small ones and a large finest one are decoded after the
+    // finest: the small ones in one launch leave the side stream to them from
+    // the start, where their decodes and sweeps slow the finest's decode and
+    // sweep, the longest chain, and the main stream needs them late. Retrieve
+    // of 513^3: 900 -> 883 us (888 with the small levels one by one), 769 x 769
+    // x 257 1138 -> 1114 (1121), 513 x 513 x 257 f64 836 -> 818 (831). A finest
+    // level below the line leaves room for them: 385^3 (49.9e6) 557 -> 556,
+    // 353^3 (38.5e6) 359 -> 362, 513 x 513 x 129 436 -> 440. The hierarchical
+    // retrieve has no sweeps and loses by it (513^3 captured 448 -> 461).
+    const bool behind = split && ahead && top < g.L - 1 && g.elems[g.L] >= kBehindFinest;
     auto level = [&](int l, hipStream_t ss) -> int {
         if (l <= top) {
             if (int r = decode_small(ss)) return r;
         } else {
+            if (behind && l == top + 1) PRODM_HIP(hipStreamWaitEvent(ss, p->join_ev, 0));
             if (int r = decode_level(l, ss)) return r;
+            if (behind && l == g.L) PRODM_HIP(hipEventRecord(p->join_ev, ss));  // the fork above is past it
             if (ahead && l >= 1)
                 if (int r = mgard_recompose_load<T>(src, g, l, fl[l], ss)) return r;
             // the finest level's solves need only its load vector: they run here,
