@@ -478,6 +478,17 @@ static int plan_pin(prodm_mdr_plan *p, size_t bytes) {
     return kOk;
 }
 
+// Waits for a stream when it goes out of scope, unless released: declared after
+// host buffers that copies on the stream use, so that a return on an error
+// leaves none of them queued.
+struct StreamDrain {
+    hipStream_t s;
+    bool on = true;
+    ~StreamDrain() {
+        if (on) (void)hipStreamSynchronize(s);
+    }
+};
+
 // PerBit planes [0, k[l]) of every level decoded on the host (the streams
 // have no index of where an element's bits begin) into the level buffers.
 // Plane bytes and values go through the pinned staging, so that every copy of
@@ -490,9 +501,17 @@ template <class T> static int perbit_decode_levels(prodm_mdr_plan *p, const uint
     const size_t nsizes = (size_t)(g.L + 1) * p->nb;
     std::vector<uint32_t> sizes(nsizes);
     std::vector<KeyOf<T>> keys(g.L + 1);
+    std::vector<uint8_t> paged;
+    StreamDrain drain{s};
     PRODM_HIP(hipMemcpyAsync(sizes.data(), p->words, nsizes * 4, hipMemcpyDeviceToHost, s));
     PRODM_HIP(hipMemcpyAsync(keys.data(), p->keys, keys.size() * sizeof(T), hipMemcpyDeviceToHost, s));
     PRODM_HIP(hipStreamSynchronize(s));
+    for (int l = 0; l <= g.L; l++)
+        for (int i = 0; i < k[l]; i++)
+            if (sizes[(size_t)l * p->nb + i] > p->plane_stride[l] * p->elem) {
+                set_error("retrieve: plane larger than its storage");
+                return kErrState;
+            }
     // a small level's planes come as they lie, in one copy; a large one's each
     // by itself, without the unused ends
     auto whole = [&](int l) { return k[l] * p->plane_stride[l] * p->elem <= (size_t(1) << 20); };
@@ -507,7 +526,6 @@ template <class T> static int perbit_decode_levels(prodm_mdr_plan *p, const uint
     const bool pinned = need <= kPinMax;
     if (pinned)
         if (int rc = plan_pin(p, need)) return rc;
-    std::vector<uint8_t> paged;
     std::vector<std::vector<const uint64_t *>> ptrs(g.L + 1);
     std::vector<T *> vals(g.L + 1);
     // places of level l's values and planes in `at`, and the copies of its planes
@@ -520,7 +538,6 @@ template <class T> static int perbit_decode_levels(prodm_mdr_plan *p, const uint
         if (whole(l) && k[l]) PRODM_HIP(hipMemcpyAsync(at, base, k[l] * pitch, hipMemcpyDeviceToHost, s));
         for (int i = 0; i < k[l]; i++) {
             const size_t bytes = sizes[(size_t)l * p->nb + i];
-            if (bytes > pitch) { set_error("retrieve: plane larger than its storage"); return kErrState; }
             ptrs[l][i] = reinterpret_cast<const uint64_t *>(at);
             if (!whole(l) && bytes) PRODM_HIP(hipMemcpyAsync(at, base + i * pitch, bytes, hipMemcpyDeviceToHost, s));
             at += whole(l) ? pitch : (bytes + 7) / 8 * 8;
@@ -557,9 +574,11 @@ template <class T> static int perbit_decode_levels(prodm_mdr_plan *p, const uint
             (hipMemcpyAsync(dst, vals[l], n * sizeof(T), hipMemcpyHostToDevice, s) != hipSuccess ||
              (!pinned && hipStreamSynchronize(s) != hipSuccess))) { set_error("retrieve: level upload"); rc = kErrHip; }
     }
-    if (pinned && hipEventRecord(p->pin_ev, s) != hipSuccess && !rc) { set_error("retrieve: event record"); rc = kErrHip; }
     prodm_perbit_state_destroy(st);
-    return rc;
+    if (rc) return rc;
+    if (pinned) PRODM_HIP(hipEventRecord(p->pin_ev, s));  // the next call waits for it
+    drain.on = false;
+    return kOk;
 }
 
 template <class T> static int plan_retrieve(prodm_mdr_plan *p, const uint8_t *k, T *out, hipStream_t s) {
