@@ -312,6 +312,7 @@ static void plan_free(prodm_mdr_plan *p) {
     if (p->join_ev) (void)hipEventDestroy(p->join_ev);
     if (p->pin) (void)hipHostFree(p->pin);
     if (p->pin_ev) (void)hipEventDestroy(p->pin_ev);
+    if (p->max_ev) (void)hipEventDestroy(p->max_ev);
     if (p->side) (void)hipStreamDestroy(p->side);
     if (p->side2) (void)hipStreamDestroy(p->side2);
     void *ptrs[] = {p->ws, p->levels, p->keys, p->planes, p->rb, p->words, p->signs, p->gbws, p->gbrows, p->flev};
@@ -503,6 +504,7 @@ template <class T> static int perbit_decode_levels(prodm_mdr_plan *p, const uint
     std::vector<KeyOf<T>> keys(g.L + 1);
     std::vector<uint8_t> paged;
     StreamDrain drain{s};
+    if (p->max_ev) PRODM_HIP(hipStreamWaitEvent(s, p->max_ev, 0));
     PRODM_HIP(hipMemcpyAsync(sizes.data(), p->words, nsizes * 4, hipMemcpyDeviceToHost, s));
     PRODM_HIP(hipMemcpyAsync(keys.data(), p->keys, keys.size() * sizeof(T), hipMemcpyDeviceToHost, s));
     PRODM_HIP(hipStreamSynchronize(s));
@@ -1162,15 +1164,29 @@ int prodm_mdr_load_plane_stream(prodm_mdr_plan *p, int level, int plane, const u
 int prodm_mdr_set_level_max(prodm_mdr_plan *p, int level, double max_abs, prodm_stream_t stream) {
     if (!p || level < 0 || level > p->g.L || !(max_abs >= 0)) { set_error("set_level_max: bad arguments"); return kErrArg; }
     hipStream_t s = (hipStream_t)stream;
+    int rc;
     if (p->dtype == PRODM_F32) {
         const float f = (float)max_abs;
         uint32_t k;
         std::memcpy(&k, &f, 4);
-        return launch_fill_u32(reinterpret_cast<uint32_t *>(p->keys) + level, 1, k, s);
+        rc = launch_fill_u32(reinterpret_cast<uint32_t *>(p->keys) + level, 1, k, s);
+    } else {
+        uint64_t k;
+        std::memcpy(&k, &max_abs, 8);
+        rc = launch_fill_u64(reinterpret_cast<uint64_t *>(p->keys) + level, 1, k, s);
     }
-    uint64_t k;
-    std::memcpy(&k, &max_abs, 8);
-    return launch_fill_u64(reinterpret_cast<uint64_t *>(p->keys) + level, 1, k, s);
+    if (rc || p->encoder != PRODM_ENC_PERBIT) return rc;
+    // the PerBit retrieve reads the maxima on the host, from any stream: it
+    // waits for this event, which comes after the other streams' ones
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone) {
+        (void)hipGetLastError();
+        return kOk;  // a graph's replays are ordered by their caller
+    }
+    if (p->max_ev) PRODM_HIP(hipStreamWaitEvent(s, p->max_ev, 0));
+    else PRODM_HIP(hipEventCreateWithFlags(&p->max_ev, hipEventDisableTiming));
+    PRODM_HIP(hipEventRecord(p->max_ev, s));
+    return kOk;
 }
 
 // Capture `body` on stream s into a graph executable (kernel nodes only).

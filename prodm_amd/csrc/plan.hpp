@@ -44,6 +44,7 @@ struct prodm_mdr_plan {
     void *pin = nullptr;          // pinned staging of the PerBit retrieve's host decode
     size_t pin_bytes = 0;
     hipEvent_t pin_ev = nullptr;  // its last upload
+    hipEvent_t max_ev = nullptr;  // PerBit: the last level maximum set by the caller
     bool capturing = false;  // a graph capture is in progress (the PerBit retrieve has no graph form)
     // per-level load vectors of the retrieve pipeline (allocated on first use)
     void *flev = nullptr;

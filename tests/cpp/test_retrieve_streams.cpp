@@ -2,6 +2,7 @@
 // HIP calls that the library makes (its own symbols come before libamdhip64's)
 // over host memory, with streams as queues that run only when something waits
 // for them and a copy that can be told to fail.
+//   - a level maximum set on another stream is waited for
 //   - no copy is left on the stream after a retrieve that failed
 #include <hip/hip_runtime_api.h>
 
@@ -136,6 +137,25 @@ static int small_plan(prodm_mdr_plan **p, int nb) {
     return 0;
 }
 
+static int maxima_of_other_streams() {
+    prodm_mdr_plan *p = nullptr;
+    CHECK(small_plan(&p, 1) == 0);
+    // level 0's maximum on one stream, level 1's on another, the retrieve on a third
+    CHECK(prodm_mdr_set_level_max(p, 0, 3.0, stream(0)) == 0);
+    CHECK(prodm_mdr_set_level_max(p, 1, 1.0, stream(1)) == 0);
+    const uint8_t k[2] = {1, 1};
+    float out[3];
+    CHECK(prodm_mdr_retrieve(p, k, out, stream(2)) == 0);
+    (void)hipStreamSynchronize(stream(2));
+    void *c = nullptr;
+    CHECK(prodm_mdr_level_coefficients(p, 0, &c) == 0);
+    const float *v = static_cast<const float *>(c);
+    printf("level 0: %g %g\n", v[0], v[1]);
+    CHECK(v[0] == 2.0f && v[1] == -2.0f);
+    prodm_mdr_plan_destroy(p);
+    return 0;
+}
+
 // copies of a retrieve that fails one after the other, then one that does not
 static int failed_copies(const uint32_t n, int L, int nb, int copies) {
     prodm_mdr_plan *p = nullptr;
@@ -176,8 +196,9 @@ int main(int argc, char **argv) {
     const std::string what = argc > 1 ? argv[1] : "";
     // errors: small levels (sizes, maxima, a copy and an upload per level), then
     // 2^24 + 1 values, past the pinned staging (sizes, maxima, a copy per plane, an upload)
-    const int bad = what == "errors" ? failed_copies(3, 1, 3, 6) || failed_copies((1u << 24) + 1, 0, 3, 6)
-                                      : 1;
+    const int bad = what == "maxima"   ? maxima_of_other_streams()
+                    : what == "errors" ? failed_copies(3, 1, 3, 6) || failed_copies((1u << 24) + 1, 0, 3, 6)
+                                       : 1;
     if (!bad) printf("PASSED\n");
     return bad;
 }

@@ -1,4 +1,4 @@
-"""The PerBit retrieve's error exits, on the
+"""The PerBit retrieve's ordering between streams and its error exits, on the
 CPU: tests/cpp/test_retrieve_streams.cpp runs the library over HIP calls of its
 own."""
 import os
@@ -10,7 +10,7 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 
 
-@pytest.mark.parametrize("what", ["errors"])
+@pytest.mark.parametrize("what", ["maxima", "errors"])
 def test_perbit_retrieve_streams(tmp_path, what):
     lib = os.path.join(ROOT, "prodm_amd")
     exe = str(tmp_path / "test_retrieve_streams")
