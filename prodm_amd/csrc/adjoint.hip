@@ -155,9 +155,28 @@ int mgard_recompose_adjoint(const T *g_in, const uint64_t *in_strides, const Lev
     double *hb[2] = {reinterpret_cast<double *>(base + A.h0), reinterpret_cast<double *>(base + A.h1)};
     void *mws = base + A.mgard;
     const size_t mws_bytes = A.total - A.mgard;
-    if (g.L == 0) {
-        hipLaunchKernelGGL((k_adj_copy<T, T>), grid_of(g.ld[0]), dim3(256), 0, s, g_in, in_strides[0], in_strides[1],
-                           g.ld[0][2], out, out_strides[0], out_strides[1]);
+    // the sweep reads g in place, after the output's first stores: a box whose
+    // memory meets the output's is first copied to a dense FP64 grid, and so
+    // is one whose plane spans 2 GiB or more of its array (31-bit offsets)
+    const uint32_t *n = g.ld[g.L];
+    auto bytes = [&](const uint64_t *st) {
+        return ((uint64_t)(n[0] - 1) * st[0] + (uint64_t)(n[1] - 1) * st[1] + n[2]) * sizeof(T);
+    };
+    const uintptr_t gi = reinterpret_cast<uintptr_t>(g_in), oi = reinterpret_cast<uintptr_t>(out);
+    bool dense = gi < oi + bytes(out_strides) && oi < gi + bytes(in_strides);
+    const double *cur = nullptr;
+    uint64_t cs[2] = {(uint64_t)n[1] * n[2], n[2]};
+    auto copy_in = [&]() -> int {
+        double *gd = reinterpret_cast<double *>(base + A.g);
+        hipLaunchKernelGGL((k_adj_copy<T, double>), grid_of(n), dim3(256), 0, s, g_in, in_strides[0], in_strides[1],
+                           n[2], gd, cs[0], cs[1]);
+        PRODM_CHECK_LAUNCH();
+        cur = gd;
+        return kOk;
+    };
+    if (g.L == 0 && !dense) {
+        hipLaunchKernelGGL((k_adj_copy<T, T>), grid_of(n), dim3(256), 0, s, g_in, in_strides[0], in_strides[1], n[2], out,
+                           out_strides[0], out_strides[1]);
         PRODM_CHECK_LAUNCH();
         return kOk;
     }
@@ -177,22 +196,13 @@ int mgard_recompose_adjoint(const T *g_in, const uint64_t *in_strides, const Lev
         PRODM_CHECK_LAUNCH();
         return kOk;
     };
-    // the sweep reads g in place; a box whose plane spans 2 GiB or more of its
-    // array (31-bit offsets) is first copied to a dense FP64 grid
-    const uint32_t *n = g.ld[g.L];
-    if ((uint64_t)n[1] * n[2] * sizeof(double) >= 0x7FFFFFFFull) {
+    if (g.L > 0 && (uint64_t)n[1] * n[2] * sizeof(double) >= 0x7FFFFFFFull) {
         set_error("a fine plane of this level spans 2 GiB or more; the sweeps address planes with 31-bit offsets");
         return kErrUnsupported;
     }
-    const double *cur = nullptr;
-    uint64_t cs[2] = {(uint64_t)n[1] * n[2], n[2]};
-    if (((uint64_t)(n[1] - 1) * in_strides[1] + n[2]) * sizeof(T) >= 0x7FFFFFFFull) {
-        double *gd = reinterpret_cast<double *>(base + A.g);
-        hipLaunchKernelGGL((k_adj_copy<T, double>), grid_of(n), dim3(256), 0, s, g_in, in_strides[0], in_strides[1],
-                           n[2], gd, cs[0], cs[1]);
-        PRODM_CHECK_LAUNCH();
-        cur = gd;
-    }
+    dense = dense || ((uint64_t)(n[1] - 1) * in_strides[1] + n[2]) * sizeof(T) >= 0x7FFFFFFFull;
+    if (dense)
+        if (int rc = copy_in()) return rc;
     for (int l = g.L, which = 0; l >= 1; l--, which ^= 1) {
         const int rc = cur ? level(cur, cs, l, hb[which]) : level(g_in, in_strides, l, hb[which]);
         if (rc) return rc;
