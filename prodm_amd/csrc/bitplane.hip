@@ -822,20 +822,26 @@ __global__ __launch_bounds__(kGbTPB) void k_gb_rb(const T *__restrict__ x, uint3
 // k_gb_sums takes the column sums of each such group, k_gb_offsets adds those
 // of the groups before its own. (One workgroup per plane that summed the
 // histogram bins of every row took 1,600 us for 57,700 rows x 64 planes; the
-// two launches take 41 us for that level, now 28,850 rows.) A level of at
-// most kGbScanRows workgroups takes no scan launch: gb_wave_base adds the rows
-// of the workgroups before its own, which costs each of them less than the
-// 6 us launch (129^3 GroupedBP refactor + retrieve 413 -> 361 us).
+// two launches take 13 us for that level, now 28,850 rows.) A level of at
+// most kGbDirectRows workgroups takes no scan launch: gb_wave_base adds the rows
+// of the workgroups before its own, which costs less than the two launches
+// (129^3 GroupedBP refactor + retrieve 413 -> 361 us; encode and a decode of two
+// planes of floats: 367 rows 25 -> 21 and 22 -> 15 us, 733 rows 29 -> 27 and
+// 24 -> 20, 977 rows 31 and 24 either way).
 constexpr int kGbScanRows = 256, kGbScanPer = kGbScanRows / kGbWaves;
+constexpr int kGbDirectRows = 768;
 __device__ __forceinline__ void gb_scan_load(const uint32_t *__restrict__ rows, uint32_t nrow, int k, uint32_t r0,
                                              uint32_t (&v)[kGbScanPer], uint32_t &sum) {
-    const int lane = (int)lane_id();
-    const bool on = lane < k;
+    const uint32_t lane = lane_id();
+    const auto r = buf_rsrc(rows, true);
+    // masked by offset (rows take at most 2^27 bytes, so a masked lane's stays
+    // out of range): a select between addresses becomes a branch per load, and
+    // each is waited for by itself (367 rows: k_gb_sums 17 us, now 3)
+    const uint32_t at = (int)lane < k ? (r0 * (uint32_t)k + lane) * 4 : kOffNone;
 #pragma unroll
     for (int i = 0; i < kGbScanPer; i++) {
-        // unconditional loads (an unused one reads the first word), so that none waits for another
-        const uint32_t t = rows[on && r0 + i < nrow ? (uint64_t)(r0 + i) * k + lane : 0];
-        v[i] = on && r0 + i < nrow ? t : 0u;
+        const uint32_t in = at + i * (uint32_t)k * 4;
+        v[i] = buf_load<uint32_t>(r, r0 + i < nrow ? in : kOffNone);
     }
     sum = 0;
 #pragma unroll
@@ -881,7 +887,7 @@ __global__ __launch_bounds__(kGbTPB) void k_gb_offsets(uint32_t *__restrict__ ro
 }
 static int gb_scan(uint32_t *rows, uint32_t nrow, int k, uint32_t *sums, uint32_t *totals, hipStream_t s) {
     const uint32_t grid = div_up(nrow, kGbScanRows);
-    if (grid <= 1) return kOk;  // gb_wave_base sums the rows itself
+    if (nrow <= (uint32_t)kGbDirectRows) return kOk;  // gb_wave_base sums the rows itself
     hipLaunchKernelGGL(k_gb_sums, dim3(grid), dim3(kGbTPB), 0, s, rows, nrow, k, sums);
     PRODM_CHECK_LAUNCH();
     hipLaunchKernelGGL(k_gb_offsets, dim3(grid), dim3(kGbTPB), 0, s, rows, nrow, k, sums, totals);
@@ -893,7 +899,7 @@ static int gb_scan(uint32_t *rows, uint32_t nrow, int k, uint32_t *sums, uint32_
 // the wave's first word of plane pstart + p goes: the workgroup's offset plus
 // the words of the waves before it, from the recording planes of the
 // workgroup's blocks (one barrier). rows: offsets per workgroup, or with at
-// most kGbScanRows workgroups their words, which are summed here; totals
+// most kGbDirectRows workgroups their words, which are summed here; totals
 // (then, if any) takes the words of every plane. r: the lane's block's rb, 255
 // past the data. Both lanes of an f64 block hold the same r.
 struct GbWaveLds {
@@ -904,7 +910,7 @@ __device__ __forceinline__ uint32_t gb_wave_base(int r, const uint32_t *__restri
                                                  uint32_t *__restrict__ totals, GbWaveLds &lds, uint32_t bid,
                                                  uint32_t nwg) {
     const uint32_t lane = lane_id(), wv = threadIdx.x / 64;
-    const bool on = (int)lane < k, direct = nwg <= (uint32_t)kGbScanRows;
+    const bool on = (int)lane < k, direct = nwg <= (uint32_t)kGbDirectRows;
     lds.hw[wv][lane] = 0;
     if (r < 64 && lane < (uint32_t)WaveRows<T>::kBlocks) atomicAdd(&lds.hw[wv][r], 1u);
     uint32_t b = 0;
@@ -1180,7 +1186,7 @@ template <class T> size_t gb_decode_workspace_bytes(uint32_t n, int start, int k
 template size_t gb_decode_workspace_bytes<float>(uint32_t, int, int);
 template size_t gb_decode_workspace_bytes<double>(uint32_t, int, int);
 
-// ---- small levels of a plan together (at most kGbScanRows workgroups each) -------
+// ---- small levels of a plan together (at most kGbDirectRows workgroups each) -------
 template <class T> __global__ __launch_bounds__(kGbTPB) void k_gb_rb_set(LevelSet<GbLevel<T>> L, int nb) {
     const uint32_t i = set_entry(L, blockIdx.x);
     const GbLevel<T> &E = L.e[i];
@@ -1208,7 +1214,7 @@ template <class T> __global__ __launch_bounds__(kGbTPB) void k_gb_decode_set(Lev
 }
 template <class T> size_t gb_set_row_words(uint32_t n, int nb) {
     const uint32_t nwg = gb_nwg<T>(n);
-    return nwg <= (uint32_t)kGbScanRows ? (size_t)nwg * nb : 0;
+    return nwg <= (uint32_t)kGbDirectRows ? (size_t)nwg * nb : 0;
 }
 template size_t gb_set_row_words<float>(uint32_t, int);
 template size_t gb_set_row_words<double>(uint32_t, int);

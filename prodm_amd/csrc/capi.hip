@@ -346,8 +346,8 @@ template <class F> static int hook_call(void *ctx, int level) { return (*static_
 // Levels 0 .. small_top(p) (-1: none) are small: at most kSmallLevel elements.
 // Their encodes, decodes and recompose load sweeps are launched together, and a
 // plan of small levels only runs on the caller's stream alone: there a launch
-// or an event costs more than it would overlap. 2^21 is also the largest level
-// whose GroupedBP rows a workgroup adds up by itself (kGbScanRows of them).
+// or an event costs more than it would overlap. A level of 2^21 elements has
+// 256 rows of GroupedBP words, which its workgroups add up without a scan launch.
 // Refactor + retrieve of 33^3: 240 -> 141 us; 129^3: 318 -> 244, GroupedBP
 // 357 -> 263 (its finest level, 1.87e6, launched by itself on a second stream:
 // 290, 309); 1025^2: 400 -> 346; 257^3 GroupedBP f64: 742 -> 696.
