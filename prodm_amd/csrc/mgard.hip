@@ -1883,26 +1883,37 @@ int seg_class_strided(uint32_t seg) {
 }
 uint32_t strided_waves(uint32_t m) { return std::max<uint32_t>(1, std::min<uint32_t>(8, (m + 15) / 16)); }
 
-// The march of one grouped sweep. A tile of a 3-D field takes 2 march + 3 fine
-// planes, halo included, a 2-D one a single plane. Measured over batches of 3 to
-// 12 uneven fields and every level, a launch takes about 0.65 us for each plane
-// of its longest tile and as much for every 68 planes of all its tiles, so the
-// march with the smallest sum is taken. (Shortening each field's march to
-// 2048 tiles of its own left two planes per march, whose halo is most of the
-// work: 12 fields of 14.6 M points 376 us per refactor, 279 us by this rule,
-// 267 us autotuned.)
+// The march of one grouped sweep: the one with the smallest cost, in staged
+// nodes of its tiles' planes (2 march + 3 fine planes of a 3-D field's tile, one
+// of a 2-D one, halo included), with 6 whole planes (17 x 69 nodes) for each
+// tile's set-up and 240 for each plane of the longest tile, which ends the
+// launch. The weights are fitted to the sweeps of 62 batches at every march: 12
+// uneven fields of 14.6 M points 269 us per refactor (375 with each field's march
+// shortened to 2048 tiles of its own, two planes each, whose halo is most of the
+// work; 266 autotuned); 32 fields of 33^3 113 us (112 so, 119 by a model that
+// counted partial tiles as whole ones), 128 of them 165 (180, 177).
 template <class T> int default_march(const std::vector<std::pair<uint32_t, LoadParams<T>>> &entries) {
+    using SH = SweepStd;
+    // staged nodes of all tiles along one dim, m coarse nodes each
+    auto staged = [](uint32_t n, uint32_t c, uint32_t m) -> uint64_t {
+        if (n == 1) return 1;
+        uint64_t sum = 0;
+        for (uint32_t j = 0; j < c; j += m) sum += std::min(n, 2 * std::min(m, c - j) + 3);
+        return sum;
+    };
+    constexpr uint64_t kWhole = (2 * SH::kM1 + 3) * (2 * SH::kM2 + 3);
     int best = 2;
     uint64_t least = ~0ull;
     for (int march = 2; march <= 16; march *= 2) {
-        uint64_t planes = 0, longest = 0;
+        uint64_t nodes = 0, tiles = 0, longest = 0;
         for (const auto &e : entries) {
             const LoadParams<T> &P = e.second;
             const uint64_t per = P.n[0] == 1 ? 1 : 2 * std::min<uint64_t>(march, P.c[0]) + 3;
-            planes += sweep_tiles<T, SweepStd>(P, march) * per;
+            nodes += march_tiles0(P.n[0], P.c[0], march) * per * staged(P.n[1], P.c[1], SH::kM1) * staged(P.n[2], P.c[2], SH::kM2);
+            tiles += sweep_tiles<T, SH>(P, march);
             longest = std::max(longest, per);
         }
-        const uint64_t cost = planes + 68 * longest;
+        const uint64_t cost = nodes + kWhole * (6 * tiles + 240 * longest);
         if (cost < least) { least = cost; best = march; }
     }
     return best;
