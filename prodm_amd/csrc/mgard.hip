@@ -1471,7 +1471,10 @@ bool launch_wide(const SolveParams<T> &S, uint32_t m, uint64_t nlines, int d, hi
     } else {
         // four lines a workgroup while more would leave CUs idle: short
         // segments and more workgroups count for more than the length of the
-        // runs (769 nodes, 385 lines: 19 -> 13 us)
+        // runs. 769 nodes, 385 lines: 19 -> 13 us. Whole one-level decomposes,
+        // four lines against 16 (769 nodes) or 8 (2049): 272 lines 30 to 44 and
+        // 50 to 55 us, 784 lines 50 to 54 and 97 to 93, 1552 lines 75 to 73
+        // and 164 to 156
         const bool few = nlines < 4 * 256;
         if (m <= 32u * 36 && !few) PRODM_WIDE(36, 16);
         else if (m <= 64u * 36 && !few) PRODM_WIDE(36, 8);

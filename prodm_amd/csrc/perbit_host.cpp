@@ -11,9 +11,9 @@
 // elements that get their sign cost a step of their own. Plane i of a group
 // needs the signs known after plane i - 1 of the same group and nothing else,
 // so long levels are parsed by a pipeline of threads, some planes each.
-// (1.87 M float elements x 32 planes on an 8-CPU host: 40 ms in one thread, 14 ms
-// in eight; a 129^3 hierarchical refactor + retrieve beside an MI355X 143 ms bit
-// by bit, 7.3 ms now.)
+// (1.87 M float elements x 32 planes on an 8-CPU host: 45 ms in one thread, 14 ms
+// in eight; a 129^3 hierarchical refactor + retrieve beside an MI355X 143 to 149
+// ms bit by bit, now 7.4 to 9.2 by the host.)
 #include <algorithm>
 #include <atomic>
 #include <cmath>
@@ -244,8 +244,10 @@ int perbit_decode(prodm_perbit_state *s, int level, const uint64_t *const *strea
         rd[i].w = streams[i];
         if (sizes) rd[i].nwords = sizes[i] / 8;
     }
-    // threads where they have more to parse than they cost to start (some
-    // 20 us each): 8192 groups of 32 planes take about 4 ms in one
+    // threads where they have more to parse than they cost to start (some 20 us
+    // each, again for every window): 128 groups of 32 planes, at the line, take
+    // 189 us in one thread and 184 in two; 256 groups 416 and 237 (in four),
+    // 512 groups 1038 and 461 (in eight)
     const uint64_t work = (uint64_t)groups * k;
     const int cpus = (int)std::max(1u, std::thread::hardware_concurrency());
     const int stages = work < 4096 ? 1 : std::min({kMaxStages, cpus, k, (int)std::min<uint64_t>(work / 2048, 64)});
