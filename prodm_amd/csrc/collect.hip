@@ -110,7 +110,6 @@ constexpr int kExThreads = 256, kExEPT = 32, kExChunk = kExThreads * kExEPT;
 constexpr int kExMaxChunks = 8;  // 2^16 terms below 2^(u + 45) per workgroup: sums stay in 63 bits
 constexpr int kExSlots = 32;     // LDS words per accumulator
 constexpr int kExBins = 35;      // nb + 1 entries and two for the tiny elements
-constexpr int kExBuckets = 2048;
 
 struct Grid3 {
     int n;     // accumulators used
@@ -165,22 +164,82 @@ struct Acc3 {
     }
 };
 
-// one term outside the grids, into the 128-bit sum of its exponent. A term that
-// is infinite or NaN has no sum and is left out, or (over) counts as its float's
-// bits read as a number: infinity is 2^128.
-__device__ __forceinline__ void add_under(double t, int bin, unsigned long long *under, uint32_t *flag, bool over) {
-    const uint64_t tb = to_bits(t);
-    int be = (int)((tb >> 52) & 0x7ff);
-    if (!(tb << 1)) return;
-    if (be == 0x7ff) {
-        if (!over) return;
-        be = 1023 + 128;
+// Terms outside the grids go to 128-bit sums of their exponents: buckets
+// [first, first + n) of double exponents for each entry.
+struct Under {
+    unsigned long long *sum;
+    uint32_t *flag;  // set once any is used
+    int first, n;
+    __device__ __forceinline__ void add(int bin, int be, unsigned long long v) const {
+        unsigned long long *bk = sum + ((size_t)bin * n + (be - first)) * 2;
+        const unsigned long long old = atomicAdd(bk, v);
+        if (old + v < old) atomicAdd(bk + 1, 1ull);
+        *flag = 1u;
     }
-    const unsigned long long M = (tb & ((1ull << 52) - 1)) | (be ? (1ull << 52) : 0);
-    unsigned long long *bk = under + ((size_t)bin * kExBuckets + (be ? be : 1)) * 2;
-    const unsigned long long old = atomicAdd(bk, M);
-    if (old + M < old) atomicAdd(bk + 1, 1ull);
-    *flag = 1u;
+};
+// exponent and mantissa of a term. One that is infinite or NaN has no sum and
+// is left out (M = 0), or (over) counts as its float's bits read as a number:
+// infinity is 2^128.
+__device__ __forceinline__ unsigned long long term_bits(double t, bool over, int &be) {
+    const uint64_t tb = to_bits(t);
+    be = (int)((tb >> 52) & 0x7ff);
+    unsigned long long M = (tb & ((1ull << 52) - 1)) | (be ? (1ull << 52) : 0);
+    if (be == 0x7ff) {
+        be = 1023 + 128;
+        if (!over) M = 0;
+    }
+    be = be ? be : 1;
+    return M;
+}
+__device__ __forceinline__ void add_under(double t, int bin, const Under &U, bool over) {
+    int be;
+    const unsigned long long M = term_bits(t, over, be);
+    if (M) U.add(bin, be, M);
+}
+// The terms of the wave's elements named by `past` (element 0 of the lane's in
+// bit 31; term(x, k) for entries 0 .. nb) through windows of 64 exponents in
+// LDS, kPastEntries entries at a time, whose used words go to the buckets in one
+// addition each: every element's own additions there meet on a few addresses
+// (3 M floats, a third of them past the bound: 6.5 ms, now 0.29). At most 2^11
+// additions below 2^53 per word.
+constexpr int kPastEntries = 4;
+template <class Term>
+__device__ __forceinline__ void add_past(uint32_t past, const float *x, int nb, bool over, const Under &U,
+                                         unsigned long long (*win)[64], Term &&term) {
+    if (!__any(past != 0)) return;
+    const int lane = (int)lane_id();
+    auto each = [&](auto &&fn) __attribute__((always_inline)) {
+        for (uint32_t left = past; left;) {
+            const int i = __clz(left);
+            left ^= 0x80000000u >> i;
+            fn(x[(uint64_t)i * kExThreads + threadIdx.x]);
+        }
+    };
+    // entry 0 has the largest terms, those of the others are at most some times that
+    int base = 0;
+    each([&](float v) __attribute__((always_inline)) {
+        int be;
+        if (term_bits(term(v, 0), over, be)) base = max(base, be);
+    });
+    for (int o = 32; o >= 1; o >>= 1) base = max(base, __shfl_xor(base, o, 64));
+    base -= 59;
+    for (int k0 = 0; k0 <= nb; k0 += kPastEntries) {
+        for (int j = 0; j < kPastEntries; j++) win[j][lane] = 0;
+        wave_lds_sync();
+        each([&](float v) __attribute__((always_inline)) {
+            for (int j = 0; j < kPastEntries && k0 + j <= nb; j++) {
+                int be;
+                const unsigned long long M = term_bits(term(v, k0 + j), over, be);
+                if (!M) continue;
+                if (be >= base && be < base + 64) atomicAdd(&win[j][be - base], M);
+                else U.add(k0 + j, be, M);
+            }
+        });
+        wave_lds_sync();
+        for (int j = 0; j < kPastEntries; j++)
+            if (win[j][lane]) U.add(k0 + j, base + lane, win[j][lane]);
+        wave_lds_sync();
+    }
 }
 
 // the workgroup's sums of every accumulator (kExBins * 3 of kExSlots words)
@@ -216,11 +275,13 @@ __global__ __launch_bounds__(kExThreads) void k_exact_totals(const uint64_t *__r
 // workspace: [totals: bins * 3 * 2 words][flag][partials][exponent buckets]
 struct ExLayout {
     uint32_t nwg;
-    int bins;
+    int bins, first, buckets;
     size_t flag, partial, under, total;
 };
-ExLayout ex_layout(uint64_t n, int nb) {
+ExLayout ex_layout(uint64_t n, int nb, int first, int buckets) {
     ExLayout L;
+    L.first = first;
+    L.buckets = buckets;
     const uint64_t chunks = std::max<uint64_t>(1, (n + kExChunk - 1) / kExChunk);
     // one chunk per workgroup up to 4 workgroups per CU, then up to kExMaxChunks
     const uint64_t per = std::min<uint64_t>(kExMaxChunks, std::max<uint64_t>(1, chunks / 1024));
@@ -229,7 +290,7 @@ ExLayout ex_layout(uint64_t n, int nb) {
     L.flag = (size_t)L.bins * 3 * 16;
     L.partial = L.flag + 16;
     L.under = L.partial + (size_t)L.bins * 3 * 8 * L.nwg;
-    L.total = L.under + (size_t)L.bins * kExBuckets * 16;
+    L.total = L.under + (size_t)L.bins * buckets * 16;
     return L;
 }
 
@@ -263,9 +324,10 @@ int exact_finish(const ExLayout &L, int nb, GridOf grid, TinyOf tiny, int scale,
                     b.add128(((__int128)(int64_t)t[1] << 32) + (__int128)t[0], g.u[a] - kEmin, neg);
                 }
                 if (!neg && !under.empty())
-                    for (int e = 1; e < kExBuckets; e++) {
-                        b.add_shifted(under[((size_t)i * kExBuckets + e) * 2], e - 1);
-                        b.add_shifted(under[((size_t)i * kExBuckets + e) * 2 + 1], e - 1 + 64);
+                    for (int e = 0; e < L.buckets; e++) {
+                        const uint64_t *u = under.data() + ((size_t)i * L.buckets + e) * 2;
+                        b.add_shifted(u[0], L.first + e - 1);
+                        b.add_shifted(u[1], L.first + e - 1 + 64);
                     }
             }
         out[k] = std::ldexp(b.to_double(kEmin), scale);
@@ -332,9 +394,8 @@ __device__ inline T sq_term(T x, int de, int le, int nb, int k) {
 // (x - x cleared of mantissa bits 0 .. b)^2 in entry k, b = le + 23 - de - k
 // (x^2 from b = 23 on, 0 below b = 0). With le - nb < de <= le its terms are at
 // most 2^(2 (le - k)) and multiples of 2^(2 (le - nb - 23)). Smaller elements
-// have the term x^2 in every entry and are summed once; subnormal ones above
-// that (whose bits do not shift with de) and ones past the bound go term by
-// term to the buckets.
+// have the term x^2 in every entry and are summed once; ones past the bound go
+// term by term to the buckets.
 // Squares are float. One past the largest float counts as 2^128, as in the CPU
 // restatement (infinity's bits read as a number), so that no term is above 2^128
 // and 2^128 is on the grid of any step up to it. Only entries with le - k > 64
@@ -348,10 +409,9 @@ __host__ __device__ inline Grid3 sq_grid(int k, int le, int nb) {
     return grid3(t < 128 ? t : 128, q < -149 ? -149 : q > 128 ? 128 : q);
 }
 __global__ __launch_bounds__(kExThreads) void k_collect_squared_f32(const float *__restrict__ x, uint64_t n, int nb,
-                                                                    int le, uint64_t *__restrict__ partial,
-                                                                    unsigned long long *__restrict__ under,
-                                                                    uint32_t *__restrict__ flag) {
+                                                                    int le, uint64_t *__restrict__ partial, Under U) {
     __shared__ unsigned long long acc[kExBins * 3 * kExSlots];
+    __shared__ unsigned long long win[kExThreads / 64][kPastEntries][64];
     for (int i = threadIdx.x; i < (nb + 3) * 3 * kExSlots; i += kExThreads) acc[i] = 0;
     __syncthreads();
     for (uint64_t c = blockIdx.x; c * kExChunk < n; c += gridDim.x) {
@@ -365,12 +425,13 @@ __global__ __launch_bounds__(kExThreads) void k_collect_squared_f32(const float 
             const float a = fabsf(v[i]);
             cut[i] = le + 24 - de;
             const bool main = de > le - nb && de <= le && a >= 1.17549435e-38f && a < __builtin_inff();
-            rest = 2 * rest + (!main && v[i] != 0.0f);
+            rest = 2 * rest + (!main && !(a < 1.17549435e-38f));  // a subnormal element's squares are 0
             v[i] = main ? v[i] : 0.0f;
             // formed here: left to the loop below, the selects and what they
             // read would both stay live (256 VGPRs instead of 111)
             asm volatile("" : "+v"(v[i]), "+v"(cut[i]));
         }
+        uint32_t past = 0;
         if (__any(rest != 0)) {
             Acc3 tiny;
             tiny.start(sq_grid(nb + 1, le, nb));
@@ -382,10 +443,9 @@ __global__ __launch_bounds__(kExThreads) void k_collect_squared_f32(const float 
                 if (de <= le - nb && fabsf(t) < __builtin_inff()) {
                     const float tt = t * t;
                     const double td = fmin((double)tt, kSqOver);
-                    if (!tiny.add_open(td)) add_under(td, nb + 1, under, flag, false);
+                    if (!tiny.add_open(td)) add_under(td, nb + 1, U, false);
                 } else {
-                    for (int k = 0; k <= nb; k++)
-                        add_under((double)sq_term<float>(t, de, le, nb, k), k, under, flag, le > nb + 23);
+                    past |= 0x80000000u >> i;
                 }
             }
             tiny.flush(acc + (nb + 1) * 3 * kExSlots);
@@ -405,23 +465,30 @@ __global__ __launch_bounds__(kExThreads) void k_collect_squared_f32(const float 
             else
                 sum_bin(g, slot, term);
         }
+        // last, when the elements' registers are free
+        add_past(past, x + c * kExChunk, nb, le > nb + 23, U, win[threadIdx.x / 64],
+                 [&](float t, int k) __attribute__((always_inline)) -> double {
+                     return (double)sq_term<float>(t, dev_frexp_exp(t), le, nb, k);
+                 });
     }
     __syncthreads();
     store_partials(acc, nb + 3, partial);
 }
 
-size_t sq_workspace_bytes_f32(uint64_t n, int nb) { return ex_layout(n, nb).total; }
+// float squares: exponents of 2^-149 to 2^128 as doubles
+ExLayout sq_layout(uint64_t n, int nb) { return ex_layout(n, nb, 1023 - 149, 149 + 128 + 1); }
+size_t sq_workspace_bytes_f32(uint64_t n, int nb) { return sq_layout(n, nb).total; }
 static int squared_errors_f32(const float *x, uint64_t n, int nb, float maxerr, double *out, void *ws, hipStream_t s) {
     int le = 0;
     std::frexp(maxerr, &le);
-    const ExLayout L = ex_layout(n, nb);
+    const ExLayout L = sq_layout(n, nb);
     char *base = static_cast<char *>(ws);
     uint32_t *flag = reinterpret_cast<uint32_t *>(base + L.flag);
     if (int rc = launch_fill_u32(flag, 4, 0u, s)) return rc;
     if (int rc = launch_fill_u64(reinterpret_cast<uint64_t *>(base + L.under), (L.total - L.under) / 8, 0ull, s)) return rc;
     hipLaunchKernelGGL(k_collect_squared_f32, dim3(L.nwg), dim3(kExThreads), 0, s, x, n, nb, le,
                        reinterpret_cast<uint64_t *>(base + L.partial),
-                       reinterpret_cast<unsigned long long *>(base + L.under), flag);
+                       Under{reinterpret_cast<unsigned long long *>(base + L.under), flag, L.first, L.buckets});
     PRODM_CHECK_LAUNCH();
     return exact_finish(L, nb, [&](int i) { return sq_grid(i, le, nb); }, [](int) { return 1; }, 0, out, ws, s);
 }
@@ -592,7 +659,7 @@ template <> int squared_errors<double>(const double *x, uint64_t n, int nb, doub
 // reference does. Each entry is the exactly rounded sum over elements, then
 // scaled by 2^(2 (e - nb)).
 //
-// Exactness: an element with 1 <= |s| < 2^min(nb, 31) has terms of at most
+// Exactness: an element with 1 <= |s| < 2^min(nb, kFeTop) has terms of at most
 // 2^(2 (nb - k) + 2) in entry k that are multiples of 2^-46 (the fraction's step
 // is at least 2^-23). One with |s| < 1 has no digit: its term is s^2 in every
 // entry, as a double, or squared in float where the reference squares in
@@ -639,19 +706,21 @@ __device__ __forceinline__ void fe_split(float x, int shift, float &s, float &m,
 }
 
 constexpr int kFeQ = -46;
+// digits end at 2^31 (int32) and 2^32 (uint32)
+template <int ENC> constexpr int kFeTop = ENC == 0 ? 31 : 32;
+ExLayout fe_layout(uint64_t n, int nb) { return ex_layout(n, nb, 1, 2046); }
 __host__ __device__ inline Grid3 fe_grid(int k, int nb) {
     return k > nb ? grid3_open(0) : grid3(2 * (nb - k) + 2, kFeQ);
 }
 
 template <int ENC>
 __global__ __launch_bounds__(kExThreads) void k_fused_errors(const float *__restrict__ x, uint64_t n, int shift,
-                                                             int nb, uint64_t *__restrict__ partial,
-                                                             unsigned long long *__restrict__ under,
-                                                             uint32_t *__restrict__ flag) {
+                                                             int nb, uint64_t *__restrict__ partial, Under U) {
     __shared__ unsigned long long acc[kExBins * 3 * kExSlots];
+    __shared__ unsigned long long win[kExThreads / 64][kPastEntries][64];
     for (int i = threadIdx.x; i < (nb + 3) * 3 * kExSlots; i += kExThreads) acc[i] = 0;
     __syncthreads();
-    const float top = ldexpf(1.0f, min(nb, 31));
+    const float top = ldexpf(1.0f, min(nb, kFeTop<ENC>));
     for (uint64_t c = blockIdx.x; c * kExChunk < n; c += gridDim.x) {
         float m[kExEPT];
         uint32_t bits[kExEPT];
@@ -668,6 +737,7 @@ __global__ __launch_bounds__(kExThreads) void k_fused_errors(const float *__rest
             bits[i] = main ? bits[i] : 0u;
             asm volatile("" : "+v"(m[i]), "+v"(bits[i]));  // as above
         }
+        uint32_t past = 0;
         if (__any(rest != 0)) {
             Acc3 tinyd, tinyf;
             tinyd.start(fe_grid(nb + 1, nb));
@@ -681,10 +751,10 @@ __global__ __launch_bounds__(kExThreads) void k_fused_errors(const float *__rest
                 if (fabsf(s) < 1.0f) {
                     const double d = (double)s * (double)s;
                     const float ff = s * s;
-                    if (!tinyd.add_open(d)) add_under(d, nb + 1, under, flag, false);
-                    if (!tinyf.add_open((double)ff)) add_under((double)ff, nb + 2, under, flag, false);
+                    if (!tinyd.add_open(d)) add_under(d, nb + 1, U, false);
+                    if (!tinyf.add_open((double)ff)) add_under((double)ff, nb + 2, U, false);
                 } else {
-                    for (int k = 0; k <= nb; k++) add_under(fe_term<ENC>(s, mm, bb, nb, k), k, under, flag, false);
+                    past |= 0x80000000u >> i;
                 }
             }
             tinyd.flush(acc + (nb + 1) * 3 * kExSlots);
@@ -706,31 +776,38 @@ __global__ __launch_bounds__(kExThreads) void k_fused_errors(const float *__rest
                 return d * d;
             });
         }
+        add_past(past, x + c * kExChunk, nb, false, U, win[threadIdx.x / 64],
+                 [&](float t, int k) __attribute__((always_inline)) -> double {
+                     float s, mm;
+                     uint32_t bb;
+                     fe_split<ENC>(t, shift, s, mm, bb);
+                     return fe_term<ENC>(s, mm, bb, nb, k);
+                 });
     }
     __syncthreads();
     store_partials(acc, nb + 3, partial);
 }
 }  // namespace
 
-size_t fused_errors_workspace_bytes(uint64_t n, int nb) { return ex_layout(n, nb).total; }
+size_t fused_errors_workspace_bytes(uint64_t n, int nb) { return fe_layout(n, nb).total; }
 
 int fused_level_errors(int enc, const float *x, uint64_t n, int32_t exp, int nb, double *out, void *ws,
                        size_t ws_bytes, hipStream_t s) {
     if (nb < 1 || nb > 32 || !out || (enc != 0 && enc != 1)) { set_error("level errors: bad arguments"); return kErrArg; }
     if (n > 0 && !x) { set_error("level errors: null input"); return kErrArg; }
-    const ExLayout L = ex_layout(n, nb);
+    const ExLayout L = fe_layout(n, nb);
     if (ws_bytes < L.total || !ws) { set_error("level errors: workspace too small"); return kErrArg; }
     const int e = enc == 0 ? exp + 2 : exp;  // NegaBinaryBPEncoder.hpp:68
     char *base = static_cast<char *>(ws);
     uint64_t *partial = reinterpret_cast<uint64_t *>(base + L.partial);
-    unsigned long long *under = reinterpret_cast<unsigned long long *>(base + L.under);
     uint32_t *flag = reinterpret_cast<uint32_t *>(base + L.flag);
+    const Under under{reinterpret_cast<unsigned long long *>(base + L.under), flag, L.first, L.buckets};
     if (int rc = launch_fill_u32(flag, 4, 0u, s)) return rc;
-    if (int rc = launch_fill_u64(reinterpret_cast<uint64_t *>(under), (L.total - L.under) / 8, 0ull, s)) return rc;
+    if (int rc = launch_fill_u64(reinterpret_cast<uint64_t *>(base + L.under), (L.total - L.under) / 8, 0ull, s)) return rc;
     if (enc == 0)
-        hipLaunchKernelGGL(k_fused_errors<0>, dim3(L.nwg), dim3(kExThreads), 0, s, x, n, nb - e, nb, partial, under, flag);
+        hipLaunchKernelGGL(k_fused_errors<0>, dim3(L.nwg), dim3(kExThreads), 0, s, x, n, nb - e, nb, partial, under);
     else
-        hipLaunchKernelGGL(k_fused_errors<1>, dim3(L.nwg), dim3(kExThreads), 0, s, x, n, nb - e, nb, partial, under, flag);
+        hipLaunchKernelGGL(k_fused_errors<1>, dim3(L.nwg), dim3(kExThreads), 0, s, x, n, nb - e, nb, partial, under);
     PRODM_CHECK_LAUNCH();
     // entries whose terms of tiny elements are squared in float take the second sum
     return exact_finish(L, nb, [&](int i) { return fe_grid(i, nb); },

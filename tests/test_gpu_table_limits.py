@@ -27,7 +27,8 @@ def squared_terms(x, nb, m):
             b = low + index - k  # mantissa bits 0..b are cleared, all of x past bit 22
             keep = np.uint32((0xffffffff << (b + 1)) & 0xffffffff) if b < 23 else np.uint32(0)
             d = np.float32(v - (np.float32(v).view(np.uint32) & keep).view(np.float32)) if b < 23 else v
-            bins[k].append(float(d * d))
+            with np.errstate(over="ignore"):
+                bins[k].append(min(float(d * d), 2.0 ** 128))  # as an infinite square counts
     return np.array([math.fsum(t) for t in bins])
 
 
@@ -52,8 +53,11 @@ def test_largest_float(gpu):
 
 def test_terms_restatement():
     """the restatement used below agrees with the oracle where both hold"""
+    for x in (spread(500, 2, 60), spread(500, 2, 60, 100)):
+        nb = 32
+        assert np.array_equal(squared_terms(x, nb, ob.maxabs(x)), ob.collect_squared(x, nb, ob.maxabs(x)))
     x = spread(500, 2, 60)
-    for nb in (1, 8, 23, 24, 32):
+    for nb in (1, 8, 23, 24):
         assert np.array_equal(squared_terms(x, nb, ob.maxabs(x)), ob.collect_squared(x, nb, ob.maxabs(x)))
 
 
@@ -92,3 +96,26 @@ def test_infinities_and_nan_are_left_out(gpu, n, low):
         for enc in (0, 1):
             want = ob.fused_level_errors(zeroed, e, nb, "nb" if enc == 0 else "gb", mode="exact")
             assert np.array_equal(mdr.level_errors(d, e, nb, enc), want)
+
+
+@pytest.mark.parametrize("enc,nb", [(0, 32), (1, 32), (1, 31), (1, 5)])
+@pytest.mark.parametrize("n", [1, 8193, 70001])
+@pytest.mark.parametrize("lo,width", [(0.5, 0.5), (270.0, 60.0), (4294967040.0, 0.0), (2.0 ** 31, 2.0 ** 31 - 256)])
+def test_encoder_top_binade(gpu, enc, nb, n, lo, width):
+    """every element's top digit set"""
+    from prodm_amd import mdr
+    x = (lo + width * np.random.default_rng(n).random(n)).astype(np.float32)
+    x[::3] *= -1
+    e = ob.frexp_exp(ob.maxabs(x), np.float32)
+    got = mdr.level_errors(torch.from_numpy(x).to(gpu), e, nb, enc)
+    assert np.array_equal(got, ob.fused_level_errors(x, e, nb, "nb" if enc == 0 else "gb", mode="exact"))
+
+
+@pytest.mark.parametrize("scale", [0, -145, 70])
+def test_squared_many_above_the_maximum(gpu, scale):
+    """a whole wave's elements past the bound, spread over more exponents than the window holds"""
+    from prodm_amd import mdr
+    x = spread(9000, 21, 0, scale)
+    x[:2048] *= np.exp2(np.random.default_rng(4).integers(0, 40 if scale < 60 else 1, 2048)).astype(np.float32)
+    m = math.ldexp(1.0, scale - 2)
+    assert np.array_equal(mdr.collect_squared(torch.from_numpy(x).to(gpu), 32, m), squared_terms(x, 32, m))
