@@ -127,6 +127,8 @@ __global__ __launch_bounds__(256) void k_adj_copy(const G *__restrict__ h, uint6
 
 dim3 grid_of(const uint32_t *n) { return dim3(div_up(n[2], 256), n[1], n[0]); }
 
+// g: the dense copy of a box that meets its output or has planes of 2 GiB (the
+// size query sees neither)
 struct AdjLayout {
     size_t g, h0, h1, mgard, total;
 };

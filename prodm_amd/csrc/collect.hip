@@ -91,6 +91,8 @@ struct Big {
 
 
 // ---- exact sums in FP64 (float data) --------------------------------------------
+// Error-free extraction onto fixed grids, the idea of Demmel and Nguyen's binned
+// summation, with every grid's sum kept as an integer.
 // A term below 2^T and a multiple of 2^Q is added to up to three accumulators
 // of decreasing grid 2^u. An accumulator starts at 1.5 2^(u + 52), so that it
 // stays in one binade, whose numbers are the multiples of 2^u: adding a term
